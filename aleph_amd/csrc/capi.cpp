@@ -1269,30 +1269,36 @@ aleph_hip_status aleph_hip_run_noisy(aleph_hip_ctx* c, uint32_t n, const uint32_
       throw f;
     }
     const std::vector<ProgInstr> prog = decode_program(words, n_words, reals, n_reals, n);
-    const TrajHost h = build_trajectories(prog, n, channels, n_channels, readout, readout_mask);
+    TrajHost h = build_trajectories(prog, n, channels, n_channels, readout, readout_mask);
     if (shots == 0) return;
+    StagedHost staged;
+    const bool in_registers = build_staged(h, n, staged);
     uint32_t workgroups = 0;
     size_t slice_bytes = 0;
-    trajectory_geometry(n, shots, budget_bytes ? budget_bytes : (size_t{4} << 30), &workgroups, &slice_bytes);
-    const size_t op_bytes = h.ops.size() * sizeof(TrajOp), real_bytes = h.reals.size() * sizeof(double);
-    const size_t mask_bytes = h.masks.size() * sizeof(uint64_t), index_bytes = h.index.size() * sizeof(uint32_t);
-    const size_t ro_bytes = std::max<size_t>(h.readout.size(), 1) * sizeof(double);
-    // One device block: program records, payloads, readout table, outcomes.
-    auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
-    const size_t o_ops = 0, o_reals = al(op_bytes), o_masks = o_reals + al(real_bytes),
-                 o_index = o_masks + al(mask_bytes), o_ro = o_index + al(index_bytes), o_out = o_ro + al(ro_bytes),
-                 total = o_out + al((size_t)shots * sizeof(uint64_t));
-    DevBuf blk(total);
+    if (!in_registers)
+      trajectory_geometry(n, shots, budget_bytes ? budget_bytes : (size_t{4} << 30), &workgroups, &slice_bytes);
+    // One device block: program records, payloads, readout table, outcomes;
+    // everything but the outcomes goes up in one copy.
+    std::vector<unsigned char> host;
+    auto place = [&](const void* src, size_t bytes) {
+      const size_t at = (host.size() + 255) & ~(size_t)255;
+      host.resize(at + std::max<size_t>(bytes, 16));
+      if (bytes) std::memcpy(host.data() + at, src, bytes);
+      return at;
+    };
+    const size_t o_ops = in_registers ? 0 : place(h.ops.data(), h.ops.size() * sizeof(TrajOp));
+    const size_t o_stages = place(staged.stages.data(), staged.stages.size() * sizeof(TStage));
+    const size_t o_tops = place(staged.ops.data(), staged.ops.size() * sizeof(TOp));
+    const size_t o_chans = place(staged.chans.data(), staged.chans.size() * sizeof(TChan));
+    const size_t o_reals = place(h.reals.data(), h.reals.size() * sizeof(double));
+    const size_t o_masks = place(h.masks.data(), h.masks.size() * sizeof(uint64_t));
+    const size_t o_index = place(h.index.data(), h.index.size() * sizeof(uint32_t));
+    const size_t o_ro = place(h.readout.data(), h.readout.size() * sizeof(double));
+    const size_t o_out = (host.size() + 255) & ~(size_t)255;
+    DevBuf blk(o_out + (size_t)shots * sizeof(uint64_t));
     DevBuf slices(slice_bytes);
     unsigned char* base = (unsigned char*)blk.p;
-    if (op_bytes)
-      ALEPH_HIP_CHECK(hipMemcpyAsync(base + o_ops, h.ops.data(), op_bytes, hipMemcpyHostToDevice, c->stream));
-    ALEPH_HIP_CHECK(hipMemcpyAsync(base + o_reals, h.reals.data(), real_bytes, hipMemcpyHostToDevice, c->stream));
-    ALEPH_HIP_CHECK(hipMemcpyAsync(base + o_masks, h.masks.data(), mask_bytes, hipMemcpyHostToDevice, c->stream));
-    ALEPH_HIP_CHECK(hipMemcpyAsync(base + o_index, h.index.data(), index_bytes, hipMemcpyHostToDevice, c->stream));
-    if (!h.readout.empty())
-      ALEPH_HIP_CHECK(hipMemcpyAsync(base + o_ro, h.readout.data(), h.readout.size() * sizeof(double),
-                                     hipMemcpyHostToDevice, c->stream));
+    ALEPH_HIP_CHECK(hipMemcpyAsync(base, host.data(), host.size(), hipMemcpyHostToDevice, c->stream));
     TrajProgram tp;
     tp.ops = (const TrajOp*)(base + o_ops);
     tp.n_ops = (uint32_t)h.ops.size();
@@ -1306,7 +1312,20 @@ aleph_hip_status aleph_hip_run_noisy(aleph_hip_ctx* c, uint32_t n, const uint32_
     tp.shot0 = shot_offset;
     tp.shots = shots;
     uint64_t* d_out = (uint64_t*)(base + o_out);
-    launch_trajectories(c->stream, tp, workgroups, slices.p, d_out);
+    if (in_registers) {
+      StagedProgram sp;
+      sp.stages = (const TStage*)(base + o_stages);
+      sp.ops = (const TOp*)(base + o_tops);
+      sp.chans = (const TChan*)(base + o_chans);
+      sp.n_stages = (uint32_t)staged.stages.size();
+      sp.n_ops = (uint32_t)staged.ops.size() - 1;
+      sp.n_chan = (uint32_t)staged.chans.size();
+      for (const TOp& op : staged.ops)
+        sp.rare |= op.kind == TOp::TWO || op.kind == TOp::DIAG || (op.kind == TOp::ONE && op.cmask != 0);
+      launch_staged(c->stream, tp, sp, d_out);
+    } else {
+      launch_trajectories(c->stream, tp, workgroups, slices.p, d_out);
+    }
     ALEPH_HIP_CHECK(hipMemcpyAsync(outcomes, d_out, (size_t)shots * sizeof(uint64_t), hipMemcpyDeviceToHost, c->stream));
     ALEPH_HIP_CHECK(hipStreamSynchronize(c->stream));
   });

@@ -168,4 +168,210 @@ TrajHost build_trajectories(const std::vector<ProgInstr>& prog, uint32_t n, cons
   return h;
 }
 
+namespace {
+
+// Dense matrix (interleaved, dim 2^k, targets MSB first) that is the identity
+// except for a 2x2 block selected by every target but one being 1: the
+// remaining target's position, or -1.
+int controlled_target(const double* m, uint32_t k) {
+  const uint32_t dim = 1u << k;
+  for (uint32_t t = 0; t < k; t++) {
+    const uint32_t tb = 1u << (k - 1 - t), cb = (dim - 1u) & ~tb;
+    bool ok = true;
+    for (uint32_t r = 0; r < dim && ok; r++)
+      for (uint32_t c = 0; c < dim && ok; c++) {
+        if ((r & cb) == cb && (c & cb) == cb) continue;
+        ok = m[2 * (r * dim + c)] == (r == c ? 1.0 : 0.0) && m[2 * (r * dim + c) + 1] == 0.0;
+      }
+    if (ok) return (int)t;
+  }
+  return -1;
+}
+
+// Smallest eigenvalue of K^dagger K.
+double min_branch_probability(const double* k) {
+  const double a = k[0] * k[0] + k[1] * k[1] + k[4] * k[4] + k[5] * k[5];
+  const double d = k[2] * k[2] + k[3] * k[3] + k[6] * k[6] + k[7] * k[7];
+  const cplx b = std::conj(cplx(k[0], k[1])) * cplx(k[2], k[3]) + std::conj(cplx(k[4], k[5])) * cplx(k[6], k[7]);
+  return 0.5 * ((a + d) - std::sqrt((a - d) * (a - d) + 4.0 * std::norm(b)));
+}
+
+void mul2x2(const double* a, const double* b, double* out) {
+  for (int r = 0; r < 2; r++)
+    for (int c = 0; c < 2; c++) {
+      cplx z = 0.0;
+      for (int j = 0; j < 2; j++)
+        z += cplx(a[2 * (2 * r + j)], a[2 * (2 * r + j) + 1]) * cplx(b[2 * (2 * j + c)], b[2 * (2 * j + c) + 1]);
+      out[2 * (2 * r + c)] = z.real();
+      out[2 * (2 * r + c) + 1] = z.imag();
+    }
+}
+
+// Draws within this relative distance of the bound look at the state, so the
+// rounding of the computed probability cannot change a decision; channels
+// whose bound is small always do (the unnormalised state would shrink fast).
+constexpr double kShortcutGuard = 1e-9;
+constexpr double kShortcutMin = 1e-3;
+
+}  // namespace
+
+bool build_staged(TrajHost& h, uint32_t n, StagedHost& out) {
+  if (n < kStagedMinQubits || n > kStagedMaxQubits) return false;
+  const uint32_t G = staged_reg_bits(n);
+  std::vector<TOp> ops;
+  std::vector<uint32_t> need;   // qubits that must sit in registers, per record
+  // `last` is a ONE record that only Pauli channels have followed: a Kraus
+  // channel on its qubit is folded into it.
+  int64_t last = -1;
+  for (const TrajOp& t : h.ops) {
+    TOp op;
+    op.f0 = op.f1 = (uint32_t)out.chans.size();
+    if (t.kind == TrajOp::PAULI) {
+      TChan c;
+      c.pauli = 1;
+      c.count = t.count;
+      c.off = t.off;
+      c.off2 = t.off2;
+      out.chans.push_back(c);
+      continue;
+    }
+    if (t.kind == TrajOp::KRAUS) {
+      TChan c;
+      c.count = t.count;
+      const double* k0 = h.reals.data() + t.off;
+      const double lam = min_branch_probability(k0);
+      if (lam >= kShortcutMin) c.thr = lam * (1.0 - kShortcutGuard);
+      const uint32_t chan = (uint32_t)out.chans.size();
+      out.chans.push_back(c);
+      if (last >= 0 && ops[(size_t)last].qmask == (1u << t.q[0]) && ops[(size_t)last].chan == ~0u) {
+        TOp& g = ops[(size_t)last];
+        g.off = (uint32_t)h.reals.size();
+        h.reals.insert(h.reals.end(), g.m, g.m + 8);
+        double f[8];
+        mul2x2(h.reals.data() + t.off, h.reals.data() + g.off, f);
+        for (int e = 0; e < 8; e++) g.m[e] = f[e];
+        g.f1 = chan;
+        g.chan = chan;
+        g.koff = t.off;
+        g.count = t.count;
+        g.lam = lam;
+        last = -1;
+        continue;
+      }
+      op.kind = TOp::KRAUS;
+      op.qmask = 1u << t.q[0];
+      op.chan = chan;
+      op.koff = t.off;
+      op.count = t.count;
+      op.lam = lam;
+      for (int e = 0; e < 8; e++) op.m[e] = k0[e];
+      ops.push_back(op);
+      need.push_back(op.qmask);
+      last = -1;
+      continue;
+    }
+    last = -1;
+    const double* m = h.reals.data() + t.off;
+    if (t.kind == TrajOp::DIAG) {
+      const uint32_t dim = 1u << t.k;
+      bool sign = true;
+      uint32_t targets = 0;
+      for (uint32_t j = 0; j < dim; j++) sign &= m[2 * j] == (j + 1 == dim ? -1.0 : 1.0) && m[2 * j + 1] == 0.0;
+      for (uint32_t j = 0; j < t.k; j++) targets |= 1u << t.q[j];
+      op.kind = sign ? TOp::SIGN : TOp::DIAG;
+      op.cmask = (uint32_t)t.cmask | (sign ? targets : 0u);
+      op.off = t.off;
+      op.qmask2 = t.k;
+      for (uint32_t j = 0; j < t.k; j++) op.qmask |= t.q[j] << (4 * j);
+      ops.push_back(op);
+      need.push_back(0);
+      continue;
+    }
+    if (t.kind != TrajOp::DENSE) return false;
+    const int ct = t.k == 1 ? 0 : controlled_target(m, t.k);
+    if (ct >= 0) {
+      const uint32_t dim = 1u << t.k, tb = 1u << (t.k - 1 - (uint32_t)ct), hi = dim - 1u, lo = hi & ~tb;
+      op.kind = TOp::ONE;
+      op.qmask = 1u << t.q[ct];
+      op.cmask = (uint32_t)t.cmask;
+      for (uint32_t j = 0; j < t.k; j++)
+        if ((int)j != ct) op.cmask |= 1u << t.q[j];
+      const uint32_t e[4] = {lo * dim + lo, lo * dim + hi, hi * dim + lo, hi * dim + hi};
+      for (int i = 0; i < 4; i++) {
+        op.m[2 * i] = m[2 * e[i]];
+        op.m[2 * i + 1] = m[2 * e[i] + 1];
+      }
+      ops.push_back(op);
+      need.push_back(op.qmask);
+      if (op.cmask == 0) last = (int64_t)ops.size() - 1;
+      continue;
+    }
+    if (t.k != 2 || t.cmask != 0) return false;
+    op.kind = TOp::TWO;
+    op.qmask = 1u << t.q[0];
+    op.qmask2 = 1u << t.q[1];
+    op.off = t.off;
+    ops.push_back(op);
+    need.push_back(op.qmask | op.qmask2);
+  }
+  if (out.chans.size() > kStagedMaxChannels || ops.size() > kStagedMaxOps) return false;
+  // Stages in program order (the outcome of a Kraus channel depends on the
+  // order of the channels): a stage takes records while their targets fit G
+  // register qubits.
+  const uint32_t all = (1u << n) - 1u;
+  for (size_t i = 0; i < ops.size() || out.stages.empty();) {
+    TStage st;
+    uint32_t reg = 0;
+    st.op_begin = (uint32_t)out.ops.size();
+    size_t j = i;
+    for (; j < ops.size() && (uint32_t)__builtin_popcount(reg | need[j]) <= G; j++) reg |= need[j];
+    for (int b = (int)n - 1; b >= 0 && (uint32_t)__builtin_popcount(reg) < G; b--) reg |= 1u << b;
+    uint32_t bit_of[32] = {0}, g = 0;
+    for (uint32_t q = 0; q < n; q++)
+      if ((reg >> q) & 1u) {
+        bit_of[q] = g;
+        st.rl[g++] = 1u << q;
+      }
+    // Thread bits: lanes' first five on qubits distinct modulo 5 where the
+    // remaining qubits allow it (one bank group each, see traj_swz).
+    uint32_t rest = all & ~reg, classes = 0;
+    for (int round = 0; round < 2; round++)
+      for (uint32_t q = 0; q < n; q++) {
+        if (!((rest >> q) & 1u)) continue;
+        if (round == 0 && (((classes >> (q % 5)) & 1u) || st.n_tb >= 5)) continue;
+        classes |= 1u << (q % 5);
+        st.tl[st.n_tb++] = 1u << q;
+        rest &= ~(1u << q);
+      }
+    for (uint32_t t = 0; t < st.n_tb; t++) st.ts[t] = traj_swz(st.tl[t]);
+    for (uint32_t r = 0; r < (1u << G); r++)
+      for (uint32_t b = 0; b < G; b++)
+        if ((r >> b) & 1u) st.ls[r] ^= traj_swz(st.rl[b]);
+    for (; i < j; i++) {
+      TOp op = ops[i];
+      auto bit = [&](uint32_t mask) { return bit_of[__builtin_ctz(mask)]; };
+      if (op.kind == TOp::TWO) {
+        if (bit(op.qmask) < bit(op.qmask2)) {   // the matrix MSB on the higher register bit
+          std::vector<double> sw(32);
+          auto x = [](int v) { return ((v & 1) << 1) | (v >> 1); };
+          for (int r = 0; r < 4; r++)
+            for (int c = 0; c < 4; c++)
+              for (int e = 0; e < 2; e++) sw[2 * (4 * r + c) + e] = h.reals[op.off + 2 * (4 * x(r) + x(c)) + e];
+          op.off = (uint32_t)h.reals.size();
+          h.reals.insert(h.reals.end(), sw.begin(), sw.end());
+          std::swap(op.qmask, op.qmask2);
+        }
+        op.bit = bit(op.qmask) * (bit(op.qmask) - 1) / 2 + bit(op.qmask2);
+      } else if (op.kind != TOp::SIGN && op.kind != TOp::DIAG) {
+        op.bit = bit(op.qmask);
+      }
+      out.ops.push_back(op);
+    }
+    st.op_end = (uint32_t)out.ops.size();
+    out.stages.push_back(st);
+  }
+  out.ops.push_back(TOp{});   // read ahead, never run
+  return true;
+}
+
 }  // namespace aleph

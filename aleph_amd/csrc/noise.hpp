@@ -13,9 +13,11 @@
 // so shot s's outcome depends only on (seed, s), never on how shots are
 // spread over workgroups or calls.
 //
-// Device layout: one workgroup owns one trajectory at a time.  Up to 13
-// qubits (FP64, 128 KiB) the state lives in LDS and never touches HBM;
-// wider states live in a per-workgroup slice of a device buffer.
+// Device layout: one workgroup owns one trajectory at a time.  Programs of
+// one- and two-qubit gates and diagonals on 2..14 qubits keep the state in
+// registers (TStage below); other programs of up to 13 qubits (FP64, 128 KiB)
+// keep it in LDS, and wider states live in a per-workgroup slice of a device
+// buffer.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -45,6 +47,88 @@ constexpr uint32_t kNoiseMaxKraus = 64;         // branches of one Kraus channel
 constexpr uint32_t kNoiseThreadsLds = 256;
 constexpr uint32_t kNoiseThreadsWide = 1024;
 
+// ---- register-resident trajectories ----
+// A staged program is the record list of a trajectory in program order, cut
+// into stages: in a stage every thread holds the 2^G amplitudes spanned by G
+// register qubits, dense operators act on register qubits, and the state is
+// re-distributed through LDS only where a stage ends.
+//
+// Pauli channels cost nothing in the record loop.  The physical state is kept
+// as psi = X^x Z^z phi (up to a global phase) with the stored phi; a drawn
+// Pauli only changes the frame (x, z), and an operator O acts on phi as
+// F^dagger O F: rows and columns of its matrix permuted by x and signed by z,
+// diagonals and controls evaluated at the stored index XOR x.  Every channel
+// draws exactly once, so all draws of a shot are made first, one lane per
+// channel, and a prefix XOR gives the frame before every record.
+//
+// A Kraus channel whose first operator K_0 has K_0^dagger K_0 >= lam takes
+// branch 0 without looking at the state when the draw is below lam (p_0 >=
+// lam whatever the state is); the state is then left unnormalised, and the
+// branch probabilities of a channel that does need them are taken relative
+// to the norm.  K_0 is multiplied into the gate before it on the host.
+constexpr uint32_t kStagedMinQubits = 2;
+constexpr uint32_t kStagedMaxQubits = 14;     // 2^14 amplitudes in 1024 threads, 128 KiB exchange buffer
+constexpr uint32_t kStagedMaxChannels = 4096; // 5 bytes of LDS each, shared with the exchange buffer
+constexpr uint32_t kStagedMaxOps = 2048;      // 8 bytes of LDS each
+
+// Two 64-byte halves, each read with one scalar load; the next record is
+// read while the current one runs.
+struct alignas(64) TOp {
+  enum Kind : uint32_t { ONE = 0, TWO = 1, SIGN = 2, DIAG = 3, KRAUS = 4 };
+  uint32_t kind = ONE;
+  uint32_t bit = 0;        // register bit of the target (ONE, KRAUS); A (A - 1) / 2 + B, A > B the matrix MSB (TWO)
+  uint32_t qmask = 0;      // physical target (ONE, KRAUS); A's qubit (TWO); DIAG: 4-bit target list, MSB first
+  uint32_t qmask2 = 0;     // TWO: B's qubit; DIAG: target count
+  uint32_t cmask = 0;      // controls (ONE, DIAG) or the sign mask (SIGN)
+  uint32_t off = 0;        // reals: ONE with a Kraus channel: the bare gate; TWO: 4x4; DIAG: entries
+  uint32_t koff = 0;       // reals: Kraus matrices
+  uint32_t count = 0;      // Kraus branches
+  uint32_t chan = ~0u;     // Kraus channel of the record, ~0: none
+  uint32_t f0 = 0;         // frame entry before the record
+  uint32_t f1 = 0;         // frame entry before its Kraus channel
+  uint32_t pad = 0;
+  double lam = 1.0;        // lower bound of the K_0 branch's probability
+  double pad2 = 0.0;
+  double m[8] = {0};       // ONE: gate (times K_0); KRAUS: K_0
+};
+static_assert(sizeof(TOp) == 128, "TOp layout");
+
+struct TChan {
+  uint32_t pauli = 0;      // 1: Pauli channel (weights, masks), 0: Kraus
+  uint32_t count = 0;
+  uint32_t off = 0;        // reals: Pauli weights
+  uint32_t off2 = 0;       // masks: (x, z) pairs
+  double thr = 0.0;        // Kraus: draws below it take branch 0 without the state
+};
+
+struct TStage {
+  uint32_t op_begin = 0, op_end = 0;
+  uint32_t n_tb = 0;
+  uint32_t pad = 0;
+  uint32_t tl[12] = {0};   // qubit mask of thread-id bit j
+  uint32_t ts[12] = {0};   // its swizzled LDS index
+  uint32_t rl[4] = {0};    // qubit mask of register bit g
+  uint32_t ls[16] = {0};   // swizzled LDS index of register slot r
+};
+
+// LDS index swizzle of the stage exchange (linear over XOR): bits 5.. folded
+// into the low 5, so 32 lanes on bits distinct modulo 5 hit distinct banks.
+__host__ __device__ inline uint32_t traj_swz(uint32_t x) { return x ^ ((x >> 5) & 31u) ^ ((x >> 10) & 31u); }
+
+struct StagedProgram {
+  const TStage* stages = nullptr;
+  const TOp* ops = nullptr;
+  const TChan* chans = nullptr;
+  uint32_t n_stages = 0;
+  uint32_t n_ops = 0;      // records; one more follows them for the read-ahead
+  uint32_t n_chan = 0;
+  bool rare = false;       // has two-qubit matrices, diagonals other than signs, or controlled gates
+};
+
+// Register qubits of an n-qubit staged trajectory: 16 amplitudes per thread
+// where that still fills a wavefront, fewer below.
+inline uint32_t staged_reg_bits(uint32_t n) { return n >= 10 ? 4u : n == 9 ? 3u : 2u; }
+
 struct TrajProgram {
   const TrajOp* ops = nullptr;
   uint32_t n_ops = 0;
@@ -62,6 +146,9 @@ struct TrajProgram {
 // Runs `p.shots` trajectories; outcome of shot i -> out[i].  `slices` is
 // null for n <= kNoiseLdsMaxQubits, else `workgroups` * 2^n complex128.
 void launch_trajectories(hipStream_t s, const TrajProgram& p, uint32_t workgroups, void* slices, uint64_t* out);
+
+// The same for a program that lowered to stages; state in registers.
+void launch_staged(hipStream_t s, const TrajProgram& p, const StagedProgram& sp, uint64_t* out);
 
 // Workgroups and device bytes the launch for an n-qubit program uses
 // (bytes = 0 when the state fits in LDS).  `budget` bounds the slices.

@@ -116,3 +116,52 @@ def test_library_rejects_malformed_channels(hip):
     assert run(ch, 1, mask=1) == L.ERR_INVALID_ARGUMENT and "readout" in kind()[1]
     ro[:4] = [0.9, 0.1, 0.0, 1.0]
     assert run(ch, 1, mask=1) == L.OK
+
+
+def _staged_case(n: int, depth: int, seed: int):
+    """A noisy circuit of the gates that keep a trajectory's state in registers: one-qubit, controlled and
+    two-qubit gates and diagonals, under Pauli and Kraus channels that often fire: damping so strong that its
+    first branch has no useful bound, a channel of dense Kraus operators, several channels on one gate."""
+    from aleph_amd.circuit import Gate
+    rng = np.random.default_rng(seed)
+    c = Circuit(n)
+    for layer in range(depth):
+        for q in range(n):
+            c.u3(*rng.uniform(0, 2 * np.pi, 3), q)
+        for q in range(layer % 2, n - 1, 2):
+            (c.cx if layer % 3 else c.cz)(q, q + 1)
+        a, b = (int(x) for x in rng.permutation(n)[:2])
+        c.gate(Gate.Iswap(), [a, b])
+        c.gate(Gate.Ry(float(rng.uniform(0.3, 2.0))), [a], [b])
+        c.gate(Gate.CRx(float(rng.uniform(0.3, 2.0))), [b, a])
+        c.rz(float(rng.uniform(0.3, 2.0)), a)
+        c.cp(float(rng.uniform(0.3, 2.0)), a, b)
+        if n > 2:
+            x, y, z = (int(v) for v in rng.permutation(n)[:3])
+            c.ccx(x, y, z)
+            c.gate(Gate.Cz(), [x, y], [z])
+    t = 0.4
+    u = np.array([[np.cos(t), -np.sin(t)], [np.sin(t), np.cos(t)]])
+    dense = N.KrausChannel((np.sqrt(0.7) * u, np.sqrt(0.3) * u.T @ np.diag([1.0, 1j])))
+    m = N.NoiseModel()
+    m.add_all_qubit_quantum_error(N.depolarizing_error(0.1, 1), ["U3"])
+    m.add_all_qubit_quantum_error(N.depolarizing_error(0.1, 2), ["Cnot", "Cz", "Iswap"])
+    m.add_all_qubit_quantum_error(N.amplitude_damping_error(0.05), ["U3"])
+    m.add_quantum_error(N.amplitude_damping_error(0.9995), ["U3"], [n - 1])
+    m.add_quantum_error(dense, ["U3", "Rz"], [0])
+    m.add_quantum_error(N.phase_damping_error(0.3), ["U3"], [1])
+    m.add_readout_error(N.ReadoutError([[0.9, 0.1], [0.2, 0.8]]), 0)
+    return c, m
+
+
+# The smallest and largest register-resident sizes and both sides of each change of the amplitudes per thread
+# (n = 8 / 9 / 10) and of the workgroup size (n = 12 / 13 / 14).
+@pytest.mark.parametrize("n,depth,shots", [(2, 6, 400), (3, 5, 400), (8, 3, 200), (9, 3, 200), (10, 3, 150),
+                                           (11, 2, 100), (12, 2, 80), (13, 2, 40), (14, 1, 24)])
+def test_register_trajectories_equal_cpu_restatement_shot_by_shot(hip, oracle_lib, n, depth, shots):
+    # Outcomes are whole numbers: a draw would have to fall within rounding (1e-15) of a boundary to differ.
+    c, m = _staged_case(n, depth, seed=n)
+    prog, att = N.resolve(c, m)
+    want = NO.trajectory_outcomes(prog, att, m.readout_map(), n, 5, shots, shot0=3)
+    got = N.outcomes(c, m, shots, 5, backend=hip, shot_offset=3)
+    assert np.array_equal(got, want), f"{int(np.sum(got != want))} of {shots} shots differ"
