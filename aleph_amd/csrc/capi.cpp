@@ -22,6 +22,7 @@
 #include "jit.hpp"
 #include "kernels.hpp"
 #include "noise_host.hpp"
+#include "pauli.hpp"
 
 using namespace aleph;
 
@@ -86,7 +87,10 @@ constexpr size_t kScratchBytes = 2u << 20;
 // Context scratch layout (doubles): reduction partials from 0 (at most
 // kExpectGroup * kReduceBlocks of them), results from kResOffset.
 constexpr size_t kResOffset = (size_t)kExpectGroup * kReduceBlocks;
-static_assert((kResOffset + 4096) * sizeof(double) <= kScratchBytes, "scratch layout");
+// From kRecOffset the records of a Pauli sum.
+constexpr size_t kRecOffset = kResOffset + 4096;
+static_assert(kRecOffset * sizeof(double) + (1u << 20) <= kScratchBytes, "scratch layout");
+static_assert(3 * kPauliRows <= kResOffset, "scratch layout");
 
 // xoshiro256** seeded through SplitMix64.
 void rng_seed(aleph_hip_ctx* c, uint64_t seed) {
@@ -217,19 +221,104 @@ void normalize_async(aleph_hip_ctx* c, aleph_hip_state* st) {
   else launch_normalize<float>(c->stream, st->d, st->n, partials, res);
 }
 
-// validate_state (crates/aleph-sv/src/measure.rs:23-39).
-void validate(aleph_hip_ctx* c, aleph_hip_state* st, double* p0, double* p1, int32_t q) {
-  double r[3];
-  reduce(c, st, q, r);
-  const double total = r[0] + r[1];
+// The verdict of validate_state (crates/aleph-sv/src/measure.rs:23-39) on a
+// norm and a count of non-finite |psi|^2.
+void check_norm(const aleph_hip_state* st, double total, double non_finite) {
   const double tol = st->precision == ALEPH_HIP_F32 ? kFp32NormDrift
                                                     : std::sqrt(std::ldexp(1.0, (int)st->n)) * kAmplitudeTol;
-  if (r[2] != 0.0) throw make_failure(ALEPH_HIP_ERR_INVALID_STATE, "non-finite amplitude norm²", "invalid state");
+  if (non_finite != 0.0) throw make_failure(ALEPH_HIP_ERR_INVALID_STATE, "non-finite amplitude norm²", "invalid state");
   if (!std::isfinite(total) || std::fabs(total - 1.0) > tol)
     throw make_failure(ALEPH_HIP_ERR_INVALID_STATE, "state norm² deviates from 1 beyond drift budget",
                        "invalid state");
+}
+
+// validate_state as a read of its own.
+void validate(aleph_hip_ctx* c, aleph_hip_state* st, double* p0, double* p1, int32_t q) {
+  double r[3];
+  reduce(c, st, q, r);
+  check_norm(st, r[0] + r[1], r[2]);
   if (p0) *p0 = r[0];
   if (p1) *p1 = r[1];
+}
+
+// Pauli string from C-ABI arrays (checked).
+PauliTerm pauli_term(const aleph_hip_state* st, double coeff, const uint32_t* qubits, const uint8_t* paulis, uint32_t nt) {
+  if (!std::isfinite(coeff))
+    throw make_failure(ALEPH_HIP_ERR_INVALID_PAULI_STRING, "non-finite coefficient", "invalid Pauli string");
+  check_distinct(qubits, nt, st, "expectation");
+  PauliTerm tm;
+  tm.coeff = coeff;
+  for (uint32_t i = 0; i < nt; i++) {
+    need(paulis[i] <= 3, "pauli code must be 0..3");
+    const uint64_t b = 1ull << qubits[i];
+    if (paulis[i] == 1 || paulis[i] == 2) tm.x |= b;
+    if (paulis[i] == 2 || paulis[i] == 3) tm.zy |= b;
+    if (paulis[i] == 2) tm.ny++;
+  }
+  return tm;
+}
+
+// sum of coeff * <P> over the terms, with the validity check of the state.
+// Terms that fit a sweep share reads with the check (k_pauli.hip); the rest
+// are grouped by X mask, up to kExpectGroup of them per read.
+double pauli_sum(aleph_hip_ctx* c, aleph_hip_state* st, const std::vector<PauliTerm>& terms) {
+  const bool f64 = st->precision == ALEPH_HIP_F64;
+  double* partials = c->d_scratch;
+  double* res = c->d_scratch + kResOffset;
+  double total = 0.0;
+  const PauliPlan plan = plan_pauli_sum(terms, st->n);
+  if (plan.sweeps.empty()) {
+    validate(c, st, nullptr, nullptr, -1);
+  } else {
+    void* dev = c->d_scratch + kRecOffset;
+    const size_t room = kScratchBytes - kRecOffset * sizeof(double);
+    if (f64) run_pauli_sweeps<double>(c->stream, st->d, st->n, plan, terms, dev, room, partials, c->h_pinned);
+    else run_pauli_sweeps<float>(c->stream, st->d, st->n, plan, terms, dev, room, partials, c->h_pinned);
+    check_norm(st, c->h_pinned[1], c->h_pinned[2]);
+    total = c->h_pinned[0];
+  }
+  struct Launch {
+    uint64_t x;
+    std::vector<uint32_t> ids;
+  };
+  std::vector<Launch> launches;      // plan.rest is ordered by X mask
+  for (uint32_t t : plan.rest) {
+    if (launches.empty() || launches.back().x != terms[t].x || launches.back().ids.size() == kExpectGroup)
+      launches.push_back(Launch{terms[t].x, {}});
+    launches.back().ids.push_back(t);
+  }
+  // Results of up to 256 launches are read back per host synchronisation.
+  const size_t per_sync = 256;
+  std::vector<double> host(per_sync * kExpectGroup);
+  for (size_t l0 = 0; l0 < launches.size(); l0 += per_sync) {
+    const size_t nl = std::min(per_sync, launches.size() - l0);
+    for (size_t j = 0; j < nl; j++) {
+      const Launch& L = launches[l0 + j];
+      uint64_t zy[kExpectGroup];
+      uint8_t use_im[kExpectGroup];
+      for (size_t t = 0; t < L.ids.size(); t++) {
+        zy[t] = terms[L.ids[t]].zy;
+        use_im[t] = (uint8_t)(terms[L.ids[t]].ny & 1);
+      }
+      double* out_j = res + j * kExpectGroup;
+      if (f64)
+        launch_expect_group<double>(c->stream, st->d, st->n, L.x, zy, use_im, (uint32_t)L.ids.size(), partials, out_j);
+      else
+        launch_expect_group<float>(c->stream, st->d, st->n, L.x, zy, use_im, (uint32_t)L.ids.size(), partials, out_j);
+    }
+    ALEPH_HIP_CHECK(hipMemcpyAsync(host.data(), res, nl * kExpectGroup * sizeof(double), hipMemcpyDeviceToHost,
+                                   c->stream));
+    ALEPH_HIP_CHECK(hipStreamSynchronize(c->stream));
+    for (size_t j = 0; j < nl; j++)
+      for (size_t t = 0; t < launches[l0 + j].ids.size(); t++) {
+        // Pairs {i, i ^ x} are summed once, so they carry a factor 2;
+        // Re(i^ny (re + i im)) is +re, -im, -re, +im.
+        const PauliTerm& tm = terms[launches[l0 + j].ids[t]];
+        const double acc = host[j * kExpectGroup + t] * (tm.x == 0 ? 1.0 : 2.0);
+        total += tm.coeff * (((tm.ny & 3) == 1 || (tm.ny & 3) == 2) ? -acc : acc);
+      }
+  }
+  return total;
 }
 
 struct DevBuf {
@@ -1037,43 +1126,15 @@ aleph_hip_status aleph_hip_expectation(aleph_hip_ctx* c, aleph_hip_state* st, do
   return guarded(c, [&] {
     check_state(c, st);
     need(out != nullptr && (nt == 0 || (qubits && paulis)), "null argument");
-    validate(c, st, nullptr, nullptr, -1);
-    if (!std::isfinite(coeff))
-      throw make_failure(ALEPH_HIP_ERR_INVALID_PAULI_STRING, "non-finite coefficient", "invalid Pauli string");
-    check_distinct(qubits, nt, st, "expectation");
-    uint64_t x = 0, zy = 0;
-    int ny = 0;
-    for (uint32_t i = 0; i < nt; i++) {
-      need(paulis[i] <= 3, "pauli code must be 0..3");
-      const uint64_t b = 1ull << qubits[i];
-      if (paulis[i] == 1) x |= b;
-      if (paulis[i] == 2) { x |= b; zy |= b; ny++; }
-      if (paulis[i] == 3) zy |= b;
+    std::vector<PauliTerm> terms;
+    try {
+      terms.push_back(pauli_term(st, coeff, qubits, paulis, nt));
+    } catch (const Failure&) {
+      validate(c, st, nullptr, nullptr, -1);   // an invalid state is reported before a bad string
+      throw;
     }
-    // One term through the grouped kernel: for x != 0 it sums over the pairs
-    // {i, i ^ x}, so every amplitude is read once (a per-element read of
-    // psi[i] and psi[i ^ x] reads the state twice when x holds high qubits).
-    double* partials = c->d_scratch;
-    double* res = c->d_scratch + kResOffset;
-    const uint64_t zys[1] = {zy};
-    const bool odd = x != 0 && (__builtin_popcountll(x & zy) & 1);
-    const uint8_t use_im[1] = {(uint8_t)odd};
-    if (st->precision == ALEPH_HIP_F64)
-      launch_expect_group<double>(c->stream, st->d, st->n, x, zys, use_im, 1u, partials, res);
-    else
-      launch_expect_group<float>(c->stream, st->d, st->n, x, zys, use_im, 1u, partials, res);
-    ALEPH_HIP_CHECK(hipMemcpyAsync(c->h_pinned, res, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    ALEPH_HIP_CHECK(hipStreamSynchronize(c->stream));
-    const double acc = c->h_pinned[0];
-    const double re = x == 0 ? acc : (odd ? 0.0 : 2.0 * acc), im = odd ? 2.0 * acc : 0.0;
-    double v;
-    switch (ny & 3) {  // Re(i^ny * (re + i im))
-      case 0: v = re; break;
-      case 1: v = -im; break;
-      case 2: v = -re; break;
-      default: v = im; break;
-    }
-    *out = coeff * v;
+    terms[0].coeff = 1.0;
+    *out = coeff * pauli_sum(c, st, terms);
   });
 }
 
@@ -1083,99 +1144,21 @@ aleph_hip_status aleph_hip_expectation_sum(aleph_hip_ctx* c, aleph_hip_state* st
   return guarded(c, [&] {
     check_state(c, st);
     need(out != nullptr && (n_terms == 0 || (coeffs && offsets)), "null argument");
-    validate(c, st, nullptr, nullptr, -1);
-    struct Term {
-      uint64_t x, zy;
-      int ny;
-      double coeff;
-    };
-    std::vector<Term> terms(n_terms);
-    for (uint32_t t = 0; t < n_terms; t++) {
-      need(offsets[t] <= offsets[t + 1], "term offsets must be non-decreasing");
-      const uint32_t nt = offsets[t + 1] - offsets[t];
-      need(nt == 0 || (qubits && paulis), "null argument");
-      if (!std::isfinite(coeffs[t]))
-        throw make_failure(ALEPH_HIP_ERR_INVALID_PAULI_STRING, "non-finite coefficient", "invalid Pauli string");
-      check_distinct(qubits + offsets[t], nt, st, "expectation");
-      Term& tm = terms[t];
-      tm = Term{0, 0, 0, coeffs[t]};
-      for (uint32_t i = offsets[t]; i < offsets[t + 1]; i++) {
-        need(paulis[i] <= 3, "pauli code must be 0..3");
-        const uint64_t b = 1ull << qubits[i];
-        if (paulis[i] == 1) tm.x |= b;
-        if (paulis[i] == 2) { tm.x |= b; tm.zy |= b; tm.ny++; }
-        if (paulis[i] == 3) tm.zy |= b;
+    std::vector<PauliTerm> terms;
+    terms.reserve(n_terms);
+    try {
+      for (uint32_t t = 0; t < n_terms; t++) {
+        need(offsets[t] <= offsets[t + 1], "term offsets must be non-decreasing");
+        const uint32_t nt = offsets[t + 1] - offsets[t];
+        need(nt == 0 || (qubits && paulis), "null argument");
+        const PauliTerm tm = pauli_term(st, coeffs[t], qubits + offsets[t], paulis + offsets[t], nt);
+        if (tm.coeff != 0.0) terms.push_back(tm);
       }
+    } catch (const Failure&) {
+      validate(c, st, nullptr, nullptr, -1);   // an invalid state is reported before a bad string
+      throw;
     }
-    // Terms are grouped by X mask; each group of up to kExpectGroup terms is
-    // one read of the state (pairs {i, i ^ x} read once each), so a
-    // diagonal Hamiltonian such as a MaxCut sum costs one sweep per 16 terms.
-    double* partials = c->d_scratch;
-    double* res = c->d_scratch + kResOffset;
-    std::vector<uint32_t> order(n_terms);
-    for (uint32_t t = 0; t < n_terms; t++) order[t] = t;
-    std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return terms[a].x < terms[b].x; });
-    struct Launch {
-      uint64_t x;
-      std::vector<uint32_t> ids;
-    };
-    std::vector<Launch> launches;
-    for (uint32_t k = 0; k < n_terms; k++) {
-      const Term& tm = terms[order[k]];
-      if (tm.coeff == 0.0) continue;
-      if (launches.empty() || launches.back().x != tm.x || launches.back().ids.size() == kExpectGroup)
-        launches.push_back(Launch{tm.x, {}});
-      launches.back().ids.push_back(order[k]);
-    }
-    // Results of up to 256 launches are read back per host synchronisation.
-    const size_t per_sync = 256;
-    std::vector<double> host(per_sync * kExpectGroup);
-    double total = 0.0;
-    for (size_t l0 = 0; l0 < launches.size(); l0 += per_sync) {
-      const size_t nl = std::min(per_sync, launches.size() - l0);
-      for (size_t j = 0; j < nl; j++) {
-        const Launch& L = launches[l0 + j];
-        uint64_t zy[kExpectGroup];
-        uint8_t use_im[kExpectGroup];
-        for (size_t t = 0; t < L.ids.size(); t++) {
-          const Term& tm = terms[L.ids[t]];
-          zy[t] = tm.zy;
-          use_im[t] = (uint8_t)(tm.x != 0 && (__builtin_popcountll(tm.x & tm.zy) & 1));
-        }
-        double* out_j = res + j * kExpectGroup;
-        if (st->precision == ALEPH_HIP_F64)
-          launch_expect_group<double>(c->stream, st->d, st->n, L.x, zy, use_im, (uint32_t)L.ids.size(), partials,
-                                      out_j);
-        else
-          launch_expect_group<float>(c->stream, st->d, st->n, L.x, zy, use_im, (uint32_t)L.ids.size(), partials,
-                                     out_j);
-      }
-      ALEPH_HIP_CHECK(hipMemcpyAsync(host.data(), res, nl * kExpectGroup * sizeof(double), hipMemcpyDeviceToHost,
-                                     c->stream));
-      ALEPH_HIP_CHECK(hipStreamSynchronize(c->stream));
-      for (size_t j = 0; j < nl; j++) {
-        const Launch& L = launches[l0 + j];
-        for (size_t t = 0; t < L.ids.size(); t++) {
-          const Term& tm = terms[L.ids[t]];
-          // (re, im) of sum_i conj(psi[i ^ x]) (-1)^{|i & zy|} psi[i]: the pair
-          // sums count each pair once, so they carry a factor 2.
-          double re = 0.0, im = 0.0;
-          const double acc = host[j * kExpectGroup + t];
-          if (tm.x == 0) re = acc;
-          else if (__builtin_popcountll(tm.x & tm.zy) & 1) im = 2.0 * acc;
-          else re = 2.0 * acc;
-          double v;
-          switch (tm.ny & 3) {  // Re(i^ny * (re + i im))
-            case 0: v = re; break;
-            case 1: v = -im; break;
-            case 2: v = -re; break;
-            default: v = im; break;
-          }
-          total += tm.coeff * v;
-        }
-      }
-    }
-    *out = total;
+    *out = pauli_sum(c, st, terms);
   });
 }
 

@@ -34,6 +34,16 @@ struct Failure {
     }                                                                                 \
   } while (0)
 
+// Device memory that is the same for a whole workgroup and not written while
+// the kernel runs (programs, descriptors), through the constant address
+// space: read with scalar loads, so the values stay in SGPRs.
+template <typename V>
+using Prog = const __attribute__((address_space(4))) V;
+template <typename V>
+__device__ __forceinline__ Prog<V>* prog(const V* p) {
+  return (Prog<V>*)(uintptr_t)p;
+}
+
 // Raises kernel `fn`'s dynamic LDS limit to the CU's 160 KiB, once per
 // (device, kernel).  Thread-safe: plans are built and launched from several
 // host threads, and a process may drive more than one device.

@@ -338,16 +338,6 @@ __device__ __forceinline__ double flip_hi(double x, uint32_t s) {
 // Plain components: arrays of the HIP vector type stay in scratch memory.
 using Amp = C2<double>;
 
-// Program memory through the constant address space: records and matrices are
-// the same for the whole workgroup and never written while the kernel runs,
-// so they are read with scalar loads and their values stay in SGPRs.
-template <typename V>
-using Prog = const __attribute__((address_space(4))) V;
-template <typename V>
-__device__ __forceinline__ Prog<V>* prog(const V* p) {
-  return (Prog<V>*)(uintptr_t)p;
-}
-
 struct Mat2 {
   double v[8];
 };

@@ -460,6 +460,11 @@ void launch_reduce_branch(hipStream_t st, const void* state, uint32_t n, int32_t
   ALEPH_HIP_CHECK(hipGetLastError());
 }
 
+void launch_reduce_rows(hipStream_t st, const double* partials, uint32_t rows, double* out) {
+  hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kThreads), 0, st, partials, rows, 3u, out);
+  ALEPH_HIP_CHECK(hipGetLastError());
+}
+
 template <typename T>
 void launch_sum_p2(hipStream_t st, const void* state, uint32_t n, double* partials, double* out) {
   const uint64_t len = 1ull << n;

@@ -121,6 +121,10 @@ void launch_reduce_branch(hipStream_t s, const void* state, uint32_t n, int32_t 
 // out[0] = sum of |a|^4, out[1] = sum of |a|^2, out[2] = non-finite count (same partials as above).
 template <typename T>
 void launch_sum_p2(hipStream_t s, const void* state, uint32_t n, double* partials, double* out);
+// Column sums of `rows` rows of three partials into out[0..3) (compensated, one workgroup; out may be
+// pinned host memory).
+void launch_reduce_rows(hipStream_t s, const double* partials, uint32_t rows, double* out);
+
 // FP64 norm into res (the reduce above), then psi /= sqrt(norm) on the device (no host sync).
 template <typename T>
 void launch_normalize(hipStream_t s, void* state, uint32_t n, double* partials, double* res);
