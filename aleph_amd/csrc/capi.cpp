@@ -89,7 +89,8 @@ constexpr size_t kScratchBytes = 2u << 20;
 constexpr size_t kResOffset = (size_t)kExpectGroup * kReduceBlocks;
 // From kRecOffset the records of a Pauli sum.
 constexpr size_t kRecOffset = kResOffset + 4096;
-static_assert(kRecOffset * sizeof(double) + (1u << 20) <= kScratchBytes, "scratch layout");
+constexpr size_t kScratchDoubles = kScratchBytes / sizeof(double);
+static_assert(kRecOffset + (1u << 17) <= kScratchDoubles, "scratch layout");
 static_assert(3 * kPauliRows <= kResOffset, "scratch layout");
 
 // xoshiro256** seeded through SplitMix64.
@@ -205,10 +206,10 @@ void* noalloc_scratch_address(int dev) {
 // Σ|ψ|² over bit q clear / set, non-finite count (q < 0: everything in [0]).
 void reduce(aleph_hip_ctx* c, aleph_hip_state* st, int32_t q, double out[3]) {
   double* partials = c->d_scratch;
-  double* res = c->d_scratch + kResOffset;
-  if (st->precision == ALEPH_HIP_F64) launch_reduce_branch<double>(c->stream, st->d, st->n, q, partials, res);
-  else launch_reduce_branch<float>(c->stream, st->d, st->n, q, partials, res);
-  ALEPH_HIP_CHECK(hipMemcpyAsync(c->h_pinned, res, 3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  if (st->precision == ALEPH_HIP_F64)
+    launch_reduce_branch<double>(c->stream, st->d, st->n, q, partials, c->h_pinned);
+  else
+    launch_reduce_branch<float>(c->stream, st->d, st->n, q, partials, c->h_pinned);
   ALEPH_HIP_CHECK(hipStreamSynchronize(c->stream));
   for (int i = 0; i < 3; i++) out[i] = c->h_pinned[i];
 }
@@ -223,11 +224,15 @@ void normalize_async(aleph_hip_ctx* c, aleph_hip_state* st) {
 
 // The verdict of validate_state (crates/aleph-sv/src/measure.rs:23-39) on a
 // norm and a count of non-finite |psi|^2.
-void check_norm(const aleph_hip_state* st, double total, double non_finite) {
+bool norm_ok(const aleph_hip_state* st, double total) {
   const double tol = st->precision == ALEPH_HIP_F32 ? kFp32NormDrift
                                                     : std::sqrt(std::ldexp(1.0, (int)st->n)) * kAmplitudeTol;
+  return std::isfinite(total) && std::fabs(total - 1.0) <= tol;
+}
+
+void check_norm(const aleph_hip_state* st, double total, double non_finite) {
   if (non_finite != 0.0) throw make_failure(ALEPH_HIP_ERR_INVALID_STATE, "non-finite amplitude norm²", "invalid state");
-  if (!std::isfinite(total) || std::fabs(total - 1.0) > tol)
+  if (!norm_ok(st, total))
     throw make_failure(ALEPH_HIP_ERR_INVALID_STATE, "state norm² deviates from 1 beyond drift budget",
                        "invalid state");
 }
@@ -271,7 +276,7 @@ double pauli_sum(aleph_hip_ctx* c, aleph_hip_state* st, const std::vector<PauliT
     validate(c, st, nullptr, nullptr, -1);
   } else {
     void* dev = c->d_scratch + kRecOffset;
-    const size_t room = kScratchBytes - kRecOffset * sizeof(double);
+    const size_t room = (kScratchDoubles - kRecOffset) * sizeof(double);
     if (f64) run_pauli_sweeps<double>(c->stream, st->d, st->n, plan, terms, dev, room, partials, c->h_pinned);
     else run_pauli_sweeps<float>(c->stream, st->d, st->n, plan, terms, dev, room, partials, c->h_pinned);
     check_norm(st, c->h_pinned[1], c->h_pinned[2]);
@@ -368,29 +373,48 @@ aleph_hip_status measure_impl(aleph_hip_ctx* c, aleph_hip_state* st, uint32_t qu
   });
 }
 
+// Draws the shots and checks the state on the sampler's own block sums: one
+// read of the state.  On an invalid state the generator goes back to `rng`
+// and nothing is written to `out`.
+void sample_checked(aleph_hip_ctx* c, aleph_hip_state* st, double* blocks, double* misc, const double* du,
+                    uint64_t* dout, uint32_t shots, uint64_t* out, const uint64_t rng[4]) {
+  if (st->precision == ALEPH_HIP_F64)
+    launch_sample<double>(c->stream, st->d, st->n, blocks, misc, du, shots, dout, c->h_pinned);
+  else
+    launch_sample<float>(c->stream, st->d, st->n, blocks, misc, du, shots, dout, c->h_pinned);
+  ALEPH_HIP_CHECK(hipStreamSynchronize(c->stream));
+  if (!norm_ok(st, c->h_pinned[0])) {
+    std::copy(rng, rng + 4, c->rng);
+    validate(c, st, nullptr, nullptr, -1);   // the error, with its reason
+  }
+  ALEPH_HIP_CHECK(hipMemcpyAsync(out, dout, shots * sizeof(uint64_t), hipMemcpyDeviceToHost, c->stream));
+  ALEPH_HIP_CHECK(hipStreamSynchronize(c->stream));
+}
+
 aleph_hip_status sample_impl(aleph_hip_ctx* c, aleph_hip_state* st, const double* uniforms, uint32_t shots,
                              uint64_t* out) {
   return guarded(c, [&] {
     check_state(c, st);
     need(shots == 0 || out != nullptr, "null output");
-    validate(c, st, nullptr, nullptr, -1);
-    if (shots == 0) return;
+    if (shots == 0) {
+      validate(c, st, nullptr, nullptr, -1);
+      return;
+    }
+    uint64_t rng[4];
+    std::copy(c->rng, c->rng + 4, rng);
     std::vector<double> u(shots);
     for (uint32_t i = 0; i < shots; i++) u[i] = uniforms ? uniforms[i] : rng_uniform(c);
+    // Workspace: the context scratch when it is large enough (every region is
+    // written before it is read), else one allocation.
     const uint64_t nb = st->n > kSampleBlockBits ? (1ull << (st->n - kSampleBlockBits)) : 1ull;
-    DevBuf blocks(2 * nb * sizeof(double));
-    DevBuf misc(64 * sizeof(double));
-    DevBuf du(shots * sizeof(double));
-    DevBuf dout(shots * sizeof(uint64_t));
-    ALEPH_HIP_CHECK(hipMemcpyAsync(du.p, u.data(), shots * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    if (st->precision == ALEPH_HIP_F64)
-      launch_sample<double>(c->stream, st->d, st->n, (double*)blocks.p, (double*)misc.p, (const double*)du.p, shots,
-                            (uint64_t*)dout.p);
-    else
-      launch_sample<float>(c->stream, st->d, st->n, (double*)blocks.p, (double*)misc.p, (const double*)du.p, shots,
-                           (uint64_t*)dout.p);
-    ALEPH_HIP_CHECK(hipMemcpyAsync(out, dout.p, shots * sizeof(uint64_t), hipMemcpyDeviceToHost, c->stream));
-    ALEPH_HIP_CHECK(hipStreamSynchronize(c->stream));
+    const size_t doubles = 2 * nb + 64 + 2 * (size_t)shots;
+    std::unique_ptr<DevBuf> own;
+    if (doubles > kScratchDoubles) own = std::make_unique<DevBuf>(doubles * sizeof(double));
+    double* blocks = own ? (double*)own->p : c->d_scratch;
+    double *misc = blocks + 2 * nb, *du = misc + 64;
+    uint64_t* dout = (uint64_t*)(du + shots);
+    ALEPH_HIP_CHECK(hipMemcpyAsync(du, u.data(), shots * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    sample_checked(c, st, blocks, misc, du, dout, shots, out, rng);
   });
 }
 
@@ -1101,8 +1125,10 @@ aleph_hip_status aleph_hip_sample_with_uniforms_noalloc(aleph_hip_ctx* c, aleph_
       throw f;
     }
     need(c->noalloc_scratch != nullptr, "sampler scratch not set up");
-    validate(c, st, nullptr, nullptr, -1);   // context scratch, allocated with the context
-    if (shots == 0) return;
+    if (shots == 0) {
+      validate(c, st, nullptr, nullptr, -1);   // context scratch, allocated with the context
+      return;
+    }
     // Every region is written before it is read (block sums, their prefix and
     // total by the first two kernels, the uniforms by the copy, every result
     // slot by the shot kernel), so nothing needs clearing between calls.
@@ -1112,12 +1138,9 @@ aleph_hip_status aleph_hip_sample_with_uniforms_noalloc(aleph_hip_ctx* c, aleph_
     double* du = reinterpret_cast<double*>(base + kNoAllocUniOff);
     uint64_t* dout = reinterpret_cast<uint64_t*>(base + kNoAllocOutOff);
     ALEPH_HIP_CHECK(hipMemcpyAsync(du, u, shots * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    if (st->precision == ALEPH_HIP_F64)
-      launch_sample<double>(c->stream, st->d, st->n, sums, misc, du, shots, dout);
-    else
-      launch_sample<float>(c->stream, st->d, st->n, sums, misc, du, shots, dout);
-    ALEPH_HIP_CHECK(hipMemcpyAsync(out, dout, shots * sizeof(uint64_t), hipMemcpyDeviceToHost, c->stream));
-    ALEPH_HIP_CHECK(hipStreamSynchronize(c->stream));
+    uint64_t rng[4];   // the caller's uniforms: the generator is not used
+    std::copy(c->rng, c->rng + 4, rng);
+    sample_checked(c, st, sums, misc, du, dout, shots, out, rng);
   });
 }
 
@@ -1167,10 +1190,10 @@ aleph_hip_status aleph_hip_linear_xeb(aleph_hip_ctx* c, aleph_hip_state* st, dou
     check_state(c, st);
     need(out != nullptr, "null output");
     double* partials = c->d_scratch;
-    double* res = c->d_scratch + kResOffset;
-    if (st->precision == ALEPH_HIP_F64) launch_sum_p2<double>(c->stream, st->d, st->n, partials, res);
-    else launch_sum_p2<float>(c->stream, st->d, st->n, partials, res);
-    ALEPH_HIP_CHECK(hipMemcpyAsync(c->h_pinned, res, 3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    if (st->precision == ALEPH_HIP_F64)
+      launch_sum_p2<double>(c->stream, st->d, st->n, partials, c->h_pinned);
+    else
+      launch_sum_p2<float>(c->stream, st->d, st->n, partials, c->h_pinned);
     ALEPH_HIP_CHECK(hipStreamSynchronize(c->stream));
     if (c->h_pinned[2] != 0.0) throw make_failure(ALEPH_HIP_ERR_INVALID_STATE, "non-finite amplitude", "invalid state");
     *out = std::ldexp(c->h_pinned[0], (int)st->n) - 1.0;
@@ -1319,18 +1342,32 @@ aleph_hip_status aleph_hip_probabilities(aleph_hip_ctx* c, aleph_hip_state* st, 
   return guarded(c, [&] {
     check_state(c, st);
     need(out != nullptr && (nq == 0 || qubits), "null argument");
-    validate(c, st, nullptr, nullptr, -1);
-    check_distinct(qubits, nq, st, "probabilities");
+    // The check rides on the histogram's read; wherever there is none, an
+    // invalid state is still reported before anything else.
+    try {
+      check_distinct(qubits, nq, st, "probabilities");
+      need(nq <= 30, "at most 30 marginal qubits");
+    } catch (const Failure&) {
+      validate(c, st, nullptr, nullptr, -1);
+      throw;
+    }
     if (nq == 0) {
+      validate(c, st, nullptr, nullptr, -1);
       out[0] = 1.0;
       return;
     }
-    need(nq <= 30, "at most 30 marginal qubits");
-    const size_t bins = 1ull << nq;
-    DevBuf d(bins * sizeof(double));
-    if (st->precision == ALEPH_HIP_F64) launch_marginal<double>(c->stream, st->d, st->n, nq, qubits, (double*)d.p);
-    else launch_marginal<float>(c->stream, st->d, st->n, nq, qubits, (double*)d.p);
-    ALEPH_HIP_CHECK(hipMemcpyAsync(out, d.p, bins * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    // Bins in the context scratch behind the reduction's partials when they fit.
+    const size_t bins = 1ull << nq, at = 3 * (size_t)kReduceBlocks;
+    std::unique_ptr<DevBuf> own;
+    if (at + bins > kScratchDoubles) own = std::make_unique<DevBuf>(bins * sizeof(double));
+    double* d = own ? (double*)own->p : c->d_scratch + at;
+    const bool checked =
+        st->precision == ALEPH_HIP_F64
+            ? launch_marginal<double>(c->stream, st->d, st->n, nq, qubits, d, c->d_scratch, c->h_pinned)
+            : launch_marginal<float>(c->stream, st->d, st->n, nq, qubits, d, c->d_scratch, c->h_pinned);
+    if (checked) ALEPH_HIP_CHECK(hipStreamSynchronize(c->stream));
+    if (!checked || !norm_ok(st, c->h_pinned[0])) validate(c, st, nullptr, nullptr, -1);
+    ALEPH_HIP_CHECK(hipMemcpyAsync(out, d, bins * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     ALEPH_HIP_CHECK(hipStreamSynchronize(c->stream));
   });
 }

@@ -6,6 +6,8 @@
 #include "common.hpp"
 #include "kernels.hpp"
 
+#include <algorithm>
+
 namespace aleph {
 namespace {
 
@@ -61,29 +63,56 @@ __device__ void block_reduce(KSum (&v)[N]) {
   }
 }
 
-// Grid-stride sweeps take kUnroll amplitudes per thread per iteration, all
-// loads issued before any arithmetic, so each wave keeps several 16-byte
-// loads in flight.
+// Compensated column sums of `rows` rows of three partials; valid in thread 0.
+__device__ __forceinline__ void sum_rows(const double* partials, uint32_t rows, KSum (&v)[3]) {
+  for (int w = 0; w < 3; w++) v[w] = KSum{0, 0};
+#pragma unroll 4
+  for (uint32_t b = threadIdx.x; b < rows; b += blockDim.x) {
+    double x[3];
+#pragma unroll
+    for (int w = 0; w < 3; w++) x[w] = partials[3 * (uint64_t)b + w];
+#pragma unroll
+    for (int w = 0; w < 3; w++) kadd(v[w], x[w]);
+  }
+  block_reduce<3>(v);
+}
+
+// A workgroup's three sums (valid in thread 0) into its row.  A second launch
+// adds the rows: with the last workgroup of the same launch doing it, the
+// device-wide fence of every workgroup cost more (19 qubits: 18 us against
+// 6.6 + 5.7).
+__device__ __forceinline__ void store_row(const KSum (&v)[3], double* partials) {
+  if (threadIdx.x == 0)
+    for (int w = 0; w < 3; w++) partials[3 * (uint64_t)blockIdx.x + w] = v[w].s + v[w].c;
+}
+
+// Sweeps take kUnroll amplitudes per thread per iteration, all loads issued
+// before any arithmetic, so each wave keeps several 16-byte loads in flight.
 constexpr int kUnroll = 4;
+constexpr int kMarginalUnroll = 8;
+// Workgroups of a reduction: four per CU, a tile of kUnroll * kThreads
+// consecutive amplitudes at a time, so that a row of partials sums many reads
+// (the second launch then takes 7 us at 27 qubits where 4096 rows took 16).
+constexpr uint32_t kReduceGrid = 1024;
 
 // MODE 0: [sum over bit q clear, sum over bit q set, non-finite count] of p = |a|^2.
 // MODE 1: [sum of p^2, sum of p, non-finite count] (collision probability).
 template <typename T, int MODE>
-__global__ void __launch_bounds__(kThreads) k_reduce_branch(const C2<T>* __restrict__ s, uint64_t len,
-                                                            uint64_t qmask, double* __restrict__ partials) {
+__global__ void __launch_bounds__(kThreads) k_reduce_branch(const C2<T>* __restrict__ s, uint64_t len, uint64_t qmask,
+                                                            double* __restrict__ partials) {
   KSum v[3] = {{0, 0}, {0, 0}, {0, 0}};
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t i0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i0 < len; i0 += kUnroll * stride) {
+  const uint64_t tile = kUnroll * kThreads;
+  for (uint64_t i0 = (uint64_t)blockIdx.x * tile + threadIdx.x; i0 < len; i0 += gridDim.x * tile) {
     C2<T> a[kUnroll];
 #pragma unroll
     for (int u = 0; u < kUnroll; u++) {
-      const uint64_t i = i0 + u * stride;
+      const uint64_t i = i0 + u * kThreads;
       if (i < len) a[u] = s[i];
       else a[u].x = a[u].y = 0;
     }
 #pragma unroll
     for (int u = 0; u < kUnroll; u++) {
-      const uint64_t i = i0 + u * stride;
+      const uint64_t i = i0 + u * kThreads;
       const double p = (double)a[u].x * (double)a[u].x + (double)a[u].y * (double)a[u].y;
       if (!isfinite(p)) {
         v[2].s += 1.0;
@@ -99,22 +128,16 @@ __global__ void __launch_bounds__(kThreads) k_reduce_branch(const C2<T>* __restr
     }
   }
   block_reduce<3>(v);
-  if (threadIdx.x == 0) {
-    partials[3 * blockIdx.x + 0] = v[0].s + v[0].c;
-    partials[3 * blockIdx.x + 1] = v[1].s + v[1].c;
-    partials[3 * blockIdx.x + 2] = v[2].s;
-  }
+  store_row(v, partials);
 }
 
-// Sums `count` interleaved groups of `width` partials into out[0..width).
+// Sums `count` rows of three partials into out[0..3) (device or pinned memory).
 __global__ void __launch_bounds__(kThreads) k_reduce_final(const double* __restrict__ partials, uint32_t count,
-                                                           uint32_t width, double* __restrict__ out) {
-  KSum v[3] = {{0, 0}, {0, 0}, {0, 0}};
-  for (uint32_t b = threadIdx.x; b < count; b += blockDim.x)
-    for (uint32_t w = 0; w < width && w < 3; w++) kadd(v[w], partials[width * b + w]);
-  block_reduce<3>(v);
+                                                           double* out) {
+  KSum v[3];
+  sum_rows(partials, count, v);
   if (threadIdx.x == 0)
-    for (uint32_t w = 0; w < width && w < 3; w++) out[w] = v[w].s + v[w].c;
+    for (int w = 0; w < 3; w++) out[w] = v[w].s + v[w].c;
 }
 
 template <typename T>
@@ -218,32 +241,91 @@ __global__ void __launch_bounds__(kThreads) k_reduce_columns(const double* __res
   }
 }
 
+// Marginal histogram.  The index bits are split so that a thread's loop runs
+// over bits outside the marginal only: its bin is fixed, the sum stays in a
+// register, and one atomic per thread (into the workgroup's LDS bins, then
+// one per workgroup and bin) replaces one per amplitude.  Thread bits are the
+// low 8 (coalesced); loop bits the lowest bits above them that the marginal
+// does not ask for, as many as leave kMarginalGroups workgroups; the rest
+// number the workgroups.  The norm of the validity check is the sum of the
+// same reads.  27 qubits FP64, 9 of them random: 678 us and a separate check
+// of 428 us -> 352 us (6.1 TB/s, what a plain read reaches; 424 us with four
+// loads in flight instead of eight).
+constexpr uint32_t kMarginalGroups = 2048;
+// Marginal qubits above the thread bits: with more, workgroups would outnumber
+// the rows of the reduction, and bins the atomics saved (k_marginal_wide).
+constexpr uint32_t kMarginalHigh = 12;
+static_assert((1u << kMarginalHigh) <= kReduceBlocks, "one row per workgroup");
+
+struct MarginalBits {
+  uint64_t loop_mask;          // index bits of a thread's loop
+  uint32_t n_group;            // workgroup bits
+  uint32_t group_pos[40];      // their index bits
+  uint32_t n_low;              // marginal bits among the thread bits
+  uint32_t low_pos[8], low_bin[8];    // their index bits and bin bits
+  uint32_t n_high;             // marginal bits among the workgroup bits
+  uint32_t high_pos[32], high_bin[32];
+};
+
+template <typename T>
+__global__ void __launch_bounds__(kThreads) k_marginal(const C2<T>* __restrict__ s, uint64_t len, MarginalBits d,
+                                                       double* __restrict__ bins, double* __restrict__ partials) {
+  __shared__ double h[kThreads];
+  const uint32_t tid = threadIdx.x;
+  h[tid] = 0.0;
+  uint64_t base = tid;
+  for (uint32_t j = 0; j < d.n_group; j++) base |= (uint64_t)((blockIdx.x >> j) & 1u) << d.group_pos[j];
+  double acc[kMarginalUnroll];
+#pragma unroll
+  for (int u = 0; u < kMarginalUnroll; u++) acc[u] = 0.0;
+  if (tid < len) {
+    uint64_t x = 0;
+    bool more = true;
+    while (more) {
+      C2<T> a[kMarginalUnroll];
+#pragma unroll
+      for (int u = 0; u < kMarginalUnroll; u++) {
+        if (more) a[u] = s[base | x];
+        else a[u].x = a[u].y = 0;
+        x = ((x | ~d.loop_mask) + 1) & d.loop_mask;      // next setting of the loop bits
+        more = more && x != 0;
+      }
+#pragma unroll
+      for (int u = 0; u < kMarginalUnroll; u++)
+        acc[u] += (double)a[u].x * (double)a[u].x + (double)a[u].y * (double)a[u].y;
+    }
+  }
+  double mine = 0.0;
+#pragma unroll
+  for (int u = 0; u < kMarginalUnroll; u++) mine += acc[u];
+  uint32_t low = 0;
+  for (uint32_t j = 0; j < d.n_low; j++) low |= ((tid >> d.low_pos[j]) & 1u) << j;
+  __syncthreads();
+  atomicAdd(&h[low], mine);
+  KSum v[3] = {{mine, 0}, {0, 0}, {0, 0}};
+  block_reduce<3>(v);
+  __syncthreads();
+  if (tid < (1u << d.n_low)) {
+    uint32_t bin = 0;
+    for (uint32_t j = 0; j < d.n_low; j++) bin |= ((tid >> j) & 1u) << d.low_bin[j];
+    for (uint32_t j = 0; j < d.n_high; j++) bin |= (uint32_t)((base >> d.high_pos[j]) & 1ull) << d.high_bin[j];
+    atomicAdd(&bins[bin], h[tid]);
+  }
+  store_row(v, partials);
+}
+
 struct Qubits64 { uint32_t q[64]; };
 
-// LDS-privatised histogram (k <= 12); wider marginals go straight to global atomics.
+// Wide marginals: one global atomic per amplitude.
 template <typename T>
-__global__ void __launch_bounds__(kThreads) k_marginal(const C2<T>* __restrict__ s, uint64_t len, uint32_t k,
-                                                       Qubits64 qs, double* __restrict__ out) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  double* h = reinterpret_cast<double*>(smem);
-  const uint32_t bins = 1u << k;
-  const bool priv = k <= 12;
-  if (priv) {
-    for (uint32_t b = threadIdx.x; b < bins; b += blockDim.x) h[b] = 0.0;
-    __syncthreads();
-  }
+__global__ void __launch_bounds__(kThreads) k_marginal_wide(const C2<T>* __restrict__ s, uint64_t len, uint32_t k,
+                                                            Qubits64 qs, double* __restrict__ out) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < len; i += (uint64_t)gridDim.x * blockDim.x) {
     const C2<T> a = s[i];
     const double p = (double)a.x * (double)a.x + (double)a.y * (double)a.y;
     uint32_t bin = 0;
     for (uint32_t j = 0; j < k; j++) bin |= (uint32_t)((i >> qs.q[j]) & 1ull) << j;
-    if (priv) atomicAdd(&h[bin], p);
-    else atomicAdd(&out[bin], p);
-  }
-  if (priv) {
-    __syncthreads();
-    for (uint32_t b = threadIdx.x; b < bins; b += blockDim.x)
-      if (h[b] != 0.0) atomicAdd(&out[b], h[b]);
+    atomicAdd(&out[bin], p);
   }
 }
 
@@ -278,27 +360,38 @@ __global__ void __launch_bounds__(kThreads) k_block_sums(const C2<T>* __restrict
 }
 
 // Exclusive prefix of `count` sums in place, one workgroup of 1024 threads;
-// the grand total lands in total[0].
-__global__ void __launch_bounds__(1024) k_scan(double* __restrict__ v, uint64_t count, double* __restrict__ total) {
-  __shared__ double part[1024];
-  const uint32_t t = threadIdx.x, nt = blockDim.x;
+// the grand total lands in total[0] and, if host is not null, in host[0].
+// 32768 sums: 72 us with the 1024 partials added by one thread, 30 us with
+// the lane scan.
+__global__ void __launch_bounds__(1024) k_scan(double* __restrict__ v, uint64_t count, double* __restrict__ total,
+                                               double* host) {
+  __shared__ double wave_total[16];
+  const uint32_t t = threadIdx.x, nt = blockDim.x, lane = t & 63u, wave = t >> 6;
   const uint64_t per = (count + nt - 1) / nt;
   const uint64_t b = t * per, e = b + per < count ? b + per : count;
   double acc = 0.0;
+#pragma unroll 8
   for (uint64_t i = b; i < e; i++) acc += v[i];
-  part[t] = acc;
-  __syncthreads();
-  if (t == 0) {
-    double run = 0.0;
-    for (uint32_t j = 0; j < nt; j++) {
-      const double x = part[j];
-      part[j] = run;
-      run += x;
-    }
-    total[0] = run;
+  double incl = acc;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const double o = __shfl_up(incl, off, 64);
+    if ((int)lane >= off) incl += o;
   }
+  if (lane == 63) wave_total[wave] = incl;
   __syncthreads();
-  double run = part[t];
+  double run = 0.0, all = 0.0;
+  for (uint32_t w = 0; w < nt / 64; w++) {
+    if (w < wave) run += wave_total[w];
+    all += wave_total[w];
+  }
+  const double before = __shfl_up(incl, 1, 64);
+  if (lane) run += before;
+  if (t == 0) {
+    total[0] = all;
+    if (host) host[0] = all;
+  }
+#pragma unroll 8
   for (uint64_t i = b; i < e; i++) {
     const double x = v[i];
     v[i] = run;
@@ -306,16 +399,20 @@ __global__ void __launch_bounds__(1024) k_scan(double* __restrict__ v, uint64_t 
   }
 }
 
-// One wavefront per shot: binary search over block prefixes, then a
-// lane-parallel scan inside the chosen block.  Zero-probability amplitudes
-// are never returned (strict `target < cumulative`, as
-// crates/aleph-sv/src/sampling.rs:61-83 does).
+// One wavefront per shot: a 64-way search over the block prefixes, then the
+// chosen block in sub-blocks of 256 amplitudes (4 consecutive ones per lane,
+// 16 loads of a lane in flight) until the one that holds the target, then a
+// lane scan inside it.  Zero-probability amplitudes are never returned
+// (strict `target < cumulative`, as crates/aleph-sv/src/sampling.rs:61-83
+// does).  4096 shots at 27 qubits: 158 us with a binary search and 64
+// amplitudes a lane -> 50 us.
 template <typename T>
 __global__ void __launch_bounds__(kThreads) k_sample(const C2<T>* __restrict__ s, uint64_t len,
                                                      const double* __restrict__ prefix, const double* __restrict__ sums,
                                                      uint64_t nblocks, const double* __restrict__ total,
                                                      const double* __restrict__ uni, uint32_t shots,
                                                      uint64_t* __restrict__ out) {
+  constexpr uint32_t kSub = kSampleBlock / 256;
   const uint32_t lane = threadIdx.x & 63u;
   const uint64_t waves = ((uint64_t)gridDim.x * blockDim.x) >> 6;
   for (uint64_t shot = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6; shot < shots; shot += waves) {
@@ -323,46 +420,76 @@ __global__ void __launch_bounds__(kThreads) k_sample(const C2<T>* __restrict__ s
     // last block whose prefix <= target among blocks with positive mass
     uint64_t lo = 0, hi = nblocks;  // invariant: answer in [lo, hi)
     while (hi - lo > 1) {
-      const uint64_t mid = (lo + hi) >> 1;
-      if (prefix[mid] <= target) lo = mid;
-      else hi = mid;
+      const uint64_t step = (hi - lo + 63) / 64, at = lo + lane * step;
+      const uint64_t below = __ballot(at < hi && prefix[at] <= target);
+      const uint64_t count = below ? __popcll(below) : 1;
+      lo += (count - 1) * step;
+      hi = lo + step < hi ? lo + step : hi;
     }
     uint64_t blk = lo;
     while (blk > 0 && sums[blk] <= 0.0) blk--;          // never land in an empty block
     while (blk + 1 < nblocks && sums[blk] <= 0.0) blk++;
-    const double local = target - prefix[blk];
+    double local = target - prefix[blk];
     const uint64_t base = blk * kSampleBlock;
-    const uint32_t per = kSampleBlock / 64;             // amplitudes per lane
-    double mine = 0.0;
-    for (uint32_t j = 0; j < per; j++) {
-      const uint64_t i = base + (uint64_t)lane * per + j;
-      if (i < len) {
-        const C2<T> a = s[i];
-        mine += (double)a.x * (double)a.x + (double)a.y * (double)a.y;
+    // Sub-blocks in order until local falls inside one; `keep` is this lane's
+    // mass in it, or in the last one with any mass when rounding leaves none.
+    double keep = 0.0, keep_local = 1e308;
+    uint32_t sub = 0;
+    bool inside = false;
+    for (uint32_t j0 = 0; j0 < kSub && !inside; j0 += 4) {
+      double mine[4];
+#pragma unroll
+      for (uint32_t j = 0; j < 4; j++) {
+        mine[j] = 0.0;
+#pragma unroll
+        for (uint32_t r = 0; r < 4; r++) {
+          const uint64_t i = base + (j0 + j) * 256 + lane * 4 + r;
+          if (i < len) {
+            const C2<T> a = s[i];
+            mine[j] += (double)a.x * (double)a.x + (double)a.y * (double)a.y;
+          }
+        }
+      }
+#pragma unroll
+      for (uint32_t j = 0; j < 4; j++) {
+        double sum = mine[j];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+        if (!inside && sum > 0.0) {
+          keep = mine[j];
+          sub = j0 + j;
+          if (local < sum) {
+            keep_local = local;
+            inside = true;
+          } else {
+            local -= sum;
+          }
+        }
       }
     }
     // inclusive scan over lanes
-    double incl = mine;
-  #pragma unroll
+    double incl = keep;
+#pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
       const double o = __shfl_up(incl, off, 64);
       if ((int)lane >= off) incl += o;
     }
-    const double excl = incl - mine;
-    const bool hit = mine > 0.0 && local < incl && local >= excl;
+    const double excl = incl - keep;
+    const bool hit = inside && keep > 0.0 && keep_local < incl && keep_local >= excl;
     const uint64_t hits = __ballot(hit);
-    const uint64_t pos_lanes = __ballot(mine > 0.0);
+    const uint64_t pos_lanes = __ballot(keep > 0.0);
     int who;
     if (hits) who = __ffsll((long long)hits) - 1;
     else who = pos_lanes ? 63 - __clzll((long long)pos_lanes) : 0;   // rounding overflow: last positive lane
     if ((int)lane == who) {
-      const double rem = hits ? local - excl : 1e308;
+      const double rem = hits ? keep_local - excl : 1e308;
       double cum = 0.0;
-      uint64_t pick = base + (uint64_t)lane * per;
-      uint64_t last_pos = pick;
+      const uint64_t first = base + sub * 256 + lane * 4;
+      uint64_t pick = first, last_pos = first;
       bool found = false;
-      for (uint32_t j = 0; j < per; j++) {
-        const uint64_t i = base + (uint64_t)lane * per + j;
+#pragma unroll
+      for (uint32_t j = 0; j < 4; j++) {
+        const uint64_t i = first + j;
         if (i >= len) break;
         const C2<T> a = s[i];
         const double p = (double)a.x * (double)a.x + (double)a.y * (double)a.y;
@@ -447,33 +574,34 @@ inline uint32_t grid_for(uint64_t items) {
 
 }  // namespace
 
+namespace {
+uint32_t reduce_blocks(uint64_t len) {
+  const uint64_t tile = (uint64_t)kUnroll * kThreads;
+  return (uint32_t)std::min<uint64_t>((len + tile - 1) / tile, kReduceGrid);
+}
+}  // namespace
+
+void launch_reduce_rows(hipStream_t st, const double* partials, uint32_t rows, double* out) {
+  hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kThreads), 0, st, partials, rows, out);
+  ALEPH_HIP_CHECK(hipGetLastError());
+}
+
 template <typename T>
 void launch_reduce_branch(hipStream_t st, const void* state, uint32_t n, int32_t qubit, double* partials,
                           double* out) {
   const uint64_t len = 1ull << n;
   const uint64_t qmask = qubit >= 0 ? (1ull << qubit) : 0ull;
-  uint32_t blocks = grid_for((len + kUnroll - 1) / kUnroll);
-  if (blocks > kReduceBlocks) blocks = kReduceBlocks;
-  hipLaunchKernelGGL((k_reduce_branch<T, 0>), dim3(blocks), dim3(kThreads), 0, st, (const C2<T>*)state, len, qmask,
-                     partials);
-  hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kThreads), 0, st, partials, blocks, 3u, out);
-  ALEPH_HIP_CHECK(hipGetLastError());
-}
-
-void launch_reduce_rows(hipStream_t st, const double* partials, uint32_t rows, double* out) {
-  hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kThreads), 0, st, partials, rows, 3u, out);
-  ALEPH_HIP_CHECK(hipGetLastError());
+  hipLaunchKernelGGL((k_reduce_branch<T, 0>), dim3(reduce_blocks(len)), dim3(kThreads), 0, st, (const C2<T>*)state,
+                     len, qmask, partials);
+  launch_reduce_rows(st, partials, reduce_blocks(len), out);
 }
 
 template <typename T>
 void launch_sum_p2(hipStream_t st, const void* state, uint32_t n, double* partials, double* out) {
   const uint64_t len = 1ull << n;
-  uint32_t blocks = grid_for((len + kUnroll - 1) / kUnroll);
-  if (blocks > kReduceBlocks) blocks = kReduceBlocks;
-  hipLaunchKernelGGL((k_reduce_branch<T, 1>), dim3(blocks), dim3(kThreads), 0, st, (const C2<T>*)state, len, 0ull,
-                     partials);
-  hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kThreads), 0, st, partials, blocks, 3u, out);
-  ALEPH_HIP_CHECK(hipGetLastError());
+  hipLaunchKernelGGL((k_reduce_branch<T, 1>), dim3(reduce_blocks(len)), dim3(kThreads), 0, st, (const C2<T>*)state,
+                     len, 0ull, partials);
+  launch_reduce_rows(st, partials, reduce_blocks(len), out);
 }
 
 template <typename T>
@@ -506,22 +634,50 @@ void launch_collapse(hipStream_t st, void* state, uint32_t n, uint32_t qubit, in
 }
 
 template <typename T>
-void launch_marginal(hipStream_t st, const void* state, uint32_t n, uint32_t k, const uint32_t* qubits, double* out) {
+bool launch_marginal(hipStream_t st, const void* state, uint32_t n, uint32_t k, const uint32_t* qubits, double* bins,
+                     double* partials, double* host) {
   const uint64_t len = 1ull << n;
-  const uint64_t bins = 1ull << k;
-  hipLaunchKernelGGL(k_zero, dim3(grid_for(bins)), dim3(kThreads), 0, st, out, bins);
-  Qubits64 qs{};
-  for (uint32_t j = 0; j < k && j < 64; j++) qs.q[j] = qubits[j];
-  uint32_t blocks = grid_for(len);
-  if (blocks > kReduceBlocks) blocks = kReduceBlocks;
-  const size_t lds = k <= 12 ? sizeof(double) * bins : 0;
-  hipLaunchKernelGGL(k_marginal<T>, dim3(blocks), dim3(kThreads), lds, st, (const C2<T>*)state, len, k, qs, out);
-  ALEPH_HIP_CHECK(hipGetLastError());
+  hipLaunchKernelGGL(k_zero, dim3(grid_for(1ull << k)), dim3(kThreads), 0, st, bins, 1ull << k);
+  MarginalBits d{};
+  uint64_t asked = 0;
+  for (uint32_t j = 0; j < k; j++) asked |= 1ull << qubits[j];
+  const uint32_t tb = std::min<uint32_t>(8u, n);
+  if ((uint32_t)__builtin_popcountll(asked >> tb) > kMarginalHigh) {
+    Qubits64 qs{};
+    for (uint32_t j = 0; j < k && j < 64; j++) qs.q[j] = qubits[j];
+    hipLaunchKernelGGL(k_marginal_wide<T>, dim3(std::min<uint32_t>(grid_for(len), kReduceBlocks)), dim3(kThreads), 0,
+                       st, (const C2<T>*)state, len, k, qs, bins);
+    ALEPH_HIP_CHECK(hipGetLastError());
+    return false;
+  }
+  // kMarginalGroups workgroups where there are as many bits; every workgroup
+  // is a row of the reduction's partials.
+  uint32_t left = n - tb;
+  for (uint32_t q = tb; q < n && (1ull << left) > kMarginalGroups; q++)
+    if (!((asked >> q) & 1ull)) {
+      d.loop_mask |= 1ull << q;
+      left--;
+    }
+  for (uint32_t q = tb; q < n; q++)
+    if (!((d.loop_mask >> q) & 1ull)) d.group_pos[d.n_group++] = q;
+  for (uint32_t j = 0; j < k; j++) {
+    if (qubits[j] < tb) {
+      d.low_pos[d.n_low] = qubits[j];
+      d.low_bin[d.n_low++] = j;
+    } else {
+      d.high_pos[d.n_high] = qubits[j];
+      d.high_bin[d.n_high++] = j;
+    }
+  }
+  hipLaunchKernelGGL(k_marginal<T>, dim3(1u << d.n_group), dim3(kThreads), 0, st, (const C2<T>*)state, len, d, bins,
+                     partials);
+  launch_reduce_rows(st, partials, 1u << d.n_group, host);
+  return true;
 }
 
 template <typename T>
 void launch_sample(hipStream_t st, const void* state, uint32_t n, double* block_sums, double* scan_tmp,
-                   const double* uniforms, uint32_t shots, uint64_t* out) {
+                   const double* uniforms, uint32_t shots, uint64_t* out, double* host_total) {
   const uint64_t len = 1ull << n;
   const uint64_t nb = n > kSampleBlockBits ? (1ull << (n - kSampleBlockBits)) : 1ull;
   double* sums = block_sums;       // nb
@@ -529,7 +685,7 @@ void launch_sample(hipStream_t st, const void* state, uint32_t n, double* block_
   double* total = scan_tmp;
   hipLaunchKernelGGL(k_block_sums<T>, dim3((uint32_t)nb), dim3(kThreads), 0, st, (const C2<T>*)state, len, sums,
                      prefix);
-  hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, st, prefix, nb, total);
+  hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, st, prefix, nb, total, host_total);
   if (shots) {
     const uint64_t threads = (uint64_t)shots * 64;
     hipLaunchKernelGGL(k_sample<T>, dim3(grid_for(threads)), dim3(kThreads), 0, st, (const C2<T>*)state, len, prefix,
@@ -568,12 +724,13 @@ template uint32_t launch_compare<float, float>(hipStream_t, const void*, const v
   template void launch_reduce_branch<T>(hipStream_t, const void*, uint32_t, int32_t, double*, double*);         \
   template void launch_sum_p2<T>(hipStream_t, const void*, uint32_t, double*, double*);                         \
   template void launch_normalize<T>(hipStream_t, void*, uint32_t, double*, double*);                            \
-  template void launch_expect_group<T>(hipStream_t, const void*, uint32_t, uint64_t, const uint64_t*,            \
+  template void launch_expect_group<T>(hipStream_t, const void*, uint32_t, uint64_t, const uint64_t*,           \
                                        const uint8_t*, uint32_t, double*, double*);                             \
   template void launch_collapse<T>(hipStream_t, void*, uint32_t, uint32_t, int32_t, double);                    \
-  template void launch_marginal<T>(hipStream_t, const void*, uint32_t, uint32_t, const uint32_t*, double*);      \
-  template void launch_sample<T>(hipStream_t, const void*, uint32_t, double*, double*, const double*, uint32_t,   \
-                                 uint64_t*);
+  template bool launch_marginal<T>(hipStream_t, const void*, uint32_t, uint32_t, const uint32_t*, double*,      \
+                                   double*, double*);                                                           \
+  template void launch_sample<T>(hipStream_t, const void*, uint32_t, double*, double*, const double*, uint32_t, \
+                                 uint64_t*, double*);
 ALEPH_INST(double)
 ALEPH_INST(float)
 #undef ALEPH_INST

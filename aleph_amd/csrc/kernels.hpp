@@ -112,13 +112,14 @@ void launch_mlp_adam(hipStream_t s, float* params, const float* grads, float* m,
                      float b2, float eps, uint32_t t);
 
 // ---- readout (k_readout.hip) ----
-// Result layout in `out` (device, 3 doubles): [sum of |a|^2 over bit q clear,
-// sum over bit q set, non-finite count]; qubit < 0 puts everything in [0].  `partials` needs 3 * kReduceBlocks doubles.
+// Three sums of one read into out[0..3) (device or pinned): [sum of |a|^2
+// over bit q clear, sum over bit q set, non-finite count]; qubit < 0 puts
+// everything in [0].  `partials` needs 3 * kReduceBlocks doubles.
 constexpr uint32_t kReduceBlocks = 4096;
 template <typename T>
 void launch_reduce_branch(hipStream_t s, const void* state, uint32_t n, int32_t qubit, double* partials,
                           double* out);
-// out[0] = sum of |a|^4, out[1] = sum of |a|^2, out[2] = non-finite count (same partials as above).
+// [0] = sum of |a|^4, [1] = sum of |a|^2, [2] = non-finite count, as above.
 template <typename T>
 void launch_sum_p2(hipStream_t s, const void* state, uint32_t n, double* partials, double* out);
 // Column sums of `rows` rows of three partials into out[0..3) (compensated, one workgroup; out may be
@@ -144,15 +145,18 @@ void launch_expect_group(hipStream_t s, const void* state, uint32_t n, uint64_t 
 template <typename T>
 void launch_collapse(hipStream_t s, void* state, uint32_t n, uint32_t qubit, int32_t outcome, double scale);
 
-// Marginal histogram over k qubits into `out` (2^k doubles, device, zeroed by the launcher).
+// Marginal histogram over k qubits into `bins` (2^k doubles, device, zeroed by the launcher).  Returns
+// true when the norm goes to host[0] (pinned) with it; marginals over more than 12 qubits above the
+// lowest 8 are one atomic per amplitude and leave the norm to a read of its own.
 template <typename T>
-void launch_marginal(hipStream_t s, const void* state, uint32_t n, uint32_t k, const uint32_t* qubits,
-                     double* out);
+bool launch_marginal(hipStream_t s, const void* state, uint32_t n, uint32_t k, const uint32_t* qubits, double* bins,
+                     double* partials, double* host);
 // Sampler: block sums (2^(n - kSampleBlockBits) doubles, scanned in place into
-// an exclusive prefix), then one wavefront per shot descends.
+// an exclusive prefix), then one wavefront per shot descends.  The norm goes to
+// host_total (pinned).
 constexpr uint32_t kSampleBlockBits = 12;
 template <typename T>
 void launch_sample(hipStream_t s, const void* state, uint32_t n, double* block_sums, double* scan_tmp,
-                   const double* uniforms, uint32_t shots, uint64_t* out);
+                   const double* uniforms, uint32_t shots, uint64_t* out, double* host_total);
 
 }  // namespace aleph

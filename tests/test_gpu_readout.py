@@ -1,0 +1,62 @@
+"""Readout in one read of the state: marginals by split index bits and shots by sub-blocks, with the validity check
+on the same read, against plain numpy."""
+
+import numpy as np
+import pytest
+
+from aleph_amd.backend import InvalidState
+from aleph_amd.backend import HipSvBackend
+
+pytestmark = pytest.mark.gpu
+
+
+def _state(hip, n, precision, seed):
+    rng = np.random.default_rng(seed)
+    psi = rng.standard_normal(1 << n) + 1j * rng.standard_normal(1 << n)
+    psi[rng.random(1 << n) < 0.3] = 0.0
+    psi[0] = 1.0
+    st = hip.allocate(n, precision)
+    st.load(psi / np.linalg.norm(psi))
+    return st, np.abs(st.amplitudes()) ** 2
+
+
+# Fewer amplitudes than threads, one workgroup, both sides of the thread bits (8), every qubit asked for, and more
+# than 12 qubits above the thread bits (the wide kernel).
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("n,qubits", [(1, [0]), (5, [4, 0]), (8, [7, 2, 3]), (9, [8]), (12, list(range(11, -1, -1))),
+                                      (20, [0, 19, 8, 7, 13]), (20, [9, 10, 11]), (21, list(range(8, 21))),
+                                      (21, list(range(21)))])
+def test_marginal_matches_numpy(hip, n, qubits, precision):
+    st, p = _state(hip, n, precision, n)
+    i = np.arange(1 << n)
+    bins = sum(((i >> q) & 1) << j for j, q in enumerate(qubits))
+    want = np.bincount(bins, weights=p, minlength=1 << len(qubits))
+    # FP64 sums of the state's own probabilities: a few hundred roundings at most.
+    assert np.max(np.abs(hip.probabilities(st, qubits) - want)) < 1e-14
+
+
+# One block, a partial block, many blocks; 64 shots on a boundary grid and random ones.
+@pytest.mark.parametrize("n", [1, 6, 11, 12, 13, 18, 21])
+def test_shots_match_the_cumulative_distribution(hip, n):
+    st, p = _state(hip, n, 64, n)
+    u = np.concatenate([np.random.default_rng(n).random(500), [0.0, 1.0 - 2.0**-53]])
+    got = hip.sample(st, u.size, u).astype(np.int64)
+    cum = np.cumsum(p)
+    assert np.all(p[got] > 0.0)
+    # The drawn index is where the running sum passes u (to the rounding of 2^n additions).
+    slack = 1e-15 * (n + 10)
+    t = u * cum[-1]
+    assert np.all(cum[got] > t - slack) and np.all(cum[got] - p[got] <= t + slack)
+
+
+def test_invalid_state_leaves_the_generator_alone(hip):
+    a, b = HipSvBackend(seed=9), HipSvBackend(seed=9)
+    sa, sb = a.allocate(6), b.allocate(6)
+    sa.load(np.full(64, 0.2))
+    with pytest.raises(InvalidState):
+        a.sample(sa, 5)
+    with pytest.raises(InvalidState):
+        a.probabilities(sa, [0])
+    for st in (sa, sb):
+        st.load(np.full(64, 0.125))
+    assert np.array_equal(a.sample(sa, 20), b.sample(sb, 20))
