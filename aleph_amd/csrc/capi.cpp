@@ -224,10 +224,12 @@ void normalize_async(aleph_hip_ctx* c, aleph_hip_state* st) {
 
 // The verdict of validate_state (crates/aleph-sv/src/measure.rs:23-39) on a
 // norm and a count of non-finite |psi|^2.
+double norm_tolerance(const aleph_hip_state* st) {
+  return st->precision == ALEPH_HIP_F32 ? kFp32NormDrift : std::sqrt(std::ldexp(1.0, (int)st->n)) * kAmplitudeTol;
+}
+
 bool norm_ok(const aleph_hip_state* st, double total) {
-  const double tol = st->precision == ALEPH_HIP_F32 ? kFp32NormDrift
-                                                    : std::sqrt(std::ldexp(1.0, (int)st->n)) * kAmplitudeTol;
-  return std::isfinite(total) && std::fabs(total - 1.0) <= tol;
+  return std::isfinite(total) && std::fabs(total - 1.0) <= norm_tolerance(st);
 }
 
 void check_norm(const aleph_hip_state* st, double total, double non_finite) {
@@ -238,12 +240,10 @@ void check_norm(const aleph_hip_state* st, double total, double non_finite) {
 }
 
 // validate_state as a read of its own.
-void validate(aleph_hip_ctx* c, aleph_hip_state* st, double* p0, double* p1, int32_t q) {
+void validate(aleph_hip_ctx* c, aleph_hip_state* st) {
   double r[3];
-  reduce(c, st, q, r);
+  reduce(c, st, -1, r);
   check_norm(st, r[0] + r[1], r[2]);
-  if (p0) *p0 = r[0];
-  if (p1) *p1 = r[1];
 }
 
 // Pauli string from C-ABI arrays (checked).
@@ -273,7 +273,7 @@ double pauli_sum(aleph_hip_ctx* c, aleph_hip_state* st, const std::vector<PauliT
   double total = 0.0;
   const PauliPlan plan = plan_pauli_sum(terms, st->n);
   if (plan.sweeps.empty()) {
-    validate(c, st, nullptr, nullptr, -1);
+    validate(c, st);
   } else {
     void* dev = c->d_scratch + kRecOffset;
     const size_t room = (kScratchDoubles - kRecOffset) * sizeof(double);
@@ -340,36 +340,29 @@ aleph_hip_status measure_impl(aleph_hip_ctx* c, aleph_hip_state* st, uint32_t qu
     check_state(c, st);
     need(outcome != nullptr, "null outcome");
     check_qubit(st, qubit, "measure");
-    double p0, p1;
-    validate(c, st, &p0, &p1, (int32_t)qubit);
-    p0 = std::min(std::max(p0, 0.0), 1.0);
-    p1 = std::min(std::max(p1, 0.0), 1.0);
-    const bool one_deg = p1 < 1e-300, zero_deg = p0 < 1e-300;  // measure.rs:12, 77-90
-    bool out;
-    double p;
+    // The draw is made up front (the device decides) and put back when the
+    // measurement does not use it.
+    uint64_t rng[4];
+    std::copy(c->rng, c->rng + 4, rng);
+    const double u = forced_u ? *forced_u : rng_uniform(c);
+    const double tol = norm_tolerance(st);
+    if (st->precision == ALEPH_HIP_F64)
+      launch_measure<double>(c->stream, st->d, st->n, qubit, u, tol, c->d_scratch, c->h_pinned);
+    else
+      launch_measure<float>(c->stream, st->d, st->n, qubit, u, tol, c->d_scratch, c->h_pinned);
+    ALEPH_HIP_CHECK(hipStreamSynchronize(c->stream));
+    const MeasureChoice ch = measure_choice(c->h_pinned[0], c->h_pinned[1], c->h_pinned[2], u, tol);
+    if (!ch.valid || !ch.drawn) std::copy(rng, rng + 4, c->rng);
+    check_norm(st, c->h_pinned[0] + c->h_pinned[1], c->h_pinned[2]);
     if (consumed) *consumed = 0;
-    if (zero_deg && one_deg) {
+    if (!ch.apply) {
       Failure f = make_failure(ALEPH_HIP_ERR_DEGENERATE_MEASUREMENT, "measure", "degenerate branch");
       f.qubit = qubit;
-      f.value = std::max(p0, p1);
+      f.value = ch.p;
       throw f;
-    } else if (zero_deg) {
-      out = true;
-      p = p1;
-    } else if (one_deg) {
-      out = false;
-      p = p0;
-    } else {
-      const double u = forced_u ? *forced_u : rng_uniform(c);
-      if (consumed) *consumed = 1;
-      out = u < p1;
-      p = out ? p1 : p0;
     }
-    const double scale = 1.0 / std::sqrt(p);
-    if (st->precision == ALEPH_HIP_F64) launch_collapse<double>(c->stream, st->d, st->n, qubit, out, scale);
-    else launch_collapse<float>(c->stream, st->d, st->n, qubit, out, scale);
-    ALEPH_HIP_CHECK(hipStreamSynchronize(c->stream));
-    *outcome = out ? 1 : 0;
+    if (consumed) *consumed = ch.drawn ? 1 : 0;
+    *outcome = ch.outcome ? 1 : 0;
   });
 }
 
@@ -385,7 +378,7 @@ void sample_checked(aleph_hip_ctx* c, aleph_hip_state* st, double* blocks, doubl
   ALEPH_HIP_CHECK(hipStreamSynchronize(c->stream));
   if (!norm_ok(st, c->h_pinned[0])) {
     std::copy(rng, rng + 4, c->rng);
-    validate(c, st, nullptr, nullptr, -1);   // the error, with its reason
+    validate(c, st);   // the error, with its reason
   }
   ALEPH_HIP_CHECK(hipMemcpyAsync(out, dout, shots * sizeof(uint64_t), hipMemcpyDeviceToHost, c->stream));
   ALEPH_HIP_CHECK(hipStreamSynchronize(c->stream));
@@ -397,7 +390,7 @@ aleph_hip_status sample_impl(aleph_hip_ctx* c, aleph_hip_state* st, const double
     check_state(c, st);
     need(shots == 0 || out != nullptr, "null output");
     if (shots == 0) {
-      validate(c, st, nullptr, nullptr, -1);
+      validate(c, st);
       return;
     }
     uint64_t rng[4];
@@ -1090,7 +1083,7 @@ aleph_hip_status aleph_hip_state_compare(aleph_hip_ctx* c, aleph_hip_state* a, a
 aleph_hip_status aleph_hip_validate(aleph_hip_ctx* c, aleph_hip_state* st) {
   return guarded(c, [&] {
     check_state(c, st);
-    validate(c, st, nullptr, nullptr, -1);
+    validate(c, st);
   });
 }
 
@@ -1126,7 +1119,7 @@ aleph_hip_status aleph_hip_sample_with_uniforms_noalloc(aleph_hip_ctx* c, aleph_
     }
     need(c->noalloc_scratch != nullptr, "sampler scratch not set up");
     if (shots == 0) {
-      validate(c, st, nullptr, nullptr, -1);   // context scratch, allocated with the context
+      validate(c, st);   // context scratch, allocated with the context
       return;
     }
     // Every region is written before it is read (block sums, their prefix and
@@ -1153,7 +1146,7 @@ aleph_hip_status aleph_hip_expectation(aleph_hip_ctx* c, aleph_hip_state* st, do
     try {
       terms.push_back(pauli_term(st, coeff, qubits, paulis, nt));
     } catch (const Failure&) {
-      validate(c, st, nullptr, nullptr, -1);   // an invalid state is reported before a bad string
+      validate(c, st);   // an invalid state is reported before a bad string
       throw;
     }
     terms[0].coeff = 1.0;
@@ -1178,7 +1171,7 @@ aleph_hip_status aleph_hip_expectation_sum(aleph_hip_ctx* c, aleph_hip_state* st
         if (tm.coeff != 0.0) terms.push_back(tm);
       }
     } catch (const Failure&) {
-      validate(c, st, nullptr, nullptr, -1);   // an invalid state is reported before a bad string
+      validate(c, st);   // an invalid state is reported before a bad string
       throw;
     }
     *out = pauli_sum(c, st, terms);
@@ -1348,11 +1341,11 @@ aleph_hip_status aleph_hip_probabilities(aleph_hip_ctx* c, aleph_hip_state* st, 
       check_distinct(qubits, nq, st, "probabilities");
       need(nq <= 30, "at most 30 marginal qubits");
     } catch (const Failure&) {
-      validate(c, st, nullptr, nullptr, -1);
+      validate(c, st);
       throw;
     }
     if (nq == 0) {
-      validate(c, st, nullptr, nullptr, -1);
+      validate(c, st);
       out[0] = 1.0;
       return;
     }
@@ -1366,7 +1359,7 @@ aleph_hip_status aleph_hip_probabilities(aleph_hip_ctx* c, aleph_hip_state* st, 
             ? launch_marginal<double>(c->stream, st->d, st->n, nq, qubits, d, c->d_scratch, c->h_pinned)
             : launch_marginal<float>(c->stream, st->d, st->n, nq, qubits, d, c->d_scratch, c->h_pinned);
     if (checked) ALEPH_HIP_CHECK(hipStreamSynchronize(c->stream));
-    if (!checked || !norm_ok(st, c->h_pinned[0])) validate(c, st, nullptr, nullptr, -1);
+    if (!checked || !norm_ok(st, c->h_pinned[0])) validate(c, st);
     ALEPH_HIP_CHECK(hipMemcpyAsync(out, d, bins * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     ALEPH_HIP_CHECK(hipStreamSynchronize(c->stream));
   });

@@ -63,18 +63,18 @@ __device__ void block_reduce(KSum (&v)[N]) {
   }
 }
 
-// Compensated column sums of `rows` rows of three partials; valid in thread 0.
-__device__ __forceinline__ void sum_rows(const double* partials, uint32_t rows, KSum (&v)[3]) {
-  for (int w = 0; w < 3; w++) v[w] = KSum{0, 0};
+// Compensated column sums of `rows` rows of three partials into total[0..3)
+// (LDS), one wavefront per column.
+__device__ __forceinline__ void sum_rows(const double* partials, uint32_t rows, double* total) {
+  const uint32_t lane = threadIdx.x & 63u, col = threadIdx.x >> 6;
+  if (col < 3) {
+    KSum v = {0, 0};
 #pragma unroll 4
-  for (uint32_t b = threadIdx.x; b < rows; b += blockDim.x) {
-    double x[3];
-#pragma unroll
-    for (int w = 0; w < 3; w++) x[w] = partials[3 * (uint64_t)b + w];
-#pragma unroll
-    for (int w = 0; w < 3; w++) kadd(v[w], x[w]);
+    for (uint32_t b = lane; b < rows; b += 64) kadd(v, partials[3 * (uint64_t)b + col]);
+    v = wave_reduce(v);
+    if (lane == 0) total[col] = v.s + v.c;
   }
-  block_reduce<3>(v);
+  __syncthreads();
 }
 
 // A workgroup's three sums (valid in thread 0) into its row.  A second launch
@@ -134,26 +134,67 @@ __global__ void __launch_bounds__(kThreads) k_reduce_branch(const C2<T>* __restr
 // Sums `count` rows of three partials into out[0..3) (device or pinned memory).
 __global__ void __launch_bounds__(kThreads) k_reduce_final(const double* __restrict__ partials, uint32_t count,
                                                            double* out) {
-  KSum v[3];
-  sum_rows(partials, count, v);
-  if (threadIdx.x == 0)
-    for (int w = 0; w < 3; w++) out[w] = v[w].s + v[w].c;
+  __shared__ double total[3];
+  sum_rows(partials, count, total);
+  if (threadIdx.x < 3) out[threadIdx.x] = total[threadIdx.x];
 }
 
+// Zero the amplitudes with bit q != outcome and scale the others, a pair
+// {q clear, q set} at a time: the zeroed half is only written.
 template <typename T>
-__global__ void k_collapse(C2<T>* __restrict__ s, uint64_t len, uint64_t qmask, int32_t outcome, double scale) {
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < len; i += (uint64_t)gridDim.x * blockDim.x) {
-    const bool keep = ((i & qmask) != 0) == (outcome != 0);
-    C2<T> a = s[i];
-    if (keep) {
-      a.x = (T)((double)a.x * scale);
-      a.y = (T)((double)a.y * scale);
-    } else {
-      a.x = 0;
-      a.y = 0;
-    }
-    s[i] = a;
+__device__ __forceinline__ void collapse_pairs(C2<T>* s, uint64_t pairs, uint32_t q, bool outcome, double scale,
+                                               uint64_t first, uint64_t stride) {
+  for (uint64_t p = first; p < pairs; p += stride) {
+    const uint64_t i0 = insert_zero(p, q), i1 = i0 | (1ull << q);
+    const uint64_t keep = outcome ? i1 : i0, drop = outcome ? i0 : i1;
+    C2<T> a = s[keep], zero;
+    a.x = (T)((double)a.x * scale);
+    a.y = (T)((double)a.y * scale);
+    zero.x = zero.y = 0;
+    s[keep] = a;
+    s[drop] = zero;
   }
+}
+
+// A measurement without a round trip to the host: every workgroup adds the
+// rows of the preceding reduction (at most kReduceGrid, a few microseconds)
+// and comes to the same decision the host reads from host[0..3); an invalid
+// state or a degenerate branch is left alone.  The reduction's second launch,
+// the copy back, a synchronisation and the reads of the zeroed half go (19
+// qubits, two rounds of 9 parity measurements with their 56 gates: 1.24 ->
+// 0.99 ms).
+template <typename T>
+__global__ void __launch_bounds__(kThreads) k_measure(C2<T>* __restrict__ s, uint64_t pairs, uint32_t q,
+                                                      const double* __restrict__ partials, uint32_t rows, double u,
+                                                      double tol, double* host) {
+  __shared__ double total[3];
+  sum_rows(partials, rows, total);
+  if (blockIdx.x == 0 && threadIdx.x < 3) host[threadIdx.x] = total[threadIdx.x];
+  const MeasureChoice c = measure_choice(total[0], total[1], total[2], u, tol);
+  if (!c.apply) return;
+  collapse_pairs(s, pairs, q, c.outcome, c.scale, (uint64_t)blockIdx.x * blockDim.x + threadIdx.x,
+                 (uint64_t)gridDim.x * blockDim.x);
+}
+
+// The same for a state of one workgroup's size, in one launch.
+template <typename T>
+__global__ void __launch_bounds__(kThreads) k_measure_small(C2<T>* __restrict__ s, uint64_t len, uint32_t q, double u,
+                                                            double tol, double* host) {
+  __shared__ double total[3];
+  KSum v[3] = {{0, 0}, {0, 0}, {0, 0}};
+  for (uint64_t i = threadIdx.x; i < len; i += blockDim.x) {
+    const C2<T> a = s[i];
+    const double p = (double)a.x * (double)a.x + (double)a.y * (double)a.y;
+    if (!isfinite(p)) v[2].s += 1.0;
+    else if ((i >> q) & 1ull) kadd(v[1], p);
+    else kadd(v[0], p);
+  }
+  block_reduce<3>(v);
+  if (threadIdx.x == 0)
+    for (int w = 0; w < 3; w++) host[w] = total[w] = v[w].s + v[w].c;
+  __syncthreads();
+  const MeasureChoice c = measure_choice(total[0], total[1], total[2], u, tol);
+  if (c.apply) collapse_pairs(s, len / 2, q, c.outcome, c.scale, threadIdx.x, blockDim.x);
 }
 
 // All Pauli terms that share one X mask `x` in one read of the state.
@@ -576,8 +617,11 @@ inline uint32_t grid_for(uint64_t items) {
 
 namespace {
 uint32_t reduce_blocks(uint64_t len) {
-  const uint64_t tile = (uint64_t)kUnroll * kThreads;
-  return (uint32_t)std::min<uint64_t>((len + tile - 1) / tile, kReduceGrid);
+  // Four tiles a workgroup before the next one: fewer rows for the second
+  // launch to add (19 qubits: a measurement's two kernels
+  // 17.7 -> 14.5 us, with the rows added by a wavefront per column).
+  const uint64_t tiles = (uint64_t)kUnroll * kThreads * 4;
+  return (uint32_t)std::min<uint64_t>((len + tiles - 1) / tiles, kReduceGrid);
 }
 }  // namespace
 
@@ -625,11 +669,22 @@ void launch_expect_group(hipStream_t st, const void* state, uint32_t n, uint64_t
   ALEPH_HIP_CHECK(hipGetLastError());
 }
 
+// One workgroup up to 11 qubits (8 amplitudes a thread).
+constexpr uint32_t kMeasureSmallQubits = 11;
+
 template <typename T>
-void launch_collapse(hipStream_t st, void* state, uint32_t n, uint32_t qubit, int32_t outcome, double scale) {
+void launch_measure(hipStream_t st, void* state, uint32_t n, uint32_t qubit, double u, double tol, double* partials,
+                    double* host) {
   const uint64_t len = 1ull << n;
-  hipLaunchKernelGGL(k_collapse<T>, dim3(grid_for(len)), dim3(kThreads), 0, st, (C2<T>*)state, len, 1ull << qubit,
-                     outcome, scale);
+  if (n <= kMeasureSmallQubits) {
+    hipLaunchKernelGGL(k_measure_small<T>, dim3(1), dim3(kThreads), 0, st, (C2<T>*)state, len, qubit, u, tol, host);
+  } else {
+    const uint32_t rows = reduce_blocks(len);
+    hipLaunchKernelGGL((k_reduce_branch<T, 0>), dim3(rows), dim3(kThreads), 0, st, (const C2<T>*)state, len,
+                       1ull << qubit, partials);
+    hipLaunchKernelGGL(k_measure<T>, dim3(std::min<uint32_t>(grid_for(len / 2), 2 * kReduceGrid)), dim3(kThreads), 0,
+                       st, (C2<T>*)state, len / 2, qubit, (const double*)partials, rows, u, tol, host);
+  }
   ALEPH_HIP_CHECK(hipGetLastError());
 }
 
@@ -726,7 +781,7 @@ template uint32_t launch_compare<float, float>(hipStream_t, const void*, const v
   template void launch_normalize<T>(hipStream_t, void*, uint32_t, double*, double*);                            \
   template void launch_expect_group<T>(hipStream_t, const void*, uint32_t, uint64_t, const uint64_t*,           \
                                        const uint8_t*, uint32_t, double*, double*);                             \
-  template void launch_collapse<T>(hipStream_t, void*, uint32_t, uint32_t, int32_t, double);                    \
+  template void launch_measure<T>(hipStream_t, void*, uint32_t, uint32_t, double, double, double*, double*);    \
   template bool launch_marginal<T>(hipStream_t, const void*, uint32_t, uint32_t, const uint32_t*, double*,      \
                                    double*, double*);                                                           \
   template void launch_sample<T>(hipStream_t, const void*, uint32_t, double*, double*, const double*, uint32_t, \

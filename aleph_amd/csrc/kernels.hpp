@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <cstdint>
 
 #include "plan.hpp"
@@ -142,8 +143,33 @@ constexpr uint32_t kExpectGroup = 16;
 template <typename T>
 void launch_expect_group(hipStream_t s, const void* state, uint32_t n, uint64_t xmask, const uint64_t* zy,
                          const uint8_t* use_im, uint32_t count, double* partials, double* out);
+// Measurement of `qubit` with the uniform u: branch sums, the choice below and the collapse, on the
+// device; host (pinned) receives [p0, p1, non-finite count].
 template <typename T>
-void launch_collapse(hipStream_t s, void* state, uint32_t n, uint32_t qubit, int32_t outcome, double scale);
+void launch_measure(hipStream_t s, void* state, uint32_t n, uint32_t qubit, double u, double tol, double* partials,
+                    double* host);
+// What a measurement does with the branch sums (crates/aleph-sv/src/measure.rs:12, 77-90): nothing on
+// an invalid norm (deviation beyond tol or a non-finite amplitude) or when both branches are
+// degenerate; a degenerate branch forces the other and uses no draw.  Evaluated alike on both sides.
+struct MeasureChoice {
+  bool valid, apply, drawn, outcome;
+  double p, scale;       // probability of the outcome (of the larger branch when both are degenerate)
+};
+__host__ __device__ inline MeasureChoice measure_choice(double p0, double p1, double non_finite, double u, double tol) {
+  MeasureChoice c{};
+  const double total = p0 + p1, dev = total - 1.0;
+  c.valid = non_finite == 0.0 && dev <= tol && -dev <= tol;      // false on a NaN too
+  p0 = p0 < 0.0 ? 0.0 : p0 > 1.0 ? 1.0 : p0;
+  p1 = p1 < 0.0 ? 0.0 : p1 > 1.0 ? 1.0 : p1;
+  const bool zero_deg = p0 < 1e-300, one_deg = p1 < 1e-300;
+  c.drawn = !zero_deg && !one_deg;
+  c.outcome = c.drawn ? u < p1 : zero_deg;
+  c.p = c.outcome ? p1 : p0;
+  if (zero_deg && one_deg) c.p = p0 > p1 ? p0 : p1;
+  c.apply = c.valid && !(zero_deg && one_deg);
+  c.scale = c.apply ? 1.0 / sqrt(c.p) : 1.0;
+  return c;
+}
 
 // Marginal histogram over k qubits into `bins` (2^k doubles, device, zeroed by the launcher).  Returns
 // true when the norm goes to host[0] (pinned) with it; marginals over more than 12 qubits above the

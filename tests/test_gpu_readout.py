@@ -60,3 +60,41 @@ def test_invalid_state_leaves_the_generator_alone(hip):
     for st in (sa, sb):
         st.load(np.full(64, 0.125))
     assert np.array_equal(a.sample(sa, 20), b.sample(sb, 20))
+
+
+# One workgroup (up to 11 qubits), the first size of several, and every position of the measured bit relative to
+# the pairs' order; forced outcomes use no draw, a refused state is left as it was.
+@pytest.mark.parametrize("precision", [64, 32])
+@pytest.mark.parametrize("n,qubit", [(1, 0), (4, 3), (11, 0), (11, 10), (12, 0), (12, 11), (17, 8), (18, 17)])
+def test_measure_collapses_like_numpy(hip, n, qubit, precision):
+    st, p = _state(hip, n, precision, n)
+    psi = st.amplitudes()
+    one = ((np.arange(1 << n) >> qubit) & 1).astype(bool)
+    p1 = float(np.sum(p[one]))
+    # FP64: two roundings of the product; FP32: the scaled amplitude is rounded once more.
+    tol = 4e-16 if precision == 64 else 1.2e-7
+    for u, bit in ((p1 * 0.5, True), (p1 + 0.5 * (1 - p1), False)):
+        st.load(psi)
+        assert hip.measure_with_uniform(st, qubit, u) == (bit, True)
+        want = np.where(one == bit, psi, 0) / np.sqrt(p1 if bit else 1.0 - p1)
+        got = st.amplitudes()
+        assert np.max(np.abs(got - want)) <= tol * max(1.0, np.max(np.abs(want))) + 1e-14 * np.max(np.abs(want))
+        assert hip.measure_with_uniform(st, qubit, 0.3) == (bit, False)
+    bad = psi.copy()
+    bad[-1] = np.inf
+    st.load(bad)
+    with pytest.raises(InvalidState):
+        hip.measure_with_uniform(st, qubit, 0.5)
+    assert np.array_equal(st.amplitudes()[:-1], psi[:-1])
+
+
+def test_unused_and_refused_draws_stay_in_the_generator(hip):
+    a, b = HipSvBackend(seed=31), HipSvBackend(seed=31)
+    sa, sb = a.allocate(5), b.allocate(5)
+    assert a.measure(sa, 2) is False                   # forced: |0...0>
+    sa.load(np.full(32, 1.0))
+    with pytest.raises(InvalidState):
+        a.measure(sa, 2)
+    for st in (sa, sb):
+        st.load(np.full(32, 32.0**-0.5))
+    assert [a.measure(sa, q) for q in range(5)] == [b.measure(sb, q) for q in range(5)]
