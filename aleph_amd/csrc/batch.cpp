@@ -18,7 +18,8 @@ namespace aleph {
 namespace {
 
 constexpr uint32_t kBatchRegBits = 4;
-constexpr uint32_t kDefaultChunksPerItem = 16;
+constexpr uint32_t kMaxDefaultChunksPerItem = 16;
+constexpr uint64_t kRoundItems = 4096, kPersistentItems = 256;
 constexpr uint32_t kDefaultSpinLimit = 1u << 20;
 
 DenseGate make_gate(uint32_t kind, std::initializer_list<uint32_t> qs, double theta, uint32_t n) {
@@ -234,7 +235,10 @@ void Batch::plan() {
     }
     for (const DevOp& op : p.ops) {
       DevOp c = op;
-      if (c.type == OP_PHASE) c.term_off += tb;
+      if (c.type == OP_PHASE) {
+        c.term_off += tb;
+        if (c.cut) c.cut += tb;
+      }
       ops.push_back(c);
     }
     terms.insert(terms.end(), p.terms.begin(), p.terms.end());
@@ -257,7 +261,22 @@ void Batch::plan() {
   std::vector<uint32_t> order(N);
   std::iota(order.begin(), order.end(), 0u);
   std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return nq[a] > nq[b]; });
-  const uint32_t cpi = cfg.chunks_per_item ? cfg.chunks_per_item : kDefaultChunksPerItem;
+  // Chunks per item by default: up to 16, halved until the first round has
+  // enough items to spread over the device; a few small instances otherwise
+  // run their chunks one after the other in a few workgroups.  A round launch
+  // wants four items per resident workgroup; the persistent executor pays
+  // 0.17 us an item (the L2 write-back of its device-wide release) and wants
+  // one per CU.  24 FP64 instances of 10..16 qubits, p = 3: 1.25 ms with 16
+  // chunks an item, 0.20 ms with 1 (rounds 1.20 / 0.14); 160 FP32 instances of
+  // 12..20 qubits, p = 4: persistent 10.3 ms with 1, 3.8 with 4, 3.1 with 16,
+  // rounds 2.5 / 2.1 / 2.6 with 1 / 4 / 16.
+  uint64_t first_round = 0;
+  for (uint32_t i = 0; i < N; i++)
+    if (nq[i] < solo_q && inst_passes[i]) first_round += 1ull << (nq[i] - passes[pass_list[i][0]].m);
+  uint32_t auto_cpi = kMaxDefaultChunksPerItem;
+  while (auto_cpi > 1 && first_round / auto_cpi < (cfg.mode == BATCH_ROUNDS ? kRoundItems : kPersistentItems))
+    auto_cpi /= 2;
+  const uint32_t cpi = cfg.chunks_per_item ? cfg.chunks_per_item : auto_cpi;
   uint32_t rounds = 0;
   for (uint32_t i = 0; i < N; i++)
     if (nq[i] < solo_q) rounds = std::max(rounds, inst_passes[i]);
@@ -287,7 +306,7 @@ void Batch::plan() {
 
   launch.threads = std::max(256u, 1u << (m_max - kBatchRegBits));
   if (launch.threads > 512) throw make_failure(ALEPH_HIP_ERR_INVALID_ARGUMENT, "batch", "chunk too large");
-  launch.lds_bytes = (size_t)(precision == ALEPH_HIP_F64 ? 16 : 8) << m_max;
+  launch.lds_bytes = (size_t)8 << m_max;   // FP64 stages exchange real and imaginary parts in turn
   launch.nontemporal = cfg.nontemporal;
   plan_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
 }

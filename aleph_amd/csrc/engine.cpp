@@ -626,6 +626,110 @@ void add_standalone(Plan& p, const LGate& g) {
   p.steps.push_back(s);
 }
 
+// The CutPhase form of a phase op for the op loop (see plan.hpp): its place
+// in the terms array plus one, or 0 when the op has none.  Worth its table
+// from kCutMinTerms terms on; the table has to stay small, the linear
+// coefficients within three binary digits and 16 register slots.
+constexpr size_t kCutMinTerms = 8;
+
+uint32_t add_cut_phase(Plan& p, const std::vector<PhaseTerm>& reg, const std::vector<PhaseTerm>& gen,
+                       const PlannerCtx& pc, const uint64_t* rg) {
+  if (!gen.empty() || reg.size() < kCutMinTerms || pc.G != 4 || pc.n > kCutQubits) return 0;
+  auto mask_of = [&](const PhaseTerm& t) {
+    uint64_t mk = t.mask_out;
+    for (uint32_t g = 0; g < 4; g++)
+      if ((t.rmask >> g) & 1u) mk |= rg[g];
+    return mk;
+  };
+  double phi0 = 0.0, theta = 0.0;
+  for (const PhaseTerm& t : reg) {
+    if (mask_of(t) == 0) phi0 += t.angle;
+    else if (t.angle != 0.0 && (theta == 0.0 || std::fabs(t.angle) < std::fabs(theta))) theta = t.angle;
+  }
+  if (theta == 0.0) return 0;
+  // The smallest angle is itself a small multiple (3 theta and -2 theta on a
+  // 3-regular graph).
+  auto multiple = [&](double t) {
+    for (const PhaseTerm& pt : reg)
+      if (mask_of(pt) != 0 && std::fabs(pt.angle / t - std::nearbyint(pt.angle / t)) > 1e-14 * std::fabs(pt.angle / t))
+        return false;
+    return true;
+  };
+  int div = 1;
+  while (div < 5 && !multiple(theta / div)) div++;
+  if (div == 5) return 0;
+  theta /= div;
+  CutPhase c{};
+  c.n = pc.n;
+  int linear[64] = {0};
+  uint64_t adj[64] = {0};
+  bool have_pair = false, negative = false;
+  for (int pass = 0; pass < 2; pass++) {
+    // Linear coefficients are kept non-negative: the sign of theta follows
+    // the first one.
+    for (const PhaseTerm& t : reg) {
+      const uint64_t mk = mask_of(t);
+      if (mk == 0) continue;
+      const double k = std::nearbyint(t.angle / theta);   // sums of a few equal angles: whole to rounding
+      if (std::fabs(k) > 64.0) return 0;
+      if (popc(mk) == 1) {
+        if (pass == 0) negative = k < 0;
+        else linear[__builtin_ctzll(mk)] += (int)k;
+      } else if (popc(mk) == 2) {
+        if (pass == 0) continue;
+        if (have_pair && (int)k != c.pair) return 0;
+        have_pair = true;
+        c.pair = (int)k;
+        const uint32_t lo = (uint32_t)__builtin_ctzll(mk), hi = 63u - (uint32_t)__builtin_clzll(mk);
+        if ((adj[hi] >> lo) & 1ull) return 0;
+        adj[hi] |= 1ull << lo;
+        adj[lo] |= 1ull << hi;
+      } else {
+        return 0;
+      }
+    }
+    if (pass == 0 && negative) theta = -theta;
+  }
+  uint64_t regs = 0;
+  for (uint32_t g = 0; g < 4; g++) regs |= rg[g];
+  int64_t lo = 0, hi = 0;
+  for (uint32_t q = 0; q < pc.n; q++) {
+    if (linear[q] < 0 || linear[q] > 7) return 0;
+    hi += linear[q];
+    const int pairs = c.pair * popc(adj[q] & ((1ull << q) - 1ull));
+    (c.pair < 0 ? lo : hi) += pairs;
+    if ((regs >> q) & 1ull) continue;
+    for (uint32_t b = 0; b < 3; b++)
+      if ((linear[q] >> b) & 1) c.linear[b] |= 1u << q;
+    c.below[q] = (uint32_t)(adj[q] & ((1ull << q) - 1ull) & ~regs);
+  }
+  // The bounds of K are loose (every qubit set, every pair counted): an op
+  // whose table would be too large keeps its terms.
+  if (hi - lo + 1 > (int64_t)kCutTable) return 0;
+  c.k_min = (int32_t)lo;
+  c.size = (uint32_t)(hi - lo + 1);
+  for (uint32_t g = 0; g < 4; g++) {
+    const uint32_t q = (uint32_t)__builtin_ctzll(rg[g]);
+    c.reg_linear[g] = linear[q];
+    c.reg_adj[g] = (uint32_t)(adj[q] & ~regs);
+  }
+  for (uint32_t r = 0; r < 16; r++)
+    for (uint32_t g = 0; g < 4; g++)
+      for (uint32_t h = g + 1; h < 4; h++)
+        if (((r >> g) & 1u) && ((r >> h) & 1u) && (adj[__builtin_ctzll(rg[g])] & rg[h])) c.slot[r] += c.pair;
+  const uint32_t at = (uint32_t)p.terms.size();
+  p.terms.resize(at + (sizeof(CutPhase) + c.size * 2 * sizeof(double) + sizeof(PhaseTerm) - 1) / sizeof(PhaseTerm));
+  std::memcpy(&p.terms[at], &c, sizeof(c));
+  double* table = reinterpret_cast<double*>(reinterpret_cast<unsigned char*>(&p.terms[at]) + sizeof(CutPhase));
+  for (uint32_t i = 0; i < c.size; i++) {
+    // In long double: the sum is exact to far below a double's rounding.
+    const long double phi = (long double)phi0 + (long double)theta * (long double)(c.k_min + (int32_t)i);
+    table[2 * i] = (double)std::cos(phi);
+    table[2 * i + 1] = (double)std::sin(phi);
+  }
+  return at + 1;
+}
+
 // Build one fused pass from the chosen gates.
 void emit_fused_pass(Plan& p, const PlannerCtx& pc, uint64_t S, const std::vector<const LGate*>& gates) {
   // chunk qubits: sorted physical positions
@@ -776,6 +880,7 @@ void emit_fused_pass(Plan& p, const PlannerCtx& pc, uint64_t S, const std::vecto
       ph.b = (uint32_t)pend_gen.size();
       p.terms.insert(p.terms.end(), pend_reg.begin(), pend_reg.end());
       p.terms.insert(p.terms.end(), pend_gen.begin(), pend_gen.end());
+      if (!p.opts.jit) ph.cut = add_cut_phase(p, pend_reg, pend_gen, pc, sd.rg);
       p.ops.push_back(ph);
       pend_reg.clear();
       pend_gen.clear();

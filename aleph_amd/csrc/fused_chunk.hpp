@@ -1,5 +1,5 @@
-// Device-side body of the fused LDS-staged pass, shared by the one-pass
-// launcher (k_fused.hip) and the batched executors (k_batch.hip).
+// Device-side pieces of the fused LDS-staged pass for kernels generated per
+// pass (the op loop is op_loop.hpp, which shares the address helpers).
 //
 // One chunk of 2^m amplitudes (the index bits outside the pass's chunk
 // qubits fixed by the chunk number) is read from HBM once; every op of the
@@ -467,49 +467,6 @@ __device__ __forceinline__ void phase_mul(C2<T>& a, double2 f) {
   a.y = x * fi + y * fr;
 }
 
-template <typename T, int G, int B>
-__device__ __forceinline__ void dispatch_1q(C2<T> (&a)[1 << G], const DevOp* op, uint64_t tgo,
-                                            const uint64_t (&rg)[G], uint32_t b) {
-  if constexpr (B < G) {
-    if (b == (uint32_t)B) op_1q<T, G, B>(a, op, tgo, rg);
-    else dispatch_1q<T, G, B + 1>(a, op, tgo, rg, b);
-  }
-}
-
-template <typename T, int G, int A, int B>
-__device__ __forceinline__ void dispatch_2q(C2<T> (&a)[1 << G], const DevOp* op, uint64_t tgo,
-                                            const uint64_t (&rg)[G], uint32_t ab) {
-  if constexpr (A < G) {
-    if constexpr (B < A) {
-      if (ab == (uint32_t)(A * 8 + B)) op_2q<T, G, A, B>(a, op, tgo, rg);
-      else dispatch_2q<T, G, A, B + 1>(a, op, tgo, rg, ab);
-    } else {
-      dispatch_2q<T, G, A + 1, 0>(a, op, tgo, rg, ab);
-    }
-  }
-}
-
-template <typename T, int G, int FEAT>
-__device__ __forceinline__ void run_ops(C2<T> (&a)[1 << G], const DevOp* __restrict__ ops,
-                                        const PhaseTerm* __restrict__ terms, uint32_t begin, uint32_t end,
-                                        uint64_t tgo, const uint64_t (&rg)[G]) {
-  for (uint32_t o = begin; o < end; o++) {
-    const DevOp* op = ops + o;
-    const uint32_t type = op->type;
-    if (type == OP_1Q) {
-      dispatch_1q<T, G, 0>(a, op, tgo, rg, op->a);
-    } else if (type == OP_SIGN) {
-      op_sign<T, G>(a, op, tgo);
-    } else if (type == OP_DIAG) {
-      op_diag<T, G>(a, op, tgo, rg);
-    } else if (type == OP_2Q) {
-      if constexpr ((FEAT & kFeat2Q) != 0) dispatch_2q<T, G, 1, 0>(a, op, tgo, rg, op->a * 8 + op->b);
-    } else {
-      if constexpr ((FEAT & kFeatPhase) != 0) op_phase<T, G>(a, op, terms, tgo);
-    }
-  }
-}
-
 typedef double v2f64 __attribute__((ext_vector_type(2)));
 typedef float v2f32 __attribute__((ext_vector_type(2)));
 
@@ -523,84 +480,6 @@ template <bool NT, typename V>
 __device__ __forceinline__ void gstore(V* p, V v) {
   if constexpr (NT) __builtin_nontemporal_store(v, p);
   else *p = v;
-}
-
-// Process chunk `chunk` of pass `pd` on `state`.  With GUARD, threads with
-// tid >= 2^(m - G) hold no amplitudes but take part in every barrier, so a
-// workgroup sized for the largest chunk can run smaller passes; without it
-// the workgroup has exactly 2^(m - G) threads.
-template <typename T, int G, int FEAT, bool NT, bool GUARD>
-__device__ __forceinline__ void fused_chunk(C2<T>* __restrict__ state, const PassDev* __restrict__ pd,
-                                            const StageDev* __restrict__ stages, const DevOp* __restrict__ ops,
-                                            const PhaseTerm* __restrict__ terms, uint64_t chunk,
-                                            C2<T>* __restrict__ lds) {
-  constexpr int SW = sizeof(T) == 8 ? 3 : 4;
-  constexpr int N = 1 << G;
-  using V = typename std::conditional<sizeof(T) == 8, v2f64, v2f32>::type;
-  const uint32_t m = pd->m;
-  uint64_t base = chunk;
-  for (uint32_t i = 0; i < m; i++) base = insert_zero(base, pd->local_pos[i]);
-  const uint32_t tid = threadIdx.x;
-  const bool active = !GUARD || tid < (1u << (m - G));
-  const uint32_t ns = pd->n_stages;
-  C2<T> a[N];
-  for (uint32_t s = 0; s < ns; s++) {
-    const StageDev* sd = stages + pd->stage_begin + s;
-    uint64_t tgo = base;
-    uint32_t tlo = 0;
-    const uint32_t ntb = sd->n_thread_bits;
-    for (uint32_t j = 0; j < ntb; j++) {
-      if ((tid >> j) & 1u) {
-        tgo |= sd->tg[j];
-        tlo |= sd->tl[j];
-      }
-    }
-    uint64_t rg[G];
-    uint32_t rl[G];
-#pragma unroll
-    for (int g = 0; g < G; g++) {
-      rg[g] = sd->rg[g];
-      rl[g] = sd->rl[g];
-    }
-    // Thread and register bits are disjoint, so the global index is the
-    // thread's base plus a uniform register offset (sd->go), and (swz being
-    // linear over XOR) the LDS slot is swz(thread part) ^ swz(register part),
-    // the latter precomputed per stage (sd->ls): one vector op per access.
-    C2<T>* const tp = state + tgo;
-    const uint32_t ts = swz<SW>(tlo);
-    if (active) {
-      if (s == 0) {
-#pragma unroll
-        for (int r = 0; r < N; r++) {
-          const V v = gload<NT>(reinterpret_cast<const V*>(tp + sd->go[r]));
-          a[r].x = v.x;
-          a[r].y = v.y;
-        }
-      } else {
-#pragma unroll
-        for (int r = 0; r < N; r++) a[r] = lds[ts ^ sd->ls[r]];
-      }
-      run_ops<T, G, FEAT>(a, ops, terms, sd->op_begin, sd->op_end, tgo, rg);
-    }
-    if (s + 1 == ns) {
-      if (active) {
-#pragma unroll
-        for (int r = 0; r < N; r++) {
-          V v;
-          v.x = a[r].x;
-          v.y = a[r].y;
-          gstore<NT>(reinterpret_cast<V*>(tp + sd->go[r]), v);
-        }
-      }
-    } else {
-      if (s > 0) __syncthreads();
-      if (active) {
-#pragma unroll
-        for (int r = 0; r < N; r++) lds[ts ^ sd->ls[r]] = a[r];
-      }
-      __syncthreads();
-    }
-  }
 }
 
 // Stage-by-stage access to one chunk, for pass kernels generated with the

@@ -15,7 +15,7 @@
 // The reference runs such sweeps as one circuit per call
 // (crates/aleph-backend/src/lib.rs:211-248, run_with_outcomes).
 #include "common.hpp"
-#include "fused_chunk.hpp"
+#include "op_loop.hpp"
 #include "kernels.hpp"
 
 namespace aleph {
@@ -26,7 +26,7 @@ using namespace fused;
 constexpr int kBatchFeat = kFeat2Q | kFeatPhase;
 
 template <typename T, int G, int BT, bool NT>
-__global__ void __launch_bounds__(BT, 2)
+__global__ void __launch_bounds__(BT, (OpLoopWaves<T, G>::kWaves))
     k_batch_round(C2<T>* __restrict__ pool, const BatchItem* __restrict__ items,
                   const PassDev* __restrict__ passes, const StageDev* __restrict__ stages,
                   const DevOp* __restrict__ ops, const PhaseTerm* __restrict__ terms) {
@@ -36,13 +36,12 @@ __global__ void __launch_bounds__(BT, 2)
   const PassDev* pd = passes + it.pass;
   for (uint32_t c = 0; c < it.chunk_count; c++) {
     if (c) __syncthreads();
-    fused_chunk<T, G, kBatchFeat, NT, true>(st, pd, stages, ops, terms, it.chunk_begin + c,
-                                            reinterpret_cast<C2<T>*>(smem));
+    fused_chunk<T, G, kBatchFeat, NT, true>(st, pd, stages, ops, terms, it.chunk_begin + c, smem);
   }
 }
 
 template <typename T, int G, int BT, bool NT>
-__global__ void __launch_bounds__(BT, 2)
+__global__ void __launch_bounds__(BT, (OpLoopWaves<T, G>::kWaves))
     k_batch_persistent(C2<T>* __restrict__ pool, const BatchItem* __restrict__ items, uint32_t n_items,
                        const PassDev* __restrict__ passes, const StageDev* __restrict__ stages,
                        const DevOp* __restrict__ ops, const PhaseTerm* __restrict__ terms, uint32_t* done,
@@ -90,8 +89,7 @@ __global__ void __launch_bounds__(BT, 2)
       const PassDev* pd = passes + it.pass;
       for (uint32_t c = 0; c < it.chunk_count; c++) {
         if (c) __syncthreads();
-        fused_chunk<T, G, kBatchFeat, NT, true>(st, pd, stages, ops, terms, it.chunk_begin + c,
-                                                reinterpret_cast<C2<T>*>(smem));
+        fused_chunk<T, G, kBatchFeat, NT, true>(st, pd, stages, ops, terms, it.chunk_begin + c, smem);
       }
     }
     // Publish this item's stores device-wide before it is counted done (a
@@ -214,12 +212,11 @@ __global__ void __launch_bounds__(256) k_batch_cut_final(const CutDesc* __restri
   if (threadIdx.x == 0) out[i] = (s_wave[0] + s_wave[1]) + (s_wave[2] + s_wave[3]);
 }
 
-// Dynamic LDS up to the CU's 160 KiB less what the kernels declare
-// statically (the persistent executor's queue slots).
+// Dynamic LDS for the largest chunk: 2^13 scalars of 8 bytes.
 template <typename K>
 void allow_big_lds(K kernel) {
   ALEPH_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 1024));
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, 8 << kMaxLocalBits));
 }
 
 template <typename T, int G, int BT, bool NT>

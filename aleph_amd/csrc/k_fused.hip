@@ -8,7 +8,7 @@
 // instead of one per gate as in the reference's per-gate launches
 // (crates/aleph-cuda/src/sv/backend.rs:515-581).
 #include "common.hpp"
-#include "fused_chunk.hpp"
+#include "op_loop.hpp"
 #include "kernels.hpp"
 
 namespace aleph {
@@ -17,12 +17,12 @@ namespace {
 using namespace fused;
 
 template <typename T, int G, int BT, int FEAT, bool NT>
-__global__ void __launch_bounds__(BT, 2) k_fused_pass(C2<T>* __restrict__ state, const PassDev* __restrict__ pd,
+__global__ void __launch_bounds__(BT, (OpLoopWaves<T, G>::kWaves)) k_fused_pass(C2<T>* __restrict__ state, const PassDev* __restrict__ pd,
                                                       const StageDev* __restrict__ stages,
                                                       const DevOp* __restrict__ ops,
                                                       const PhaseTerm* __restrict__ terms) {
   extern __shared__ __align__(16) unsigned char smem[];
-  fused_chunk<T, G, FEAT, NT, false>(state, pd, stages, ops, terms, blockIdx.x, reinterpret_cast<C2<T>*>(smem));
+  fused_chunk<T, G, FEAT, NT, false>(state, pd, stages, ops, terms, blockIdx.x, smem);
 }
 
 }  // namespace
@@ -32,8 +32,9 @@ static void launch_bt(hipStream_t stream, void* state, uint32_t n, uint32_t m, u
                       const StageDev* stages, const DevOp* ops, const PhaseTerm* terms) {
   const uint64_t blocks = 1ull << (n - m);
   const uint32_t threads = 1u << (m - G);
-  const size_t lds = n_stages > 1 ? (sizeof(C2<T>) << m) : 0;
-  allow_full_lds(reinterpret_cast<const void*>(&k_fused_pass<T, G, BT, FEAT, NT>));
+  const size_t lds = n_stages > 1 ? (size_t)8 << m : 0;
+  // The largest chunk (2^13 scalars of 8 bytes) beside the kernel's own phase table.
+  allow_full_lds(reinterpret_cast<const void*>(&k_fused_pass<T, G, BT, FEAT, NT>), 8 << kMaxLocalBits);
   hipLaunchKernelGGL((k_fused_pass<T, G, BT, FEAT, NT>), dim3((uint32_t)blocks), dim3(threads), lds, stream,
                      reinterpret_cast<C2<T>*>(state), pd, stages, ops, terms);
   ALEPH_HIP_CHECK(hipGetLastError());

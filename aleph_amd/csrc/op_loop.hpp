@@ -1,0 +1,441 @@
+// The fused pass as an op loop: the kernel body of plans without generated
+// kernels (k_fused.hip) and of the batched executors (k_batch.hip).
+//
+// One chunk of 2^m amplitudes (the index bits outside the pass's chunk
+// qubits fixed by the chunk number) is read from HBM once, every op of the
+// pass is applied to registers (2^G amplitudes per thread), the chunk is
+// re-distributed through LDS between stages and written back once.
+//
+// Bound by vector issue and by how much latency its waves hide, so it is
+// written to stay at 128 registers (four waves per SIMD in FP64):
+//  - the loop body is a row of plain ifs on selector words the compiler knows
+//    nothing about, and the operators change the amplitudes in place (one asm
+//    block per pair or quartet): with a chain of alternatives in C++ it moved
+//    all amplitudes to new registers at every join and took 250 registers;
+//  - descriptors and matrices come through the constant address space, so
+//    they are scalar loads and the matrices SGPR operands; the next op's
+//    header is read ahead;
+//  - FP64 stages exchange real and imaginary parts in turn through 2^m
+//    doubles (32 KiB at m = 12), half of what whole amplitudes need;
+//  - a phase op forms one class factor at a time.
+// MI355X, 23-qubit FP64 ansatz (CX ladders, 10 4x4 ops a pass): 104 -> 97 us a
+// pass, one-qubit passes 76 -> 57 us, the circuit 0.90 -> 0.78 ms.
+#pragma once
+
+#include "common.hpp"
+#include "fused_chunk.hpp"
+
+namespace aleph {
+namespace fused {
+
+// Waves per SIMD the op loop is compiled for.
+template <typename T, int G>
+struct OpLoopWaves {
+  static constexpr int kWaves = G > 4 ? 2 : sizeof(T) == 8 ? 3 : 4;
+};
+
+// A uniform value the compiler knows nothing about.
+__device__ __forceinline__ uint32_t opaque(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// In-place operators.  s_nop: a matrix entry may have been written to its
+// SGPR by a vector instruction (a reloaded spill), which needs two wait
+// states before a vector read.
+#define ALEPH_PAIR_UPDATE(T, MUL, FMA, MOV)                                                                          \
+  __device__ __forceinline__ void pair_update(C2<T>& x, C2<T>& y, const T (&m)[8]) {                                 \
+    T t0, t1, t2, t3;                                                                                                \
+    asm volatile("s_nop 1\n" MUL " %[t0], %[a], %[xr]\n" MUL " %[t1], %[a], %[xi]\n" MUL " %[t2], %[e], %[xr]\n" MUL \
+                 " %[t3], %[e], %[xi]\n" FMA " %[t0], -%[b], %[xi], %[t0]\n" FMA                                     \
+                 " %[t1], %[b], %[xr], %[t1]\n" FMA " %[t2], -%[f], %[xi], %[t2]\n" FMA                              \
+                 " %[t3], %[f], %[xr], %[t3]\n" FMA " %[t0], %[c], %[yr], %[t0]\n" FMA                               \
+                 " %[t1], %[c], %[yi], %[t1]\n" FMA " %[t2], %[g], %[yr], %[t2]\n" FMA                               \
+                 " %[t3], %[g], %[yi], %[t3]\n" FMA " %[xr], -%[d], %[yi], %[t0]\n" FMA                              \
+                 " %[xi], %[d], %[yr], %[t1]\n" FMA " %[t3], %[h], %[yr], %[t3]\n" FMA                               \
+                 " %[yr], -%[h], %[yi], %[t2]\n" MOV " %[yi], %[t3]\n"                                               \
+                 : [xr] "+v"(x.x), [xi] "+v"(x.y), [yr] "+v"(y.x), [yi] "+v"(y.y), [t0] "=&v"(t0), [t1] "=&v"(t1),   \
+                   [t2] "=&v"(t2), [t3] "=&v"(t3)                                                                    \
+                 : [a] "s"(m[0]), [b] "s"(m[1]), [c] "s"(m[2]), [d] "s"(m[3]), [e] "s"(m[4]), [f] "s"(m[5]),         \
+                   [g] "s"(m[6]), [h] "s"(m[7]));                                                                    \
+  }                                                                                                                  \
+  /* Two matrix rows (m: 16 entries) times (v0, v1, v2, v3), into (p, q). */                                         \
+  __device__ __forceinline__ void two_rows(const C2<T>& v0, const C2<T>& v1, C2<T>& p, C2<T>& q, const T* m,         \
+                                           bool first) {                                                             \
+    if (first) {                                                                                                     \
+      asm volatile("s_nop 1\n" MUL " %[pr], %[a], %[xr]\n" MUL " %[pi], %[a], %[xi]\n" MUL " %[qr], %[e], %[xr]\n"   \
+                   MUL " %[qi], %[e], %[xi]\n"                                                                       \
+                   : [pr] "=&v"(p.x), [pi] "=&v"(p.y), [qr] "=&v"(q.x), [qi] "=&v"(q.y)                              \
+                   : [xr] "v"(v0.x), [xi] "v"(v0.y), [a] "s"(m[0]), [e] "s"(m[8]));                                  \
+    } else {                                                                                                         \
+      asm volatile("s_nop 1\n" FMA " %[pr], %[a], %[xr], %[pr]\n" FMA " %[pi], %[a], %[xi], %[pi]\n" FMA             \
+                   " %[qr], %[e], %[xr], %[qr]\n" FMA " %[qi], %[e], %[xi], %[qi]\n"                                 \
+                   : [pr] "+v"(p.x), [pi] "+v"(p.y), [qr] "+v"(q.x), [qi] "+v"(q.y)                                  \
+                   : [xr] "v"(v0.x), [xi] "v"(v0.y), [a] "s"(m[0]), [e] "s"(m[8]));                                  \
+    }                                                                                                                \
+    asm volatile(FMA " %[pr], -%[b], %[xi], %[pr]\n" FMA " %[pi], %[b], %[xr], %[pi]\n" FMA                          \
+                 " %[qr], -%[f], %[xi], %[qr]\n" FMA " %[qi], %[f], %[xr], %[qi]\n" FMA                              \
+                 " %[pr], %[c], %[yr], %[pr]\n" FMA " %[pi], %[c], %[yi], %[pi]\n" FMA                               \
+                 " %[qr], %[g], %[yr], %[qr]\n" FMA " %[qi], %[g], %[yi], %[qi]\n" FMA                               \
+                 " %[pr], -%[d], %[yi], %[pr]\n" FMA " %[pi], %[d], %[yr], %[pi]\n" FMA                              \
+                 " %[qr], -%[h], %[yi], %[qr]\n" FMA " %[qi], %[h], %[yr], %[qi]\n"                                  \
+                 : [pr] "+v"(p.x), [pi] "+v"(p.y), [qr] "+v"(q.x), [qi] "+v"(q.y)                                    \
+                 : [xr] "v"(v0.x), [xi] "v"(v0.y), [yr] "v"(v1.x), [yi] "v"(v1.y), [b] "s"(m[1]), [c] "s"(m[2]),     \
+                   [d] "s"(m[3]), [f] "s"(m[9]), [g] "s"(m[10]), [h] "s"(m[11]));                                    \
+  }                                                                                                                  \
+  /* a = v, in a's own registers. */                                                                                 \
+  __device__ __forceinline__ void put(C2<T>& a, const C2<T>& v) {                                                    \
+    asm volatile(MOV " %0, %2\n" MOV " %1, %3\n" : "+v"(a.x), "+v"(a.y) : "v"(v.x), "v"(v.y));                       \
+  }                                                                                                                  \
+  /* a *= (fr, fi), per-lane factor. */                                                                              \
+  __device__ __forceinline__ void rotate(C2<T>& a, T fr, T fi) {                                                     \
+    T t0, t1;                                                                                                        \
+    asm volatile(MUL " %[t0], %[fi], %[ai]\n" MUL " %[t1], %[fi], %[ar]\n" FMA " %[ar], %[fr], %[ar], -%[t0]\n" FMA  \
+                 " %[ai], %[fr], %[ai], %[t1]\n"                                                                     \
+                 : [ar] "+v"(a.x), [ai] "+v"(a.y), [t0] "=&v"(t0), [t1] "=&v"(t1)                                    \
+                 : [fr] "v"(fr), [fi] "v"(fi));                                                                      \
+  }
+ALEPH_PAIR_UPDATE(double, "v_mul_f64", "v_fma_f64", "v_mov_b64")
+ALEPH_PAIR_UPDATE(float, "v_mul_f32", "v_fma_f32", "v_mov_b32")
+#undef ALEPH_PAIR_UPDATE
+
+template <typename T, int G, int B, bool CTL>
+__device__ __forceinline__ void loop_1q(C2<T> (&a)[1 << G], const T (&m)[8], uint64_t tgo, const uint64_t (&rg)[G],
+                                        uint64_t cm) {
+#pragma unroll
+  for (int r = 0; r < (1 << G); r++) {
+    if (r & (1 << B)) continue;
+    if (CTL && ((tgo | roff<G>(rg, r)) & cm) != cm) continue;
+    pair_update(a[r], a[r | (1 << B)], m);
+  }
+}
+
+// Rows 0 and 1 (m: 16 entries) of quartet Q and up into p.
+template <typename T, int G, int A, int B, int Q = 0>
+__device__ __forceinline__ void upper_rows(C2<T> (&a)[1 << G], C2<T> (&p)[1 << (G - 1)], const T* m) {
+  if constexpr (Q < (1 << (G - 2))) {
+    constexpr int r = ins0(ins0(Q, B), A);
+    two_rows(a[r], a[r | (1 << B)], p[2 * Q], p[2 * Q + 1], m, true);
+    two_rows(a[r | (1 << A)], a[r | (1 << A) | (1 << B)], p[2 * Q], p[2 * Q + 1], m + 4, false);
+    upper_rows<T, G, A, B, Q + 1>(a, p, m);
+  }
+}
+
+// Rows 2 and 3 of quartet Q and up, and the quartet's results into place.
+template <typename T, int G, int A, int B, bool CTL, int Q = 0>
+__device__ __forceinline__ void lower_rows(C2<T> (&a)[1 << G], const C2<T> (&p)[1 << (G - 1)], const T* m,
+                                           uint64_t tgo, const uint64_t (&rg)[G], uint64_t cm) {
+  if constexpr (Q < (1 << (G - 2))) {
+    constexpr int r = ins0(ins0(Q, B), A), r1 = r | (1 << B), r2 = r | (1 << A), r3 = r1 | r2;
+    C2<T> p2, p3;
+    two_rows(a[r], a[r1], p2, p3, m, true);
+    two_rows(a[r2], a[r3], p2, p3, m + 4, false);
+    if (!CTL || ((tgo | roff<G>(rg, r)) & cm) == cm) {
+      put(a[r], p[2 * Q]);
+      put(a[r1], p[2 * Q + 1]);
+      put(a[r2], p2);
+      put(a[r3], p3);
+    }
+    lower_rows<T, G, A, B, CTL, Q + 1>(a, p, m, tgo, rg, cm);
+  }
+}
+
+// A = matrix MSB register bit, B = LSB, A > B.  The matrix is used a half at
+// a time (32 SGPRs in FP64): rows 0 and 1 of every quartet, whose results
+// wait in temporaries, then rows 2 and 3.
+template <typename T, int G, int A, int B, bool CTL>
+__device__ __forceinline__ void loop_2q(C2<T> (&a)[1 << G], const T* upper, Prog<T>* mm, uint64_t tgo,
+                                        const uint64_t (&rg)[G], uint64_t cm) {
+  C2<T> p[1 << (G - 1)];
+  upper_rows<T, G, A, B>(a, p, upper);
+  T lower[16];
+#pragma unroll
+  for (int e = 0; e < 16; e++) lower[e] = mm[16 + e];
+  lower_rows<T, G, A, B, CTL>(a, p, lower, tgo, rg, cm);
+}
+
+// Selector words: 1q op on register bit B: bit B, controlled bit 8 + B;
+// 2q op on bits A > B: bit A (A - 1) / 2 + B, controlled 16 above.
+template <typename T, int G, int B = 0>
+__device__ __forceinline__ void select_1q(C2<T> (&a)[1 << G], uint32_t sel, const T (&m)[8], uint64_t tgo,
+                                          const uint64_t (&rg)[G], uint64_t cm) {
+  if constexpr (B < G) {
+    if (sel & (1u << B)) loop_1q<T, G, B, false>(a, m, tgo, rg, cm);
+    if (sel & (256u << B)) loop_1q<T, G, B, true>(a, m, tgo, rg, cm);
+    select_1q<T, G, B + 1>(a, sel, m, tgo, rg, cm);
+  }
+}
+
+template <typename T, int G, bool CTL, int A = 1, int B = 0>
+__device__ __forceinline__ void select_2q(C2<T> (&a)[1 << G], uint32_t sel, const T* upper, Prog<T>* mm, uint64_t tgo,
+                                          const uint64_t (&rg)[G], uint64_t cm) {
+  if constexpr (A < G) {
+    if constexpr (B < A) {
+      if (sel & (1u << (A * (A - 1) / 2 + B))) loop_2q<T, G, A, B, CTL>(a, upper, mm, tgo, rg, cm);
+      select_2q<T, G, CTL, A, B + 1>(a, sel, upper, mm, tgo, rg, cm);
+    } else {
+      select_2q<T, G, CTL, A + 1, 0>(a, sel, upper, mm, tgo, rg, cm);
+    }
+  }
+}
+
+// Multiply class K's factor into the slots it selects: class 0 every slot,
+// linear classes the slots with that register bit, pair classes those with both.
+template <typename T, int G, int K = 0>
+__device__ __forceinline__ void select_class(C2<T> (&a)[1 << G], uint32_t sel, T fr, T fi) {
+  if constexpr (K < PhaseSlots<G>::kCount) {
+    if (sel & (1u << K)) {
+#pragma unroll
+      for (int r = 0; r < (1 << G); r++) {
+        bool in = K == 0;
+#pragma unroll
+        for (int g = 0; g < G; g++) {
+          if (K == PhaseSlots<G>::linear(g) && ((r >> g) & 1)) in = true;
+#pragma unroll
+          for (int h = g + 1; h < G; h++)
+            if (K == PhaseSlots<G>::pair(g, h) && ((r >> g) & 1) && ((r >> h) & 1)) in = true;
+        }
+        if (in) rotate(a[r], fr, fi);
+      }
+    }
+    select_class<T, G, K + 1>(a, sel, fr, fi);
+  }
+}
+
+// psi *= e^{i phi}: one factor per non-empty class (FP64 angle sum, one
+// sincos), then the terms on three and more register bits with their own
+// unit factors.
+template <typename T, int G>
+__device__ __forceinline__ void loop_phase(C2<T> (&a)[1 << G], Prog<DevOp>* op, Prog<PhaseTerm>* terms, uint64_t tgo) {
+  const Prog<uint32_t>* bounds = (const Prog<uint32_t>*)op->m;
+  const uint32_t t0 = op->term_off;
+#pragma nounroll
+  for (uint32_t k = 0; k < (uint32_t)PhaseSlots<G>::kCount; k++) {
+    const uint32_t b = bounds[k], e = bounds[k + 1];
+    if (b == e) continue;
+    double phi = 0.0;
+#pragma unroll 4
+    for (uint32_t t = t0 + b; t < t0 + e; t++) {
+      const uint64_t mo = terms[t].mask_out;
+      phi += ((tgo & mo) == mo) ? terms[t].angle : 0.0;
+    }
+    double s, c;
+    phase_sincos<T>(phi, &s, &c);
+    select_class<T, G>(a, opaque(1u << k), (T)c, (T)s);
+  }
+  const uint32_t g0 = t0 + op->n_terms, g1 = g0 + op->b;
+#pragma nounroll
+  for (uint32_t t = g0; t < g1; t++) {
+    const uint64_t mo = terms[t].mask_out;
+    const uint32_t rm = opaque(terms[t].rmask);
+    const bool on = (tgo & mo) == mo;
+    const T c = on ? (T)terms[t].c : (T)1, s = on ? (T)terms[t].s : (T)0;
+#pragma unroll
+    for (int r = 0; r < (1 << G); r++)
+      if (((uint32_t)r & rm) == rm) rotate(a[r], c, s);
+  }
+}
+
+// A phase op in CutPhase form: the integer K of each amplitude from parities
+// and popcounts, its factor from the op's table (copied to LDS, `table`).
+// Against one sincos per class and a pass over the terms per thread:
+// 160 FP32 QAOA instances of 12..20 qubits, p = 4, 3.73 -> 3.34 ms a run.
+template <typename T>
+__device__ __forceinline__ void loop_cut(C2<T> (&a)[16], Prog<CutPhase>* c, const double* table_src, uint64_t tgo,
+                                         C2<T>* table) {
+  const uint32_t x = (uint32_t)tgo, size = c->size;
+  __syncthreads();                         // the previous op's table has been read
+  for (uint32_t i = threadIdx.x; i < size; i += blockDim.x) {
+    table[i].x = (T)table_src[2 * i];
+    table[i].y = (T)table_src[2 * i + 1];
+  }
+  int32_t pairs = 0;
+  const uint32_t n = c->n;
+#pragma unroll 4
+  for (uint32_t u = 0; u < n; u++) pairs += (int32_t)(__popc(x & c->below[u]) & (0u - ((x >> u) & 1u)));
+  const int32_t pk = c->pair;
+  int32_t k0 = pk * pairs - c->k_min + (int32_t)(__popc(x & c->linear[0]) + 2 * __popc(x & c->linear[1]) +
+                                                4 * __popc(x & c->linear[2]));
+  int32_t lin[4];
+#pragma unroll
+  for (int g = 0; g < 4; g++) lin[g] = c->reg_linear[g] + pk * (int32_t)__popc(x & c->reg_adj[g]);
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < 16; r++) {
+    int32_t k = k0 + c->slot[r];
+#pragma unroll
+    for (int g = 0; g < 4; g++)
+      if (r & (1 << g)) k += lin[g];
+    const C2<T> f = table[k];
+    rotate(a[r], f.x, f.y);
+  }
+}
+
+template <typename T, int G>
+__device__ __forceinline__ void loop_diag(C2<T> (&a)[1 << G], Prog<DevOp>* op, uint64_t tgo, const uint64_t (&rg)[G]) {
+  const uint64_t ma = op->ma, mb = op->mb, cm = op->cmask;
+  Prog<T>* d = (Prog<T>*)op->m;
+#pragma unroll
+  for (int r = 0; r < (1 << G); r++) {
+    const uint64_t idx = tgo | roff<G>(rg, r);
+    const bool hi = (idx & ma) != 0, lo = (idx & mb) != 0, on = (idx & cm) == cm;
+    const T dr = hi ? (lo ? d[6] : d[4]) : (lo ? d[2] : d[0]);
+    const T di = hi ? (lo ? d[7] : d[5]) : (lo ? d[3] : d[1]);
+    rotate(a[r], on ? dr : (T)1, on ? di : (T)0);
+  }
+}
+
+// Process chunk `chunk` of pass `pd` on `state`.  With GUARD, threads with
+// tid >= 2^(m - G) hold no amplitudes but take part in every barrier, so a
+// workgroup sized for the largest chunk can run smaller passes; without it
+// the workgroup has exactly 2^(m - G) threads.  `lds` holds 2^m scalars of 8
+// bytes: the real, then the imaginary parts of FP64 amplitudes, whole FP32 ones.
+template <typename T, int G, int FEAT, bool NT, bool GUARD>
+__device__ __forceinline__ void fused_chunk(C2<T>* __restrict__ state, const PassDev* __restrict__ pass,
+                                            const StageDev* __restrict__ stage_list, const DevOp* __restrict__ op_list,
+                                            const PhaseTerm* __restrict__ term_list, uint64_t chunk,
+                                            unsigned char* __restrict__ lds) {
+  constexpr int SW = sizeof(T) == 8 ? 3 : 4;
+  constexpr int N = 1 << G;
+  using V = typename std::conditional<sizeof(T) == 8, v2f64, v2f32>::type;
+  Prog<PassDev>* const pd = prog(pass);
+  Prog<DevOp>* const ops = prog(op_list);
+  Prog<PhaseTerm>* const terms = prog(term_list);
+  const uint32_t m = pd->m, ns = pd->n_stages, tid = threadIdx.x;
+  Prog<StageDev>* const stages = prog(stage_list) + pd->stage_begin;
+  uint64_t base = chunk;
+  for (uint32_t i = 0; i < m; i++) base = insert_zero(base, pd->local_pos[i]);
+  const bool active = !GUARD || tid < (1u << (m - G));
+  C2<T> a[N];
+#pragma unroll
+  for (int r = 0; r < N; r++) a[r].x = a[r].y = 0;
+  uint64_t tgo = 0;
+  uint32_t slot = 0;       // byte offset of the thread's part in LDS
+  for (uint32_t s = 0; s < ns; s++) {
+    Prog<StageDev>* const sd = stages + s;
+    const uint32_t ntb = sd->n_thread_bits, from = slot;
+    uint32_t tlo = 0;
+    tgo = base;
+    for (uint32_t j = 0; j < ntb; j++) {
+      if ((tid >> j) & 1u) {
+        tgo |= sd->tg[j];
+        tlo |= sd->tl[j];
+      }
+    }
+    slot = swz<SW>(tlo) * 8u;
+    uint64_t rg[G];
+#pragma unroll
+    for (int g = 0; g < G; g++) rg[g] = sd->rg[g];
+    if (s == 0) {
+      if (active) {
+        const C2<T>* const tp = state + tgo;
+#pragma unroll
+        for (int r = 0; r < N; r++) {
+          const V v = gload<NT>(reinterpret_cast<const V*>(tp + sd->go[r]));
+          a[r].x = v.x;
+          a[r].y = v.y;
+        }
+      }
+    } else {
+      // Thread and register bits are disjoint and the swizzle is linear over
+      // XOR: an element's byte offset is the thread's XOR the slot's (lb).
+      Prog<StageDev>* const pv = sd - 1;
+      if (s > 1) __syncthreads();      // the previous exchange has been read
+      if constexpr (sizeof(T) == 8) {
+        uint32_t w = from, g = slot;
+        if (active) {
+#pragma unroll
+          for (int r = 0; r < N; r++) *reinterpret_cast<T*>(lds + (w ^ pv->lb[r])) = a[r].x;
+        }
+        __syncthreads();
+        if (active) {
+#pragma unroll
+          for (int r = 0; r < N; r++) a[r].x = *reinterpret_cast<const T*>(lds + (g ^ sd->lb[r]));
+        }
+        __syncthreads();
+        // Opaque: the addresses are formed again instead of kept.
+        asm volatile("" : "+v"(w), "+v"(g));
+        if (active) {
+#pragma unroll
+          for (int r = 0; r < N; r++) *reinterpret_cast<T*>(lds + (w ^ pv->lb[r])) = a[r].y;
+        }
+        __syncthreads();
+        if (active) {
+#pragma unroll
+          for (int r = 0; r < N; r++) a[r].y = *reinterpret_cast<const T*>(lds + (g ^ sd->lb[r]));
+        }
+      } else {
+        if (active) {
+#pragma unroll
+          for (int r = 0; r < N; r++) *reinterpret_cast<V*>(lds + (from ^ pv->lb[r])) = V{a[r].x, a[r].y};
+        }
+        __syncthreads();
+        if (active) {
+#pragma unroll
+          for (int r = 0; r < N; r++) {
+            const V v = *reinterpret_cast<const V*>(lds + (slot ^ sd->lb[r]));
+            a[r].x = v.x;
+            a[r].y = v.y;
+          }
+        }
+      }
+    }
+    const uint32_t end = sd->op_end;
+    for (uint32_t o = sd->op_begin; o < end; o++) {
+      Prog<DevOp>* const op = ops + o;
+      const uint32_t type = op->type, ra = op->a, rb = op->b;
+      const uint64_t cm = op->cmask;
+      // The first half of the matrix slots is read with the header, one
+      // memory latency for both, whatever the op is.
+      constexpr int H = (FEAT & kFeat2Q) != 0 ? 16 : 8;
+      Prog<T>* const mm = (Prog<T>*)op->m;
+      T head[H], one[8];
+#pragma unroll
+      for (int e = 0; e < H; e++) {
+        head[e] = mm[e];
+        asm volatile("" : : "s"(head[e]));
+      }
+#pragma unroll
+      for (int e = 0; e < 8; e++) one[e] = head[e];
+      const uint32_t s1 = type == OP_1Q ? (cm ? 256u : 1u) << ra : 0u;
+      select_1q<T, G>(a, opaque(s1), one, tgo, rg, cm);
+      if constexpr ((FEAT & kFeat2Q) != 0) {
+        const uint32_t s2 = opaque(type == OP_2Q ? (cm ? 65536u : 1u) << (ra * (ra - 1) / 2 + rb) : 0u);
+        select_2q<T, G, false>(a, s2, head, mm, tgo, rg, cm);
+        if (s2 >> 16) select_2q<T, G, true>(a, s2 >> 16, head, mm, tgo, rg, cm);
+      }
+      if (opaque(type) == OP_SIGN) {
+        // Sign-bit XOR with (thread condition) & (uniform slot condition).
+        const uint32_t tm = ((tgo & cm) == cm) ? ~0u : 0u;
+#pragma unroll
+        for (int r = 0; r < N; r++) {
+          const uint32_t sr = (((uint32_t)r & ra) == ra) ? 0x80000000u : 0u;
+          a[r].x = flip_sign(a[r].x, sr, tm);
+          a[r].y = flip_sign(a[r].y, sr, tm);
+        }
+      }
+      if (opaque(type) == OP_DIAG) loop_diag<T, G>(a, op, tgo, rg);
+      if constexpr ((FEAT & kFeatPhase) != 0) {
+        const uint32_t cut = type == OP_PHASE ? op->cut : 0u;
+        if (G == 4 && opaque(cut)) {
+          __shared__ C2<T> table[kCutTable];
+          const unsigned char* d = reinterpret_cast<const unsigned char*>(term_list + cut - 1);
+          loop_cut<T>(reinterpret_cast<C2<T>(&)[16]>(a), prog(reinterpret_cast<const CutPhase*>(d)),
+                      reinterpret_cast<const double*>(d + sizeof(CutPhase)), tgo, table);
+        }
+        if (opaque(type == OP_PHASE && !(G == 4 && cut) ? 1u : 0u)) loop_phase<T, G>(a, op, terms, tgo);
+      }
+    }
+  }
+  if (active) {
+    Prog<StageDev>* const sd = stages + (ns - 1);
+    C2<T>* const tp = state + tgo;
+#pragma unroll
+    for (int r = 0; r < N; r++) {
+      V v;
+      v.x = a[r].x;
+      v.y = a[r].y;
+      gstore<NT>(reinterpret_cast<V*>(tp + sd->go[r]), v);
+    }
+  }
+}
+
+}  // namespace fused
+}  // namespace aleph

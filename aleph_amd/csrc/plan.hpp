@@ -35,7 +35,7 @@ struct alignas(16) DevOp {
   uint64_t cmask;     // OP_1Q/2Q/DIAG: controls (global); OP_SIGN: thread-side mask
   uint64_t ma, mb;    // OP_DIAG target masks
   uint32_t term_off;
-  uint32_t pad;
+  uint32_t cut;       // OP_PHASE: 1 + index into the terms of a CutPhase describing the same op, 0: none
   double m[32];       // OP_1Q: 2x2, OP_2Q: 4x4, OP_DIAG: 4 entries (interleaved complex)
 };
 
@@ -59,6 +59,29 @@ struct alignas(16) PhaseTerm {
   double c, s;       // cos(angle), sin(angle): the term's unit factor
   uint64_t pad;
 };
+
+// A phase op whose terms (one or two bits each) are whole multiples of one
+// angle theta, such as a MaxCut layer: the phase of index x is
+// phi0 + theta K(x) with
+//   K(x) = sum_q linear_q x_q + pair * (number of listed pairs inside x),
+// so an amplitude needs an integer and one entry of a table of unit factors.
+// Stored in the terms array after the op's terms; the table (cos, sin of
+// phi0 + theta k for k = k_min ..) follows it.
+constexpr uint32_t kCutQubits = 26;
+constexpr uint32_t kCutTable = 256;
+struct alignas(16) CutPhase {
+  int32_t k_min;
+  uint32_t size;               // table entries
+  int32_t pair;                // coefficient of every pair
+  uint32_t n;
+  uint32_t linear[3];          // linear coefficients 0..7 of the qubits that are not register bits, by binary digit
+  int32_t reg_linear[4];       // of the register bits
+  uint32_t reg_adj[4];         // their pairs with other qubits
+  int32_t slot[16];            // K of register setting r among the register bits
+  uint32_t below[kCutQubits];  // pairs of qubit u with lower qubits (register bits aside)
+  uint32_t pad[7];
+};
+static_assert(sizeof(CutPhase) % 16 == 0, "the table follows at 16 bytes");
 
 struct alignas(16) StageDev {
   uint32_t op_begin, op_end;

@@ -359,7 +359,7 @@ enum {
 typedef struct aleph_hip_batch_opts {
   uint32_t mode;             /* ALEPH_HIP_BATCH_* */
   uint32_t local_qubits;     /* chunk qubits per pass, 5..13 (0 = 12) */
-  uint32_t chunks_per_item;  /* chunks one workgroup takes per claim (0 = 16) */
+  uint32_t chunks_per_item;  /* chunks one workgroup takes per claim (0: up to 16, fewer for small batches) */
   uint32_t groups_per_cu;    /* persistent workgroups per CU (0 = occupancy limit) */
   uint32_t max_ops_per_pass; /* planner budget (0 = default) */
   uint32_t spin_limit;       /* bound on a dependency wait, in polls (0 = default) */

@@ -1,0 +1,65 @@
+"""The compiled op loop (no generated kernels): every op family on every register bit, controlled and not, and
+phase ops with their integer form (equal multiples of one angle) and without, against the oracle."""
+
+import numpy as np
+import pytest
+
+from aleph_amd.circuit import Circuit, DiagonalPhase, Gate, PhaseTerm
+from tests.helpers import max_abs
+
+pytestmark = pytest.mark.gpu
+
+
+def _mixed(n, seed):
+    rng = np.random.default_rng(seed)
+    c = Circuit(n)
+    for q in range(n):
+        c.u3(*rng.uniform(0, 6, 3), q)
+    for _ in range(6):
+        a, b, d = (int(x) for x in rng.permutation(n)[:3])
+        c.gate(Gate.Iswap(), [a, b])
+        c.gate(Gate.Iswap(), [b, d], [a])
+        c.gate(Gate.Ry(float(rng.uniform(0, 3))), [d], [b])
+        c.ccx(a, b, d)
+        c.gate(Gate.diag(np.exp(1j * rng.uniform(0, 6, 4)) * 1.0), [a, d], [b])
+        c.cz(a, d)
+        c.cp(float(rng.uniform(0, 3)), b, d)
+        c.add(DiagonalPhase(n, [PhaseTerm((1 << a, 1 << b, 1 << d), 0.4), PhaseTerm((1 << a | 1 << d,), -0.9)]))
+        c.u3(*rng.uniform(0, 6, 3), a)
+    return c
+
+
+def _cut_layers(n, seed, weighted):
+    """MaxCut layers on a random graph with vertex fields: whole multiples of one angle, or (weighted) not."""
+    rng = np.random.default_rng(seed)
+    c = Circuit(n)
+    for q in range(n):
+        c.h(q)
+    edges = sorted({tuple(sorted(int(x) for x in rng.permutation(n)[:2])) for _ in range(2 * n)})
+    for g in (0.83, -1.9, 2.9):
+        for k, (u, v) in enumerate(edges):
+            w = 1.0 + (0.1 * k if weighted else 0.0)
+            c.cx(u, v).rz(g * w, v).cx(u, v)
+        for q in range(n):
+            c.rx(0.3 + g, q)
+    return c
+
+
+# One register stage, one chunk, and several chunks; FP32 rounds each op to 6e-8.
+@pytest.mark.parametrize("precision,tol", [(64, 1e-13), (32, 3e-6)])
+@pytest.mark.parametrize("n", [4, 7, 11, 12, 13, 15])
+def test_op_loop_matches_oracle(hip, oracle_lib, n, precision, tol):
+    for c in (_mixed(n, n), _cut_layers(n, n, False), _cut_layers(n, n, True)):
+        for kw in ({}, {"fuse_2q": False}, {"reg_bits": 5} if n >= 5 else {}):
+            st = hip.allocate(n, precision)
+            hip.run_program(st, c, **kw)
+            assert max_abs(st.amplitudes(), oracle_lib.OracleSv().run(c).amplitudes()) < tol, kw
+            st.free()
+
+
+def test_cut_form_is_taken_and_left():
+    from aleph_amd.plan_tools import HostPlan
+    phases = [o for o in HostPlan(_cut_layers(14, 3, False)).ops if o.type == 5]
+    assert phases and all(o.pad for o in phases)
+    phases = [o for o in HostPlan(_cut_layers(14, 3, True)).ops if o.type == 5]
+    assert phases and not any(o.pad for o in phases)
