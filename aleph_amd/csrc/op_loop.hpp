@@ -300,6 +300,7 @@ __device__ __forceinline__ void fused_chunk(C2<T>* __restrict__ state, const Pas
   Prog<PhaseTerm>* const terms = prog(term_list);
   const uint32_t m = pd->m, ns = pd->n_stages, tid = threadIdx.x;
   Prog<StageDev>* const stages = prog(stage_list) + pd->stage_begin;
+  const uint32_t last_op = stages[ns - 1].op_end;
   uint64_t base = chunk;
   for (uint32_t i = 0; i < m; i++) base = insert_zero(base, pd->local_pos[i]);
   const bool active = !GUARD || tid < (1u << (m - G));
@@ -380,6 +381,16 @@ __device__ __forceinline__ void fused_chunk(C2<T>* __restrict__ state, const Pas
     const uint32_t end = sd->op_end;
     for (uint32_t o = sd->op_begin; o < end; o++) {
       Prog<DevOp>* const op = ops + o;
+      // One word of each cache line of the next op (the pass's last op has
+      // none): a workgroup with a SIMD to itself otherwise waits on memory
+      // for every op's header and matrix (23-qubit ansatz 97 -> 92 us a pass, an
+      // 11-qubit one-workgroup pass 24.1 -> 21.5).
+      constexpr int kLines = (sizeof(DevOp) + 63) / 64;
+      static_assert((kLines - 1) * 64 + 4 <= (int)sizeof(DevOp), "the touched words lie inside the op");
+      Prog<uint32_t>* const ahead = (Prog<uint32_t>*)(ops + (o + 1 < last_op ? o + 1 : o));
+      uint32_t touched[kLines];
+#pragma unroll
+      for (int e = 0; e < kLines; e++) touched[e] = ahead[16 * e];
       const uint32_t type = op->type, ra = op->a, rb = op->b;
       const uint64_t cm = op->cmask;
       // The first half of the matrix slots is read with the header, one
@@ -422,6 +433,8 @@ __device__ __forceinline__ void fused_chunk(C2<T>* __restrict__ state, const Pas
         }
         if (opaque(type == OP_PHASE && !(G == 4 && cut) ? 1u : 0u)) loop_phase<T, G>(a, op, terms, tgo);
       }
+#pragma unroll
+      for (int e = 0; e < kLines; e++) asm volatile("" : : "s"(touched[e]));
     }
   }
   if (active) {
