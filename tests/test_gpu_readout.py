@@ -62,6 +62,44 @@ def test_invalid_state_leaves_the_generator_alone(hip):
     assert np.array_equal(a.sample(sa, 20), b.sample(sb, 20))
 
 
+def test_shots_of_a_state_at_the_norm_budget(hip):
+    # Norms within a few roundings of the budget's edge, where the sampler's own sum and the validity check's
+    # compensated one fall on different sides (all but the first eighth of the state adds 0.55 units in the last
+    # place of the norm an eighth, which a plain sum rounds up): what is accepted gives shots of the state and
+    # moves the generator on, what is refused leaves it alone.
+    n = 21
+    part = 1 << (n - 3)
+    psi = np.full(1 << n, np.sqrt(0.55 * 2.0**-52 / part))
+    psi[:part] = 1.0 + 0.1 * np.random.default_rng(2).standard_normal(part)
+    psi[:part] *= np.sqrt(0.75) / np.linalg.norm(psi[:part])
+    psi[5] = 0.0
+    psi[5] = np.sqrt(1.0 + 1e-10 * 2.0 ** (0.5 * n) - float(np.sum(psi.astype(np.longdouble) ** 2)))
+    unit = psi / np.linalg.norm(psi)
+
+    def fresh(v):
+        b = HipSvBackend(seed=77)
+        st = b.allocate(n, 64)
+        st.load(v)
+        return b, st
+
+    b, st = fresh(unit)
+    want = [b.sample(st, 8), b.sample(st, 8)]
+    refused = accepted = 0
+    for step in range(-14, 15):
+        v = psi.copy()
+        v[5] += step * np.spacing(psi[5])     # half a unit in the last place of the norm
+        b, st = fresh(v)
+        try:
+            got = [b.sample(st, 8), b.sample(st, 8)]
+            accepted += 1
+            assert np.array_equal(got, want)
+        except InvalidState:
+            refused += 1
+            st.load(unit)
+            assert np.array_equal(b.sample(st, 8), want[0])
+    assert refused and accepted
+
+
 # One workgroup (up to 11 qubits), the first size of several, and every position of the measured bit relative to
 # the pairs' order; forced outcomes use no draw, a refused state is left as it was.
 @pytest.mark.parametrize("precision", [64, 32])
