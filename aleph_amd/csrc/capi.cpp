@@ -287,8 +287,8 @@ double pauli_sum(aleph_hip_ctx* c, aleph_hip_state* st, const std::vector<PauliT
     const size_t room = (kScratchDoubles - kRecOffset) * sizeof(double);
     if (f64) run_pauli_sweeps<double>(c->stream, st->d, st->n, plan, terms, dev, room, partials, c->h_pinned);
     else run_pauli_sweeps<float>(c->stream, st->d, st->n, plan, terms, dev, room, partials, c->h_pinned);
-    check_norm(st, c->h_pinned[1], c->h_pinned[2]);
     total = c->h_pinned[0];
+    if (!norm_sure(st, c->h_pinned[1])) validate(c, st);
   }
   struct Launch {
     uint64_t x;
@@ -1374,7 +1374,7 @@ aleph_hip_status aleph_hip_probabilities(aleph_hip_ctx* c, aleph_hip_state* st, 
             ? launch_marginal<double>(c->stream, st->d, st->n, nq, qubits, d, c->d_scratch, c->h_pinned)
             : launch_marginal<float>(c->stream, st->d, st->n, nq, qubits, d, c->d_scratch, c->h_pinned);
     if (checked) ALEPH_HIP_CHECK(hipStreamSynchronize(c->stream));
-    if (!checked || !norm_ok(st, c->h_pinned[0])) validate(c, st);
+    if (!checked || !norm_sure(st, c->h_pinned[0])) validate(c, st);
     ALEPH_HIP_CHECK(hipMemcpyAsync(out, d, bins * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     ALEPH_HIP_CHECK(hipStreamSynchronize(c->stream));
   });

@@ -6,6 +6,7 @@ import pytest
 
 from aleph_amd.backend import InvalidState
 from aleph_amd.backend import HipSvBackend
+from aleph_amd.circuit import PauliString
 
 pytestmark = pytest.mark.gpu
 
@@ -98,6 +99,36 @@ def test_shots_of_a_state_at_the_norm_budget(hip):
             st.load(unit)
             assert np.array_equal(b.sample(st, 8), want[0])
     assert refused and accepted
+
+
+def test_readouts_accept_what_the_compensated_norm_accepts(hip):
+    # Norms around the budget's edge, in states whose plain sums round up (one amplitude in 16 holds the mass, the
+    # others 0.55 units in the last place of its probability each): marginals, energies and shots are given exactly
+    # when the compensated norm is within the budget.
+    n, budget = 22, 1e-10 * 2.0**11
+    psi = np.full(1 << n, np.sqrt(0.55 * 2.0**-70))
+    psi[((np.arange(1 << n) >> 8) & 15) == 0] = 2.0**-9
+    psi[0] = 0.0
+    psi[0] = np.sqrt(1.0 + budget - float(np.sum(psi.astype(np.longdouble) ** 2)))
+    st = hip.allocate(n, 64)
+    z, x = PauliString.new(1.0, [(0, "Z")]), PauliString.new(1.0, [(12, "X")])
+    calls = [lambda: hip.probabilities(st, [0]), lambda: hip.probabilities(st, [20, 21]),
+             lambda: hip.expectation_pauli_sum(st, [z]), lambda: hip.expectation_pauli_sum(st, [z, x]),
+             lambda: hip.sample(st, 4, [0.1, 0.4, 0.7, 0.9])]
+    seen = set()
+    scale = psi[0]
+    for step in range(-20, 21):
+        psi[0] = scale + step * 2.0**-53 / (2.0 * scale)
+        st.load(psi)
+        accept = abs(hip.norm_sqr(st) - 1.0) <= budget
+        for call in calls:
+            try:
+                call()
+                assert accept
+            except InvalidState:
+                assert not accept
+        seen.add(accept)
+    assert seen == {True, False}
 
 
 # One workgroup (up to 11 qubits), the first size of several, and every position of the measured bit relative to
