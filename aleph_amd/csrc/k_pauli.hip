@@ -40,6 +40,7 @@ namespace {
 constexpr uint32_t kRegs = 4;
 constexpr uint32_t kSlots = 1u << kRegs;
 constexpr uint32_t kChunkBits = 12;      // 64 KiB FP64, 32 KiB FP32: two and more workgroups per CU
+constexpr uint32_t kMaxSweeps = 4096;    // bounds the search for a sweep that a string fits
 constexpr uint32_t kRunBits = 4;         // chunks keep the 4 lowest qubits: runs of 16 amplitudes
 
 struct alignas(16) PauliTermDev {
@@ -67,7 +68,7 @@ struct SweepArgs {
   uint32_t m;
   uint32_t group_end[kLayouts];   // groups of layout k end here (cumulative)
   uint32_t pos[kChunkBits];   // ascending chunk qubits
-  uint32_t with_norm;
+  uint32_t first;             // the call's first sweep: carries the norm and starts the rows of partial sums
 };
 
 __device__ __forceinline__ double signed_one(uint32_t parity) {
@@ -142,7 +143,7 @@ __global__ void __launch_bounds__(256, 2) k_pauli_sweep(const C2<T>* __restrict_
       if (active) a[r] = p[o];
       else a[r].x = a[r].y = 0;
     }
-    if (d.with_norm) {
+    if (d.first) {
       double part = 0.0;
 #pragma unroll
       for (uint32_t r = 0; r < kSlots; r++) part += (double)a[r].x * (double)a[r].x + (double)a[r].y * (double)a[r].y;
@@ -234,7 +235,8 @@ __global__ void __launch_bounds__(256, 2) k_pauli_sweep(const C2<T>* __restrict_
   if (tid < 3) {
     double t = 0.0;
     for (uint32_t w = 0; w < (blockDim.x + 63u) / 64u; w++) t += red[tid][w];
-    partials[3 * (uint64_t)blockIdx.x + tid] = t;
+    double* const row = partials + 3 * (uint64_t)blockIdx.x;
+    row[tid] = d.first ? t : row[tid] + t;
   }
 }
 
@@ -260,7 +262,7 @@ PauliPlan plan_pauli_sum(const std::vector<PauliTerm>& terms, uint32_t n) {
     }
     size_t k = 0;
     while (k < plan.sweeps.size() && (uint32_t)__builtin_popcountll(plan.sweeps[k].qubits | x) > m) k++;
-    if (k == kPauliRows) {
+    if (k == kMaxSweeps) {
       plan.rest.push_back(t);
       continue;
     }
@@ -362,7 +364,7 @@ void run_pauli_sweeps(hipStream_t st, const void* state, uint32_t n, const Pauli
   for (size_t k = 0; k < plan.sweeps.size(); k++) {
     first[k] = (uint32_t)groups.size();
     sweep_records(plan.sweeps[k], terms, n, args[k], groups, recs);
-    args[k].with_norm = k == 0;
+    args[k].first = k == 0;
   }
   const size_t gb = groups.size() * sizeof(PauliGroupDev), tb = recs.size() * sizeof(PauliTermDev);
   std::vector<unsigned char> host(gb + tb);
@@ -382,18 +384,18 @@ void run_pauli_sweeps(hipStream_t st, const void* state, uint32_t n, const Pauli
   const PauliGroupDev* dg = reinterpret_cast<const PauliGroupDev*>(dev);
   const PauliTermDev* dt = reinterpret_cast<const PauliTermDev*>((const unsigned char*)dev + gb);
   allow_full_lds(reinterpret_cast<const void*>(&k_pauli_sweep<T>), 96 * 1024);
-  // All sweeps' partials are summed by one final kernel: at most
-  // kReduceBlocks of them, and at least one workgroup per sweep.
+  // Every sweep has the same number of chunks and adds its sums to the same
+  // rows of partials, so each gets a full grid however many there are: 1000
+  // random strings on two to eight of 24 qubits are 120 sweeps and take 143 ms
+  // with the rows divided between them (34 workgroups each), 13.8 ms now (89 ms as group
+  // reads); 200 strings on four of 26 qubits 29.2 -> 10.8 ms (group reads 48.3).
   uint32_t rows = 0;
-  for (size_t k0 = 0; k0 < plan.sweeps.size(); k0++) {
-    const uint64_t chunks = len >> args[k0].m;
-    const uint32_t threads = std::max<uint32_t>(64u, 1u << (args[k0].m - kRegs));
-    const uint32_t left = (uint32_t)(plan.sweeps.size() - k0);
-    const uint32_t room = (kPauliRows - rows) / left;
-    const uint32_t blocks = (uint32_t)std::min<uint64_t>(chunks, std::max<uint32_t>(1u, std::min<uint32_t>(room, 1024u)));
-    hipLaunchKernelGGL(k_pauli_sweep<T>, dim3(blocks), dim3(threads), sizeof(C2<T>) << args[k0].m, st,
-                       (const C2<T>*)state, chunks, args[k0], dg + first[k0], dt, partials + 3 * (size_t)rows);
-    rows += blocks;
+  for (size_t k = 0; k < plan.sweeps.size(); k++) {
+    const uint64_t chunks = len >> args[k].m;
+    const uint32_t threads = std::max<uint32_t>(64u, 1u << (args[k].m - kRegs));
+    rows = (uint32_t)std::min<uint64_t>(chunks, kPauliRows);
+    hipLaunchKernelGGL(k_pauli_sweep<T>, dim3(rows), dim3(threads), sizeof(C2<T>) << args[k].m, st,
+                       (const C2<T>*)state, chunks, args[k], dg + first[k], dt, partials);
   }
   ALEPH_HIP_CHECK(hipGetLastError());
   launch_reduce_rows(st, partials, rows, result);

@@ -31,8 +31,8 @@ struct PauliPlan {
 
 PauliPlan plan_pauli_sum(const std::vector<PauliTerm>& terms, uint32_t n);
 
-// Rows of three partial sums that run_pauli_sweeps may use.
-constexpr uint32_t kPauliRows = 4096;
+// Workgroups of a sweep at most, each with a row of three partial sums.
+constexpr uint32_t kPauliRows = 1024;
 
 // Runs the sweeps and waits: result = {sum of the sweeps' terms, sum |psi|^2,
 // amplitudes with a non-finite |psi|^2} (host-visible).  `dev` is scratch for

@@ -57,3 +57,21 @@ def test_pauli_sum_matches_numpy(hip, n, precision):
     st.load(psi)
     with pytest.raises(InvalidState, match="non-finite|invalid"):
         hip.expectation_pauli_sum(st, terms)
+
+
+# Random strings whose X masks spread over many sweeps (about 20 at 14 qubits, 100 at 16): their sums meet in the
+# same rows of partial sums.
+@pytest.mark.parametrize("n,count,precision", [(14, 300, 64), (16, 300, 32)])
+def test_strings_of_many_sweeps_add_up(hip, n, count, precision):
+    rng = np.random.default_rng(n)
+    psi = rng.standard_normal(1 << n) + 1j * rng.standard_normal(1 << n)
+    st = hip.allocate(n, precision)
+    st.load(psi / np.linalg.norm(psi))
+    psi = st.amplitudes()
+    terms = []
+    for _ in range(count):
+        qs = np.sort(rng.permutation(n)[:rng.integers(2, 9)])
+        terms.append(PauliString.new(float(rng.normal()), [(int(q), str(rng.choice(list("XYZ")))) for q in qs]))
+    want = sum(t.coefficient * _expect(psi, t.terms) for t in terms)
+    # As above: rounding of 1e-16 per unit weight and product.
+    assert abs(hip.expectation_pauli_sum(st, terms) - want) < 1e-13 * sum(abs(t.coefficient) for t in terms)
