@@ -244,15 +244,15 @@ __global__ void __launch_bounds__(256, 2) k_pauli_sweep(const C2<T>* __restrict_
 
 PauliPlan plan_pauli_sum(const std::vector<PauliTerm>& terms, uint32_t n) {
   PauliPlan plan;
+  std::vector<uint32_t> order(terms.size());
+  for (uint32_t t = 0; t < order.size(); t++) order[t] = t;
+  std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return terms[a].x < terms[b].x; });
   if (n < kRegs) {
-    for (uint32_t t = 0; t < terms.size(); t++) plan.rest.push_back(t);
+    plan.rest = std::move(order);
     return plan;
   }
   const uint32_t m = std::min(n, kChunkBits), L = std::min(kRunBits, m);
   const uint64_t low = (1ull << L) - 1ull;
-  std::vector<uint32_t> order(terms.size());
-  for (uint32_t t = 0; t < order.size(); t++) order[t] = t;
-  std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return terms[a].x < terms[b].x; });
   plan.sweeps.push_back(PauliSweep{low, {}});
   for (uint32_t t : order) {
     const uint64_t x = terms[t].x;

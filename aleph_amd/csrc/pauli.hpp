@@ -23,7 +23,8 @@ struct PauliSweep {
 };
 
 // sweeps[0] always exists when n >= 4 and carries the norm; `rest` lists the
-// terms that no sweep can hold (all of them when n < 4).
+// terms that no sweep can hold (all of them when n < 4), ordered by X mask so
+// that those with the same one share a read.
 struct PauliPlan {
   std::vector<PauliSweep> sweeps;
   std::vector<uint32_t> rest;
