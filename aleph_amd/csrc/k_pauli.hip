@@ -28,6 +28,7 @@
 // Partners of one-qubit masks from LDS instead of the second and third layout:
 // 483 us a sweep.
 #include <algorithm>
+#include <cmath>
 #include <vector>
 
 #include "common.hpp"
@@ -275,9 +276,9 @@ PauliPlan plan_pauli_sum(const std::vector<PauliTerm>& terms, uint32_t n) {
   return plan;
 }
 
-// Device records of one sweep.
-static void sweep_records(const PauliSweep& sw, const std::vector<PauliTerm>& terms, uint32_t n, SweepArgs& d,
-                          std::vector<PauliGroupDev>& groups, std::vector<PauliTermDev>& out) {
+// Device records of one sweep; coefficients are scaled by 2^-shift.
+static void sweep_records(const PauliSweep& sw, const std::vector<PauliTerm>& terms, uint32_t n, int shift,
+                          SweepArgs& d, std::vector<PauliGroupDev>& groups, std::vector<PauliTermDev>& out) {
   d = SweepArgs{};
   for (uint32_t q = 0; q < n; q++)
     if ((sw.qubits >> q) & 1ull) d.pos[d.m++] = q;
@@ -335,7 +336,7 @@ static void sweep_records(const PauliSweep& sw, const std::vector<PauliTerm>& te
       td.z_thread = local(t.zy) & ~regs;
       // Re(i^ny (re + i im)): +re, -im, -re, +im; each pair counted once when
       // a register bit picks its half.
-      td.c = ((t.ny & 3) == 1 || (t.ny & 3) == 2) ? -t.coeff : t.coeff;
+      td.c = std::ldexp(((t.ny & 3) == 1 || (t.ny & 3) == 2) ? -t.coeff : t.coeff, -shift);
       if (g.half) td.c *= 2.0;
       if (items[j].zr) g.flat = 0;
       out.push_back(td);
@@ -361,9 +362,15 @@ void run_pauli_sweeps(hipStream_t st, const void* state, uint32_t n, const Pauli
   std::vector<PauliGroupDev> groups;
   std::vector<PauliTermDev> recs;
   std::vector<uint32_t> first(plan.sweeps.size());
+  // The kernel adds coefficients, twice those of pairs, before it multiplies:
+  // very large ones are scaled down (exactly) so that only a sum that is
+  // itself out of range overflows.
+  double largest = 0.0;
+  for (const PauliTerm& t : terms) largest = std::max(largest, std::fabs(t.coeff));
+  const int shift = largest > std::ldexp(1.0, 960) ? 128 : 0;
   for (size_t k = 0; k < plan.sweeps.size(); k++) {
     first[k] = (uint32_t)groups.size();
-    sweep_records(plan.sweeps[k], terms, n, args[k], groups, recs);
+    sweep_records(plan.sweeps[k], terms, n, shift, args[k], groups, recs);
     args[k].first = k == 0;
   }
   const size_t gb = groups.size() * sizeof(PauliGroupDev), tb = recs.size() * sizeof(PauliTermDev);
@@ -400,6 +407,7 @@ void run_pauli_sweeps(hipStream_t st, const void* state, uint32_t n, const Pauli
   ALEPH_HIP_CHECK(hipGetLastError());
   launch_reduce_rows(st, partials, rows, result);
   ALEPH_HIP_CHECK(hipStreamSynchronize(st));   // before `host` and an own buffer go
+  result[0] = std::ldexp(result[0], shift);
 }
 
 template void run_pauli_sweeps<double>(hipStream_t, const void*, uint32_t, const PauliPlan&,

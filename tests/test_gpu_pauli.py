@@ -75,3 +75,14 @@ def test_strings_of_many_sweeps_add_up(hip, n, count, precision):
     want = sum(t.coefficient * _expect(psi, t.terms) for t in terms)
     # As above: rounding of 1e-16 per unit weight and product.
     assert abs(hip.expectation_pauli_sum(st, terms) - want) < 1e-13 * sum(abs(t.coefficient) for t in terms)
+
+
+# Coefficients near the largest double: their sum is in range where each string's value is small enough.
+@pytest.mark.parametrize("n", [6, 13])
+def test_large_coefficients_do_not_overflow(hip, n):
+    st = hip.allocate(n, 64)
+    st.load(np.full(1 << n, 2.0 ** (-0.5 * n)))             # <X> = 1, <Z> = 0 on every qubit
+    assert hip.expectation_pauli_sum(st, [PauliString.new(1.5e308, [(1, "X")])]) == pytest.approx(1.5e308, rel=1e-12)
+    terms = [PauliString.new(1e308, [(0, "X"), (2, "X")]), PauliString.new(1.2e308, [(0, "X"), (2, "X"), (3, "Z")]),
+             PauliString.new(-1.7e308, [(n - 1, "Z")]), PauliString.new(2.0, [])]
+    assert hip.expectation_pauli_sum(st, terms) == pytest.approx(1e308, rel=1e-12)
