@@ -12,6 +12,7 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <limits>
 #include <map>
 
 #include "jit.hpp"
@@ -648,10 +649,12 @@ uint32_t add_cut_phase(Plan& p, const std::vector<PhaseTerm>& reg, const std::ve
   }
   if (theta == 0.0) return 0;
   // The smallest angle is itself a small multiple (3 theta and -2 theta on a
-  // 3-regular graph).
+  // 3-regular graph).  Multiples are exact to the rounding of a sum of a few
+  // equal angles: angles that differ by more keep their own values.
+  constexpr double kSame = 4.0 * std::numeric_limits<double>::epsilon();
   auto multiple = [&](double t) {
     for (const PhaseTerm& pt : reg)
-      if (mask_of(pt) != 0 && std::fabs(pt.angle / t - std::nearbyint(pt.angle / t)) > 1e-14 * std::fabs(pt.angle / t))
+      if (mask_of(pt) != 0 && std::fabs(pt.angle / t - std::nearbyint(pt.angle / t)) > kSame * std::fabs(pt.angle / t))
         return false;
     return true;
   };

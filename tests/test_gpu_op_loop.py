@@ -30,7 +30,7 @@ def _mixed(n, seed):
 
 
 def _cut_layers(n, seed, weighted):
-    """MaxCut layers on a random graph with vertex fields: whole multiples of one angle, or (weighted) not."""
+    """MaxCut layers on a random graph: whole multiples of one angle, or not (edge k weighted 1 + weighted * k)."""
     rng = np.random.default_rng(seed)
     c = Circuit(n)
     for q in range(n):
@@ -38,7 +38,7 @@ def _cut_layers(n, seed, weighted):
     edges = sorted({tuple(sorted(int(x) for x in rng.permutation(n)[:2])) for _ in range(2 * n)})
     for g in (0.83, -1.9, 2.9):
         for k, (u, v) in enumerate(edges):
-            w = 1.0 + (0.1 * k if weighted else 0.0)
+            w = 1.0 + weighted * k
             c.cx(u, v).rz(g * w, v).cx(u, v)
         for q in range(n):
             c.rx(0.3 + g, q)
@@ -49,7 +49,7 @@ def _cut_layers(n, seed, weighted):
 @pytest.mark.parametrize("precision,tol", [(64, 1e-13), (32, 3e-6)])
 @pytest.mark.parametrize("n", [4, 7, 11, 12, 13, 15])
 def test_op_loop_matches_oracle(hip, oracle_lib, n, precision, tol):
-    for c in (_mixed(n, n), _cut_layers(n, n, False), _cut_layers(n, n, True)):
+    for c in (_mixed(n, n), _cut_layers(n, n, 0.0), _cut_layers(n, n, 0.1)):
         for kw in ({}, {"fuse_2q": False}, {"reg_bits": 5} if n >= 5 else {}):
             st = hip.allocate(n, precision)
             hip.run_program(st, c, **kw)
@@ -59,10 +59,12 @@ def test_op_loop_matches_oracle(hip, oracle_lib, n, precision, tol):
 
 def test_cut_form_is_taken_and_left():
     from aleph_amd.plan_tools import HostPlan
-    phases = [o for o in HostPlan(_cut_layers(14, 3, False)).ops if o.type == 5]
+    phases = [o for o in HostPlan(_cut_layers(14, 3, 0.0)).ops if o.type == 5]
     assert phases and all(o.pad for o in phases)
-    phases = [o for o in HostPlan(_cut_layers(14, 3, True)).ops if o.type == 5]
-    assert phases and not any(o.pad for o in phases)
+    # Weights up to some 20 units in the last place apart are different angles too.
+    for weighted in (0.1, 2e-16):
+        phases = [o for o in HostPlan(_cut_layers(14, 3, weighted)).ops if o.type == 5]
+        assert phases and not any(o.pad for o in phases)
 
 
 def test_fp32_phase_op_rounds_an_amplitude_once(hip):
