@@ -733,6 +733,21 @@ uint32_t add_cut_phase(Plan& p, const std::vector<PhaseTerm>& reg, const std::ve
   return at + 1;
 }
 
+// Cache lines of an op that the op loop reads: the header and the used part
+// of the matrix slots.
+uint32_t op_lines(const DevOp& op, uint32_t precision, uint32_t G) {
+  const uint32_t entry = precision == ALEPH_HIP_F32 ? 4 : 8;
+  uint32_t bytes = 0;
+  switch (op.type) {
+    case OP_1Q:
+    case OP_DIAG: bytes = 8 * entry; break;
+    case OP_2Q: bytes = 32 * entry; break;
+    case OP_PHASE: bytes = (2 + G + G * (G - 1) / 2) * 4; break;   // class boundaries
+    default: break;
+  }
+  return 1 + (bytes + 63) / 64;
+}
+
 // Build one fused pass from the chosen gates.
 void emit_fused_pass(Plan& p, const PlannerCtx& pc, uint64_t S, const std::vector<const LGate*>& gates) {
   // chunk qubits: sorted physical positions
@@ -881,6 +896,8 @@ void emit_fused_pass(Plan& p, const PlannerCtx& pc, uint64_t S, const std::vecto
       ph.term_off = (uint32_t)p.terms.size();
       ph.n_terms = (uint32_t)pend_reg.size();
       ph.b = (uint32_t)pend_gen.size();
+      for (uint32_t k = 0; k < n_classes; k++)
+        if (bounds[k] < bounds[k + 1]) ph.a |= 1u << k;
       p.terms.insert(p.terms.end(), pend_reg.begin(), pend_reg.end());
       p.terms.insert(p.terms.end(), pend_gen.begin(), pend_gen.end());
       if (!p.opts.jit) ph.cut = add_cut_phase(p, pend_reg, pend_gen, pc, sd.rg);
@@ -955,6 +972,12 @@ void emit_fused_pass(Plan& p, const PlannerCtx& pc, uint64_t S, const std::vecto
     }
     p.stages.push_back(sd);
   }
+  uint32_t lines = 1;
+  for (uint32_t o = (uint32_t)p.ops.size(); o-- > p.stages[pd.stage_begin].op_begin;) {
+    p.ops[o].next_lines = lines;
+    lines = op_lines(p.ops[o], p.precision, pc.G);
+  }
+  pd.first_lines = lines;
   Step s;
   s.kind = Step::FUSED;
   s.pass = (uint32_t)p.passes.size();

@@ -7,19 +7,28 @@
 // re-distributed through LDS between stages and written back once.
 //
 // Bound by vector issue and by how much latency its waves hide, so it is
-// written to stay at 128 registers (four waves per SIMD in FP64):
+// written for few registers (92 to 128 in FP64 with one kind of dense or phase
+// op, 145 with both; 60 to 115 in FP32; none spilled), and a workgroup with
+// its SIMDs to itself by the scalar loads of the ops:
 //  - the loop body is a row of plain ifs on selector words the compiler knows
-//    nothing about, and the operators change the amplitudes in place (one asm
-//    block per pair or quartet): with a chain of alternatives in C++ it moved
-//    all amplitudes to new registers at every join and took 250 registers;
+//    nothing about, behind one if per kind of op, and the operators change the
+//    amplitudes in place (one asm block per pair or quartet): with a chain of
+//    alternatives in C++ it moved all amplitudes to new registers at every
+//    join and took 250 registers;
 //  - descriptors and matrices come through the constant address space, so
-//    they are scalar loads and the matrices SGPR operands; the next op's
-//    header is read ahead;
+//    they are scalar loads and the matrices SGPR operands; every op's cache
+//    lines are read ahead, and no more lines than it uses (the misses of the
+//    scalar cache are served one after the other: all five lines of every op
+//    made small passes a quarter slower);
+//  - nothing is kept across ops but the amplitudes and the thread's index: the
+//    slots' indices alone took 32 registers;
 //  - FP64 stages exchange real and imaginary parts in turn through 2^m
 //    doubles (32 KiB at m = 12), half of what whole amplitudes need;
 //  - a phase op forms one class factor at a time.
-// MI355X, 23-qubit FP64 ansatz (CX ladders, 10 4x4 ops a pass): 104 -> 97 us a
-// pass, one-qubit passes 76 -> 57 us, the circuit 0.90 -> 0.78 ms.
+// MI355X, a pass list run 20 times, against the C++ chains: FP64 QFT of 24
+// qubits 23.7 -> 13.1 ms, CX-ladder ansatz of 22 qubits 7.2 -> 5.2 ms and of
+// 10 qubits (one workgroup) 0.75 ms both; FP32 24-qubit QFT 18.8 -> 10.0 ms,
+// brickwall of 10 qubits 0.63 -> 0.60 ms.
 #pragma once
 
 #include "common.hpp"
@@ -153,13 +162,12 @@ __device__ __forceinline__ void loop_2q(C2<T> (&a)[1 << G], const T* upper, Prog
 
 // Selector words: 1q op on register bit B: bit B, controlled bit 8 + B;
 // 2q op on bits A > B: bit A (A - 1) / 2 + B, controlled 16 above.
-template <typename T, int G, int B = 0>
+template <typename T, int G, bool CTL, int B = 0>
 __device__ __forceinline__ void select_1q(C2<T> (&a)[1 << G], uint32_t sel, const T (&m)[8], uint64_t tgo,
                                           const uint64_t (&rg)[G], uint64_t cm) {
   if constexpr (B < G) {
-    if (sel & (1u << B)) loop_1q<T, G, B, false>(a, m, tgo, rg, cm);
-    if (sel & (256u << B)) loop_1q<T, G, B, true>(a, m, tgo, rg, cm);
-    select_1q<T, G, B + 1>(a, sel, m, tgo, rg, cm);
+    if (sel & (1u << B)) loop_1q<T, G, B, CTL>(a, m, tgo, rg, cm);
+    select_1q<T, G, CTL, B + 1>(a, sel, m, tgo, rg, cm);
   }
 }
 
@@ -210,20 +218,19 @@ __device__ __forceinline__ double class_angle(Prog<PhaseTerm>* terms, uint32_t b
   return phi;
 }
 
-// psi *= e^{i phi}: one factor per non-empty class (FP64 angle sum, one
-// sincos), then the terms on three and more register bits with their own
-// unit factors.
-template <int G>
-__device__ __forceinline__ void loop_phase(C2<double> (&a)[1 << G], Prog<DevOp>* op, Prog<PhaseTerm>* terms,
-                                           uint64_t tgo) {
+// psi *= e^{i phi} on FP64 amplitudes: one factor per non-empty class (FP64
+// angle sum, one sincos as for a state of type T), then the terms on three and
+// more register bits with their own unit factors.
+template <typename T, int G>
+__device__ __forceinline__ void rotate_classes(C2<double> (&a)[1 << G], Prog<DevOp>* op, Prog<PhaseTerm>* terms,
+                                               uint64_t tgo) {
   const Prog<uint32_t>* bounds = (const Prog<uint32_t>*)op->m;
   const uint32_t t0 = op->term_off;
 #pragma nounroll
-  for (uint32_t k = 0; k < (uint32_t)PhaseSlots<G>::kCount; k++) {
-    const uint32_t b = bounds[k], e = bounds[k + 1];
-    if (b == e) continue;
+  for (uint32_t left = op->a; left; left &= left - 1) {
+    const uint32_t k = (uint32_t)__builtin_ctz(left);
     double s, c;
-    phase_sincos<double>(class_angle(terms, t0 + b, t0 + e, tgo), &s, &c);
+    phase_sincos<T>(class_angle(terms, t0 + bounds[k], t0 + bounds[k + 1], tgo), &s, &c);
     select_class<double, G>(a, opaque(1u << k), c, s);
   }
   const uint32_t g0 = t0 + op->n_terms, g1 = g0 + op->b;
@@ -239,65 +246,22 @@ __device__ __forceinline__ void loop_phase(C2<double> (&a)[1 << G], Prog<DevOp>*
   }
 }
 
-// The same for FP32 amplitudes, each rotated once, by the FP64 product of its
-// factors: a rotation per factor rounds an amplitude up to eleven times an op
+// FP32 amplitudes are rotated in FP64 and rounded once, at the end of the op:
+// a rotation in FP32 per factor rounds an amplitude up to eleven times an op,
 // and once more per term on three and more register bits (1.29e-7 RMS an op
-// with all classes filled against 1.17e-7).  The class factors come from the
-// FP32 sincos, so they are kept as floats until they are multiplied.
-template <int G>
-__device__ __forceinline__ void loop_phase(C2<float> (&a)[1 << G], Prog<DevOp>* op, Prog<PhaseTerm>* terms,
-                                           uint64_t tgo) {
-  using L = PhaseSlots<G>;
-  const Prog<uint32_t>* bounds = (const Prog<uint32_t>*)op->m;
-  const uint32_t t0 = op->term_off;
-  float fc[L::kCount], fs[L::kCount];
+// with all classes filled, against 1.17e-7 for one rotation by the product).
+// An FP64 multiply-add takes no longer than an unpacked FP32 one.
+template <typename T, int G>
+__device__ __forceinline__ void loop_phase(C2<T> (&a)[1 << G], Prog<DevOp>* op, Prog<PhaseTerm>* terms, uint64_t tgo) {
+  if constexpr (sizeof(T) == 8) {
+    rotate_classes<T, G>(a, op, terms, tgo);
+  } else {
+    C2<double> d[1 << G];
 #pragma unroll
-  for (int k = 0; k < L::kCount; k++) {
-    fc[k] = 1.f;
-    fs[k] = 0.f;
-  }
-#pragma nounroll
-  for (uint32_t k = 0; k < (uint32_t)L::kCount; k++) {
-    const uint32_t b = bounds[k], e = bounds[k + 1];
-    if (b == e) continue;
-    double s, c;
-    phase_sincos<float>(class_angle(terms, t0 + b, t0 + e, tgo), &s, &c);
-    const uint32_t at = opaque(k);
+    for (int r = 0; r < (1 << G); r++) d[r] = C2<double>{a[r].x, a[r].y};
+    rotate_classes<T, G>(d, op, terms, tgo);
 #pragma unroll
-    for (int j = 0; j < L::kCount; j++) {
-      fc[j] = at == (uint32_t)j ? (float)c : fc[j];
-      fs[j] = at == (uint32_t)j ? (float)s : fs[j];
-    }
-  }
-  const uint32_t g0 = t0 + op->n_terms, g1 = g0 + op->b;
-#pragma unroll
-  for (int r = 0; r < (1 << G); r++) {
-    // One slot's product at a time, without the factors' FP64 values kept
-    // from one to the next.
-#pragma unroll
-    for (int j = 0; j < L::kCount; j++) asm volatile("" : "+v"(fc[j]), "+v"(fs[j]));
-    double pr = fc[0], pi = fs[0];
-    auto times = [&](double c, double s) {
-      const double t = pr * c - pi * s;
-      pi = pr * s + pi * c;
-      pr = t;
-    };
-#pragma unroll
-    for (int g = 0; g < G; g++) {
-      if (!(r & (1 << g))) continue;
-      times(fc[L::linear(g)], fs[L::linear(g)]);
-#pragma unroll
-      for (int h = g + 1; h < G; h++)
-        if (r & (1 << h)) times(fc[L::pair(g, h)], fs[L::pair(g, h)]);
-    }
-#pragma nounroll
-    for (uint32_t t = g0; t < g1; t++) {
-      const uint64_t mo = terms[t].mask_out;
-      const uint32_t rm = terms[t].rmask;
-      const bool on = (tgo & mo) == mo && ((uint32_t)r & rm) == rm;
-      times(on ? terms[t].c : 1.0, on ? terms[t].s : 0.0);
-    }
-    rotate(a[r], (float)pr, (float)pi);
+    for (int r = 0; r < (1 << G); r++) a[r] = C2<float>{(float)d[r].x, (float)d[r].y};
   }
 }
 
@@ -369,6 +333,7 @@ __device__ __forceinline__ void fused_chunk(C2<T>* __restrict__ state, const Pas
   const uint32_t m = pd->m, ns = pd->n_stages, tid = threadIdx.x;
   Prog<StageDev>* const stages = prog(stage_list) + pd->stage_begin;
   const uint32_t last_op = stages[ns - 1].op_end;
+  uint32_t lines = pd->first_lines;
   uint64_t base = chunk;
   for (uint32_t i = 0; i < m; i++) base = insert_zero(base, pd->local_pos[i]);
   const bool active = !GUARD || tid < (1u << (m - G));
@@ -448,61 +413,77 @@ __device__ __forceinline__ void fused_chunk(C2<T>* __restrict__ state, const Pas
     }
     const uint32_t end = sd->op_end;
     for (uint32_t o = sd->op_begin; o < end; o++) {
-      Prog<DevOp>* const op = ops + o;
-      // One word of each cache line of the next op (the pass's last op has
-      // none): a workgroup with a SIMD to itself otherwise waits on memory
-      // for every op's header and matrix (23-qubit ansatz 97 -> 92 us a pass, an
-      // 11-qubit one-workgroup pass 24.1 -> 21.5).
-      constexpr int kLines = (sizeof(DevOp) + 63) / 64;
-      static_assert((kLines - 1) * 64 + 4 <= (int)sizeof(DevOp), "the touched words lie inside the op");
-      Prog<uint32_t>* const ahead = (Prog<uint32_t>*)(ops + (o + 1 < last_op ? o + 1 : o));
-      uint32_t touched[kLines];
+      // Opaque: the slots' indices (tgo with the register bits) are formed
+      // where a controlled or diagonal op needs them; hoisted out of the loop
+      // they took 32 vector or scalar registers and spilled others.
+      asm volatile("" : "+v"(tgo));
 #pragma unroll
-      for (int e = 0; e < kLines; e++) touched[e] = ahead[16 * e];
+      for (int g = 0; g < G; g++) asm volatile("" : "+s"(rg[g]));
+      Prog<DevOp>* const op = ops + o;
       const uint32_t type = op->type, ra = op->a, rb = op->b;
       const uint64_t cm = op->cmask;
-      // The first half of the matrix slots is read with the header, one
-      // memory latency for both, whatever the op is.
-      constexpr int H = (FEAT & kFeat2Q) != 0 ? 16 : 8;
+      // The first line of the matrix slots (FP64) or the first half of an FP32
+      // 4x4 is read with the header, one memory latency for both; an op
+      // without a matrix reads its header in that place.
+      constexpr int H = (FEAT & kFeat2Q) != 0 && sizeof(T) == 4 ? 16 : 8;
       Prog<T>* const mm = (Prog<T>*)op->m;
+      Prog<T>* const m0 = lines > 1 ? mm : (Prog<T>*)op;
       T head[H], one[8];
 #pragma unroll
-      for (int e = 0; e < H; e++) {
-        head[e] = mm[e];
-        asm volatile("" : : "s"(head[e]));
-      }
+      for (int e = 0; e < H; e++) head[e] = m0[e];
+      // Then one word of each line of the next op (the pass's last op reads
+      // its own again): a workgroup with a SIMD to itself otherwise waits on
+      // memory for every op's header and matrix.  The asm keeps these loads
+      // behind the wait for the header and the matrix.
+      lines = op->next_lines;
+      Prog<uint32_t>* ahead = (Prog<uint32_t>*)(ops + (o + 1 < last_op ? o + 1 : o));
+      asm volatile("" : "+s"(ahead) : "s"(head[0]), "s"(head[H - 1]), "s"(type), "s"(lines));
+      constexpr uint32_t kLines = sizeof(DevOp) / 64;
+      uint32_t touched[kLines];
+#pragma unroll
+      for (uint32_t e = 0; e < kLines; e++) touched[e] = ahead[16 * (e < lines ? e : 0u)];
 #pragma unroll
       for (int e = 0; e < 8; e++) one[e] = head[e];
-      const uint32_t s1 = type == OP_1Q ? (cm ? 256u : 1u) << ra : 0u;
-      select_1q<T, G>(a, opaque(s1), one, tgo, rg, cm);
+      const uint32_t s1 = opaque(type == OP_1Q ? (cm ? 256u : 1u) << ra : 0u);
+      if (s1) {
+        select_1q<T, G, false>(a, s1, one, tgo, rg, cm);
+        if (s1 >> 8) select_1q<T, G, true>(a, s1 >> 8, one, tgo, rg, cm);
+      }
       if constexpr ((FEAT & kFeat2Q) != 0) {
         const uint32_t s2 = opaque(type == OP_2Q ? (cm ? 65536u : 1u) << (ra * (ra - 1) / 2 + rb) : 0u);
-        select_2q<T, G, false>(a, s2, head, mm, tgo, rg, cm);
-        if (s2 >> 16) select_2q<T, G, true>(a, s2 >> 16, head, mm, tgo, rg, cm);
-      }
-      if (opaque(type) == OP_SIGN) {
-        // Sign-bit XOR with (thread condition) & (uniform slot condition).
-        const uint32_t tm = ((tgo & cm) == cm) ? ~0u : 0u;
+        if (s2) {
+          T upper[16];
 #pragma unroll
-        for (int r = 0; r < N; r++) {
-          const uint32_t sr = (((uint32_t)r & ra) == ra) ? 0x80000000u : 0u;
-          a[r].x = flip_sign(a[r].x, sr, tm);
-          a[r].y = flip_sign(a[r].y, sr, tm);
+          for (int e = 0; e < 16; e++) upper[e] = e < H ? head[e] : mm[e];
+          select_2q<T, G, false>(a, s2, upper, mm, tgo, rg, cm);
+          if (s2 >> 16) select_2q<T, G, true>(a, s2 >> 16, upper, mm, tgo, rg, cm);
         }
       }
-      if (opaque(type) == OP_DIAG) loop_diag<T, G>(a, op, tgo, rg);
-      if constexpr ((FEAT & kFeatPhase) != 0) {
-        const uint32_t cut = type == OP_PHASE ? op->cut : 0u;
-        if (G == 4 && opaque(cut)) {
-          __shared__ C2<T> table[kCutTable];
-          const unsigned char* d = reinterpret_cast<const unsigned char*>(term_list + cut - 1);
-          loop_cut<T>(reinterpret_cast<C2<T>(&)[16]>(a), prog(reinterpret_cast<const CutPhase*>(d)),
-                      reinterpret_cast<const double*>(d + sizeof(CutPhase)), tgo, table);
+      if (opaque(type != OP_1Q && type != OP_2Q ? 1u : 0u)) {
+        if (opaque(type) == OP_SIGN) {
+          // Sign-bit XOR with (thread condition) & (uniform slot condition).
+          const uint32_t tm = ((tgo & cm) == cm) ? ~0u : 0u;
+#pragma unroll
+          for (int r = 0; r < N; r++) {
+            const uint32_t sr = (((uint32_t)r & ra) == ra) ? 0x80000000u : 0u;
+            a[r].x = flip_sign(a[r].x, sr, tm);
+            a[r].y = flip_sign(a[r].y, sr, tm);
+          }
         }
-        if (opaque(type == OP_PHASE && !(G == 4 && cut) ? 1u : 0u)) loop_phase<G>(a, op, terms, tgo);
+        if (opaque(type) == OP_DIAG) loop_diag<T, G>(a, op, tgo, rg);
+        if constexpr ((FEAT & kFeatPhase) != 0) {
+          const uint32_t cut = type == OP_PHASE ? op->cut : 0u;
+          if (G == 4 && opaque(cut)) {
+            __shared__ C2<T> table[kCutTable];
+            const unsigned char* d = reinterpret_cast<const unsigned char*>(term_list + cut - 1);
+            loop_cut<T>(reinterpret_cast<C2<T>(&)[16]>(a), prog(reinterpret_cast<const CutPhase*>(d)),
+                        reinterpret_cast<const double*>(d + sizeof(CutPhase)), tgo, table);
+          }
+          if (opaque(type == OP_PHASE && !(G == 4 && cut) ? 1u : 0u)) loop_phase<T, G>(a, op, terms, tgo);
+        }
       }
 #pragma unroll
-      for (int e = 0; e < kLines; e++) asm volatile("" : : "s"(touched[e]));
+      for (uint32_t e = 0; e < kLines; e++) asm volatile("" : : "s"(touched[e]));
     }
   }
   if (active) {

@@ -28,16 +28,22 @@ enum OpType : uint32_t {
   OP_PHASE = 5,  // multiply by exp(i*phi): terms[term_off, +n_terms) of PhaseSlots classes, then `b` general terms
 };
 
-struct alignas(16) DevOp {
+// Header and matrix start a 64-byte cache line each: the op loop reads, and
+// reads ahead, as many lines as the op uses (op_lines).
+struct alignas(64) DevOp {
   uint32_t type;
-  uint32_t a, b;
+  uint32_t a, b;      // register bits; OP_PHASE: set of its non-empty classes, number of general terms
   uint32_t n_terms;
   uint64_t cmask;     // OP_1Q/2Q/DIAG: controls (global); OP_SIGN: thread-side mask
   uint64_t ma, mb;    // OP_DIAG target masks
   uint32_t term_off;
   uint32_t cut;       // OP_PHASE: 1 + index into the terms of a CutPhase describing the same op, 0: none
+  uint32_t next_lines;   // cache lines of the pass's next op (1 for the last one)
+  uint32_t pad[3];
   double m[32];       // OP_1Q: 2x2, OP_2Q: 4x4, OP_DIAG: 4 entries (interleaved complex)
 };
+
+static_assert(sizeof(DevOp) == 320 && __builtin_offsetof(DevOp, m) == 64, "DevOp layout");
 
 // Accumulator slots of OP_PHASE for G register bits: 0 constant, then one
 // per register bit (linear), then one per register pair (g < h).
@@ -115,7 +121,7 @@ struct alignas(16) PassDev {
   uint32_t features;             // kFeat* bits
   uint32_t local_pos[14];        // ascending physical positions of chunk qubits
   uint32_t reg_bits;             // G of this pass
-  uint32_t pad2;
+  uint32_t first_lines;          // cache lines of its first op
 };
 
 // ---- batched execution of many small plans ----

@@ -17,7 +17,7 @@ OP_NAMES = {1: "1q", 2: "2q", 3: "diag", 4: "sign", 5: "phase"}
 
 class PassDev(C.Structure):
     _fields_ = [("m", u32), ("n_stages", u32), ("stage_begin", u32), ("features", u32), ("local_pos", u32 * 14),
-                ("reg_bits", u32), ("pad2", u32)]
+                ("reg_bits", u32), ("first_lines", u32)]
 
 
 class StageDev(C.Structure):
@@ -28,7 +28,7 @@ class StageDev(C.Structure):
 
 class DevOp(C.Structure):
     _fields_ = [("type", u32), ("a", u32), ("b", u32), ("n_terms", u32), ("cmask", u64), ("ma", u64), ("mb", u64),
-                ("term_off", u32), ("pad", u32), ("m", f64 * 32)]
+                ("term_off", u32), ("cut", u32), ("next_lines", u32), ("pad", u32 * 3), ("m", f64 * 32)]
 
 
 class PhaseTerm(C.Structure):

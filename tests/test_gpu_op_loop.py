@@ -60,11 +60,11 @@ def test_op_loop_matches_oracle(hip, oracle_lib, n, precision, tol):
 def test_cut_form_is_taken_and_left():
     from aleph_amd.plan_tools import HostPlan
     phases = [o for o in HostPlan(_cut_layers(14, 3, 0.0)).ops if o.type == 5]
-    assert phases and all(o.pad for o in phases)
+    assert phases and all(o.cut for o in phases)
     # Weights up to some 20 units in the last place apart are different angles too.
     for weighted in (0.1, 2e-16):
         phases = [o for o in HostPlan(_cut_layers(14, 3, weighted)).ops if o.type == 5]
-        assert phases and not any(o.pad for o in phases)
+        assert phases and not any(o.cut for o in phases)
 
 
 def test_fp32_phase_op_rounds_an_amplitude_once(hip):

@@ -9,7 +9,7 @@ import pytest
 
 from aleph_amd import workloads as W
 from aleph_amd.circuit import Circuit, DiagonalPhase, Gate, PhaseTerm
-from aleph_amd.plan_tools import HostPlan
+from aleph_amd.plan_tools import OP_NAMES, HostPlan
 from tests.helpers import max_abs
 from tests.plan_emulator import emulate
 from tests.test_oracle import random_circuit
@@ -307,3 +307,23 @@ def test_cancel_inverse_pairs_random_mirrors(oracle_lib):
     assert hp.stats["cancelled_gates"] == 2 * len(seq)
     psi = W.gaussian_state(n, 9)
     assert max_abs(emulate(hp, psi), oracle_state(oracle_lib, c, psi)) < 1e-12
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+def test_ops_name_the_cache_lines_of_the_next_op(precision):
+    # A header line and the used part of the matrix slots: the op loop reads that much ahead, and a matrix only
+    # where the count says that there is one.
+    c = W.brickwall(14, 6, seed=3)
+    for g in W.qft(14).instructions + W.hea(14, 2, seed=4).instructions:
+        c.add(g)
+    p = HostPlan(c, precision=precision)
+    entry = 8 if precision == 64 else 4
+    size = {"1q": 8 * entry, "2q": 32 * entry, "diag": 8 * entry, "sign": 0, "phase": 12 * 4}
+    kinds = set()
+    for q in p.passes:
+        stages = p.stages[q.stage_begin:q.stage_begin + q.n_stages]
+        ops = p.ops[stages[0].op_begin:stages[-1].op_end]
+        lines = [1 + -(-size[OP_NAMES[o.type]] // 64) for o in ops]
+        assert [q.first_lines] + [o.next_lines for o in ops] == lines + [1]
+        kinds |= {OP_NAMES[o.type] for o in ops}
+    assert kinds >= {"1q", "2q", "sign", "phase"}
