@@ -48,7 +48,15 @@ __device__ __forceinline__ uint32_t opaque(uint32_t v) { return __builtin_amdgcn
 
 // In-place operators.  s_nop: a matrix entry may have been written to its
 // SGPR by a vector instruction (a reloaded spill), which needs two wait
-// states before a vector read.
+// states before a vector read; every block with matrix operands starts with it.
+#define ALEPH_ROWS_TAIL(FMA)                                                                                         \
+  FMA " %[pr], -%[b], %[xi], %[pr]\n" FMA " %[pi], %[b], %[xr], %[pi]\n" FMA " %[qr], -%[f], %[xi], %[qr]\n" FMA      \
+      " %[qi], %[f], %[xr], %[qi]\n" FMA " %[pr], %[c], %[yr], %[pr]\n" FMA " %[pi], %[c], %[yi], %[pi]\n" FMA        \
+      " %[qr], %[g], %[yr], %[qr]\n" FMA " %[qi], %[g], %[yi], %[qi]\n" FMA " %[pr], -%[d], %[yi], %[pr]\n" FMA       \
+      " %[pi], %[d], %[yr], %[pi]\n" FMA " %[qr], -%[h], %[yi], %[qr]\n" FMA " %[qi], %[h], %[yr], %[qi]\n"
+#define ALEPH_ROWS_IN(v0, v1, m)                                                                                     \
+  [xr] "v"((v0).x), [xi] "v"((v0).y), [yr] "v"((v1).x), [yi] "v"((v1).y), [a] "s"((m)[0]), [b] "s"((m)[1]),          \
+      [c] "s"((m)[2]), [d] "s"((m)[3]), [e] "s"((m)[8]), [f] "s"((m)[9]), [g] "s"((m)[10]), [h] "s"((m)[11])
 #define ALEPH_PAIR_UPDATE(T, MUL, FMA, MOV)                                                                          \
   __device__ __forceinline__ void pair_update(C2<T>& x, C2<T>& y, const T (&m)[8]) {                                 \
     T t0, t1, t2, t3;                                                                                                \
@@ -65,29 +73,20 @@ __device__ __forceinline__ uint32_t opaque(uint32_t v) { return __builtin_amdgcn
                  : [a] "s"(m[0]), [b] "s"(m[1]), [c] "s"(m[2]), [d] "s"(m[3]), [e] "s"(m[4]), [f] "s"(m[5]),         \
                    [g] "s"(m[6]), [h] "s"(m[7]));                                                                    \
   }                                                                                                                  \
-  /* Two matrix rows (m: 16 entries) times (v0, v1, v2, v3), into (p, q). */                                         \
-  __device__ __forceinline__ void two_rows(const C2<T>& v0, const C2<T>& v1, C2<T>& p, C2<T>& q, const T* m,         \
-                                           bool first) {                                                             \
-    if (first) {                                                                                                     \
-      asm volatile("s_nop 1\n" MUL " %[pr], %[a], %[xr]\n" MUL " %[pi], %[a], %[xi]\n" MUL " %[qr], %[e], %[xr]\n"   \
-                   MUL " %[qi], %[e], %[xi]\n"                                                                       \
+  /* Two matrix rows (m: 16 entries) times a half of (v0, v1, v2, v3): into (p, q), or added to them. */             \
+  template <bool FIRST>                                                                                              \
+  __device__ __forceinline__ void two_rows(const C2<T>& v0, const C2<T>& v1, C2<T>& p, C2<T>& q, const T* m) {       \
+    if constexpr (FIRST) {                                                                                           \
+      asm volatile("s_nop 1\n" MUL " %[pr], %[a], %[xr]\n" MUL " %[pi], %[a], %[xi]\n"                               \
+                   MUL " %[qr], %[e], %[xr]\n" MUL " %[qi], %[e], %[xi]\n" ALEPH_ROWS_TAIL(FMA)                      \
                    : [pr] "=&v"(p.x), [pi] "=&v"(p.y), [qr] "=&v"(q.x), [qi] "=&v"(q.y)                              \
-                   : [xr] "v"(v0.x), [xi] "v"(v0.y), [a] "s"(m[0]), [e] "s"(m[8]));                                  \
+                   : ALEPH_ROWS_IN(v0, v1, m));                                                                      \
     } else {                                                                                                         \
-      asm volatile("s_nop 1\n" FMA " %[pr], %[a], %[xr], %[pr]\n" FMA " %[pi], %[a], %[xi], %[pi]\n" FMA             \
-                   " %[qr], %[e], %[xr], %[qr]\n" FMA " %[qi], %[e], %[xi], %[qi]\n"                                 \
+      asm volatile("s_nop 1\n" FMA " %[pr], %[a], %[xr], %[pr]\n" FMA " %[pi], %[a], %[xi], %[pi]\n"                 \
+                   FMA " %[qr], %[e], %[xr], %[qr]\n" FMA " %[qi], %[e], %[xi], %[qi]\n" ALEPH_ROWS_TAIL(FMA)        \
                    : [pr] "+v"(p.x), [pi] "+v"(p.y), [qr] "+v"(q.x), [qi] "+v"(q.y)                                  \
-                   : [xr] "v"(v0.x), [xi] "v"(v0.y), [a] "s"(m[0]), [e] "s"(m[8]));                                  \
+                   : ALEPH_ROWS_IN(v0, v1, m));                                                                      \
     }                                                                                                                \
-    asm volatile(FMA " %[pr], -%[b], %[xi], %[pr]\n" FMA " %[pi], %[b], %[xr], %[pi]\n" FMA                          \
-                 " %[qr], -%[f], %[xi], %[qr]\n" FMA " %[qi], %[f], %[xr], %[qi]\n" FMA                              \
-                 " %[pr], %[c], %[yr], %[pr]\n" FMA " %[pi], %[c], %[yi], %[pi]\n" FMA                               \
-                 " %[qr], %[g], %[yr], %[qr]\n" FMA " %[qi], %[g], %[yi], %[qi]\n" FMA                               \
-                 " %[pr], -%[d], %[yi], %[pr]\n" FMA " %[pi], %[d], %[yr], %[pi]\n" FMA                              \
-                 " %[qr], -%[h], %[yi], %[qr]\n" FMA " %[qi], %[h], %[yr], %[qi]\n"                                  \
-                 : [pr] "+v"(p.x), [pi] "+v"(p.y), [qr] "+v"(q.x), [qi] "+v"(q.y)                                    \
-                 : [xr] "v"(v0.x), [xi] "v"(v0.y), [yr] "v"(v1.x), [yi] "v"(v1.y), [b] "s"(m[1]), [c] "s"(m[2]),     \
-                   [d] "s"(m[3]), [f] "s"(m[9]), [g] "s"(m[10]), [h] "s"(m[11]));                                    \
   }                                                                                                                  \
   /* a = v, in a's own registers. */                                                                                 \
   __device__ __forceinline__ void put(C2<T>& a, const C2<T>& v) {                                                    \
@@ -104,6 +103,8 @@ __device__ __forceinline__ uint32_t opaque(uint32_t v) { return __builtin_amdgcn
 ALEPH_PAIR_UPDATE(double, "v_mul_f64", "v_fma_f64", "v_mov_b64")
 ALEPH_PAIR_UPDATE(float, "v_mul_f32", "v_fma_f32", "v_mov_b32")
 #undef ALEPH_PAIR_UPDATE
+#undef ALEPH_ROWS_TAIL
+#undef ALEPH_ROWS_IN
 
 template <typename T, int G, int B, bool CTL>
 __device__ __forceinline__ void loop_1q(C2<T> (&a)[1 << G], const T (&m)[8], uint64_t tgo, const uint64_t (&rg)[G],
@@ -121,8 +122,8 @@ template <typename T, int G, int A, int B, int Q = 0>
 __device__ __forceinline__ void upper_rows(C2<T> (&a)[1 << G], C2<T> (&p)[1 << (G - 1)], const T* m) {
   if constexpr (Q < (1 << (G - 2))) {
     constexpr int r = ins0(ins0(Q, B), A);
-    two_rows(a[r], a[r | (1 << B)], p[2 * Q], p[2 * Q + 1], m, true);
-    two_rows(a[r | (1 << A)], a[r | (1 << A) | (1 << B)], p[2 * Q], p[2 * Q + 1], m + 4, false);
+    two_rows<true>(a[r], a[r | (1 << B)], p[2 * Q], p[2 * Q + 1], m);
+    two_rows<false>(a[r | (1 << A)], a[r | (1 << A) | (1 << B)], p[2 * Q], p[2 * Q + 1], m + 4);
     upper_rows<T, G, A, B, Q + 1>(a, p, m);
   }
 }
@@ -134,8 +135,8 @@ __device__ __forceinline__ void lower_rows(C2<T> (&a)[1 << G], const C2<T> (&p)[
   if constexpr (Q < (1 << (G - 2))) {
     constexpr int r = ins0(ins0(Q, B), A), r1 = r | (1 << B), r2 = r | (1 << A), r3 = r1 | r2;
     C2<T> p2, p3;
-    two_rows(a[r], a[r1], p2, p3, m, true);
-    two_rows(a[r2], a[r3], p2, p3, m + 4, false);
+    two_rows<true>(a[r], a[r1], p2, p3, m);
+    two_rows<false>(a[r2], a[r3], p2, p3, m + 4);
     if (!CTL || ((tgo | roff<G>(rg, r)) & cm) == cm) {
       put(a[r], p[2 * Q]);
       put(a[r1], p[2 * Q + 1]);
