@@ -634,64 +634,72 @@ void add_standalone(Plan& p, const LGate& g) {
 constexpr size_t kCutMinTerms = 8;
 
 uint32_t add_cut_phase(Plan& p, const std::vector<PhaseTerm>& reg, const std::vector<PhaseTerm>& gen,
-                       const PlannerCtx& pc, const uint64_t* rg) {
+                       const PlannerCtx& pc, uint32_t m, const uint64_t* rg) {
   if (!gen.empty() || reg.size() < kCutMinTerms || pc.G != 4 || pc.n > kCutQubits) return 0;
-  auto mask_of = [&](const PhaseTerm& t) {
+  struct Item {
+    uint64_t mask;
+    double k;
+  };
+  std::vector<Item> items;
+  items.reserve(reg.size());
+  double phi0 = 0.0, theta = 0.0;
+  for (const PhaseTerm& t : reg) {
     uint64_t mk = t.mask_out;
     for (uint32_t g = 0; g < 4; g++)
       if ((t.rmask >> g) & 1u) mk |= rg[g];
-    return mk;
-  };
-  double phi0 = 0.0, theta = 0.0;
-  for (const PhaseTerm& t : reg) {
-    if (mask_of(t) == 0) phi0 += t.angle;
-    else if (t.angle != 0.0 && (theta == 0.0 || std::fabs(t.angle) < std::fabs(theta))) theta = t.angle;
+    if (mk == 0) {
+      phi0 += t.angle;
+      continue;
+    }
+    if (popc(mk) > 2 || !std::isfinite(t.angle)) return 0;
+    items.push_back(Item{mk, t.angle});
+    if (t.angle != 0.0 && (theta == 0.0 || std::fabs(t.angle) < std::fabs(theta))) theta = t.angle;
   }
   if (theta == 0.0) return 0;
   // The smallest angle is itself a small multiple (3 theta and -2 theta on a
   // 3-regular graph).  Multiples are exact to the rounding of a sum of a few
   // equal angles: angles that differ by more keep their own values.
-  constexpr double kSame = 4.0 * std::numeric_limits<double>::epsilon();
-  auto multiple = [&](double t) {
-    for (const PhaseTerm& pt : reg)
-      if (mask_of(pt) != 0 && std::fabs(pt.angle / t - std::nearbyint(pt.angle / t)) > kSame * std::fabs(pt.angle / t))
-        return false;
-    return true;
-  };
+  constexpr double kSame = 4.0 * std::numeric_limits<double>::epsilon(), kMost = 64.0;
+  for (Item& it : items) {
+    it.k /= theta;
+    if (!(std::fabs(it.k) <= kMost)) return 0;
+  }
+  auto whole = [](double x) { return (double)(int)(x + (x < 0.0 ? -0.5 : 0.5)); };
   int div = 1;
-  while (div < 5 && !multiple(theta / div)) div++;
+  for (; div < 5; div++) {
+    bool all = true;
+    for (const Item& it : items) all &= std::fabs(it.k * div - whole(it.k * div)) <= kSame * std::fabs(it.k * div);
+    if (all) break;
+  }
   if (div == 5) return 0;
   theta /= div;
+  for (Item& it : items) {
+    it.k = whole(it.k * div);
+    if (std::fabs(it.k) > kMost) return 0;
+  }
   CutPhase c{};
   c.n = pc.n;
   int linear[64] = {0};
   uint64_t adj[64] = {0};
-  bool have_pair = false, negative = false;
-  for (int pass = 0; pass < 2; pass++) {
-    // Linear coefficients are kept non-negative: the sign of theta follows
-    // the first one.
-    for (const PhaseTerm& t : reg) {
-      const uint64_t mk = mask_of(t);
-      if (mk == 0) continue;
-      const double k = std::nearbyint(t.angle / theta);   // sums of a few equal angles: whole to rounding
-      if (std::fabs(k) > 64.0) return 0;
-      if (popc(mk) == 1) {
-        if (pass == 0) negative = k < 0;
-        else linear[__builtin_ctzll(mk)] += (int)k;
-      } else if (popc(mk) == 2) {
-        if (pass == 0) continue;
-        if (have_pair && (int)k != c.pair) return 0;
-        have_pair = true;
-        c.pair = (int)k;
-        const uint32_t lo = (uint32_t)__builtin_ctzll(mk), hi = 63u - (uint32_t)__builtin_clzll(mk);
-        if ((adj[hi] >> lo) & 1ull) return 0;
-        adj[hi] |= 1ull << lo;
-        adj[lo] |= 1ull << hi;
-      } else {
-        return 0;
-      }
+  bool have_pair = false;
+  int sign = 0;
+  // Linear coefficients are kept non-negative: the sign of theta follows the
+  // last one.
+  for (const Item& it : items)
+    if (popc(it.mask) == 1) sign = it.k < 0.0 ? -1 : 1;
+  if (sign < 0) theta = -theta;
+  for (const Item& it : items) {
+    const int k = (int)(sign < 0 ? -it.k : it.k);
+    const uint32_t lo = (uint32_t)__builtin_ctzll(it.mask), hi = 63u - (uint32_t)__builtin_clzll(it.mask);
+    if (lo == hi) {
+      linear[lo] += k;
+      continue;
     }
-    if (pass == 0 && negative) theta = -theta;
+    if ((have_pair && k != c.pair) || ((adj[hi] >> lo) & 1ull)) return 0;
+    have_pair = true;
+    c.pair = k;
+    adj[hi] |= 1ull << lo;
+    adj[lo] |= 1ull << hi;
   }
   uint64_t regs = 0;
   for (uint32_t g = 0; g < 4; g++) regs |= rg[g];
@@ -707,8 +715,11 @@ uint32_t add_cut_phase(Plan& p, const std::vector<PhaseTerm>& reg, const std::ve
     c.below[q] = (uint32_t)(adj[q] & ((1ull << q) - 1ull) & ~regs);
   }
   // The bounds of K are loose (every qubit set, every pair counted): an op
-  // whose table would be too large keeps its terms.
-  if (hi - lo + 1 > (int64_t)kCutTable) return 0;
+  // whose table would be too large keeps its terms, and so does one whose
+  // workgroup is too small to form it: eight entries a thread at most (a
+  // 4-qubit circuit, one thread: 30 entries took 1.4 times as long as the
+  // terms, 16 threads at 8 qubits 0.8 times).
+  if (hi - lo + 1 > (int64_t)std::min(kCutTable, 8u << (m - 4))) return 0;
   c.k_min = (int32_t)lo;
   c.size = (uint32_t)(hi - lo + 1);
   for (uint32_t g = 0; g < 4; g++) {
@@ -720,16 +731,11 @@ uint32_t add_cut_phase(Plan& p, const std::vector<PhaseTerm>& reg, const std::ve
     for (uint32_t g = 0; g < 4; g++)
       for (uint32_t h = g + 1; h < 4; h++)
         if (((r >> g) & 1u) && ((r >> h) & 1u) && (adj[__builtin_ctzll(rg[g])] & rg[h])) c.slot[r] += c.pair;
+  c.phi0 = phi0;
+  c.theta = theta;
   const uint32_t at = (uint32_t)p.terms.size();
-  p.terms.resize(at + (sizeof(CutPhase) + c.size * 2 * sizeof(double) + sizeof(PhaseTerm) - 1) / sizeof(PhaseTerm));
+  p.terms.resize(at + (sizeof(CutPhase) + sizeof(PhaseTerm) - 1) / sizeof(PhaseTerm));
   std::memcpy(&p.terms[at], &c, sizeof(c));
-  double* table = reinterpret_cast<double*>(reinterpret_cast<unsigned char*>(&p.terms[at]) + sizeof(CutPhase));
-  for (uint32_t i = 0; i < c.size; i++) {
-    // In long double: the sum is exact to far below a double's rounding.
-    const long double phi = (long double)phi0 + (long double)theta * (long double)(c.k_min + (int32_t)i);
-    table[2 * i] = (double)std::cos(phi);
-    table[2 * i + 1] = (double)std::sin(phi);
-  }
   return at + 1;
 }
 
@@ -900,7 +906,7 @@ void emit_fused_pass(Plan& p, const PlannerCtx& pc, uint64_t S, const std::vecto
         if (bounds[k] < bounds[k + 1]) ph.a |= 1u << k;
       p.terms.insert(p.terms.end(), pend_reg.begin(), pend_reg.end());
       p.terms.insert(p.terms.end(), pend_gen.begin(), pend_gen.end());
-      if (!p.opts.jit) ph.cut = add_cut_phase(p, pend_reg, pend_gen, pc, sd.rg);
+      if (!p.opts.jit) ph.cut = add_cut_phase(p, pend_reg, pend_gen, pc, m, sd.rg);
       p.ops.push_back(ph);
       pend_reg.clear();
       pend_gen.clear();

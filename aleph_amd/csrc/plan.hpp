@@ -71,12 +71,13 @@ struct alignas(16) PhaseTerm {
 // phi0 + theta K(x) with
 //   K(x) = sum_q linear_q x_q + pair * (number of listed pairs inside x),
 // so an amplitude needs an integer and one entry of a table of unit factors.
-// Stored in the terms array after the op's terms; the table (cos, sin of
-// phi0 + theta k for k = k_min ..) follows it.
+// Stored in the terms array after the op's terms.  The kernel forms the table,
+// one entry a thread.
 constexpr uint32_t kCutQubits = 26;
 constexpr uint32_t kCutTable = 256;
 struct alignas(16) CutPhase {
-  int32_t k_min;
+  double phi0, theta;
+  int32_t k_min;               // K of the table's first entry
   uint32_t size;               // table entries
   int32_t pair;                // coefficient of every pair
   uint32_t n;
@@ -85,9 +86,9 @@ struct alignas(16) CutPhase {
   uint32_t reg_adj[4];         // their pairs with other qubits
   int32_t slot[16];            // K of register setting r among the register bits
   uint32_t below[kCutQubits];  // pairs of qubit u with lower qubits (register bits aside)
-  uint32_t pad[7];
+  uint32_t pad[3];
 };
-static_assert(sizeof(CutPhase) % 16 == 0, "the table follows at 16 bytes");
+static_assert(sizeof(CutPhase) == 256, "CutPhase layout");
 
 struct alignas(16) StageDev {
   uint32_t op_begin, op_end;

@@ -9,7 +9,8 @@ import numpy as np
 import pytest
 
 from aleph_amd import workloads as W
-from aleph_amd.plan_tools import HostBatch
+from aleph_amd.circuit import Circuit
+from aleph_amd.plan_tools import HostBatch, HostPlan
 from tests.helpers import max_abs
 from tests.plan_emulator import emulate
 
@@ -83,3 +84,22 @@ def test_batch_instances_emulate_to_oracle(oracle_lib):
             o.run(c, st)
             got = emulate(hb.instance_plan(i), psi0, precision=prec)
             assert max_abs(got, st.amplitudes()) < tol, (prec, i)
+
+
+def test_equal_weight_phases_stay_small_on_the_host():
+    # New angles plan and upload the terms again: the integer form of a MaxCut layer adds 256 bytes to its terms,
+    # and no table.
+    graphs, ga, be = W.qaoa_batch(24, seed=5, n_min=8, n_max=16, p=3)
+    hb = HostBatch(graphs, ga, be, precision=32)
+    phases = [o for o in hb.ops if o.type == 5]
+    assert phases and all(o.cut for o in phases)
+    assert len(hb.terms) == sum(o.n_terms + 6 for o in phases)
+
+
+@pytest.mark.parametrize("n,cut", [(4, False), (6, False), (8, True), (12, True)])
+def test_equal_weight_phases_need_threads_for_their_table(n, cut):
+    c = Circuit(n)
+    for u, v in W.random_3_regular(n, 3):
+        c.cx(u, v).rz(0.3, v).cx(u, v)
+    phases = [o for o in HostPlan(c).ops if o.type == 5]
+    assert phases and all(bool(o.cut) == cut for o in phases)
