@@ -93,6 +93,8 @@ constexpr int kMarginalUnroll = 8;
 // Workgroups of a reduction: four per CU, a tile of kUnroll * kThreads
 // consecutive amplitudes at a time, so that a row of partials sums many reads
 // (the second launch then takes 7 us at 27 qubits where 4096 rows took 16).
+// Twice as many for FP32, whose loads are half as long: the norm at 27 qubits
+// takes 309 us with 1024, 217 with 2048 and 223 with 4096 (FP64 374, 384, 382).
 constexpr uint32_t kReduceGrid = 1024;
 
 // MODE 0: [sum over bit q clear, sum over bit q set, non-finite count] of p = |a|^2.
@@ -157,7 +159,7 @@ __device__ __forceinline__ void collapse_pairs(C2<T>* s, uint64_t pairs, uint32_
 }
 
 // A measurement without a round trip to the host: every workgroup adds the
-// rows of the preceding reduction (at most kReduceGrid, a few microseconds)
+// rows of the preceding reduction (at most 2 * kReduceGrid, a few microseconds)
 // and comes to the same decision the host reads from host[0..3); an invalid
 // state or a degenerate branch is left alone.  The reduction's second launch,
 // the copy back, a synchronisation and the reads of the zeroed half go (19
@@ -174,6 +176,44 @@ __global__ void __launch_bounds__(kThreads) k_measure(C2<T>* __restrict__ s, uin
   if (!c.apply) return;
   collapse_pairs(s, pairs, q, c.outcome, c.scale, (uint64_t)blockIdx.x * blockDim.x + threadIdx.x,
                  (uint64_t)gridDim.x * blockDim.x);
+}
+
+// The same for large states in three launches: one workgroup adds the rows and
+// decides, and a collapse with a grid of an amplitude a thread reads the
+// decision.  FP64 27 qubits 1039 -> 923 us, 28 qubits 2101 -> 1817 (FP32 622
+// -> 508, 1245 -> 946); 24 qubits 113 either way, below the launch counts.
+struct MeasureDecision {
+  double scale;
+  uint32_t apply, outcome;
+};
+
+__global__ void __launch_bounds__(kThreads) k_measure_decide(const double* __restrict__ partials, uint32_t rows,
+                                                             double u, double tol, MeasureDecision* decision,
+                                                             double* host) {
+  __shared__ double total[3];
+  sum_rows(partials, rows, total);
+  if (threadIdx.x < 3) host[threadIdx.x] = total[threadIdx.x];
+  if (threadIdx.x == 0) {
+    const MeasureChoice c = measure_choice(total[0], total[1], total[2], u, tol);
+    *decision = MeasureDecision{c.scale, c.apply ? 1u : 0u, c.outcome ? 1u : 0u};
+  }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(kThreads) k_collapse(C2<T>* __restrict__ s, uint64_t len, uint64_t qmask,
+                                                       const MeasureDecision* __restrict__ decision) {
+  const MeasureDecision d = *decision;
+  if (!d.apply) return;
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < len; i += (uint64_t)gridDim.x * blockDim.x) {
+    C2<T> a;
+    a.x = a.y = 0;
+    if (((i & qmask) != 0) == (d.outcome != 0)) {
+      a = s[i];
+      a.x = (T)((double)a.x * d.scale);
+      a.y = (T)((double)a.y * d.scale);
+    }
+    s[i] = a;
+  }
 }
 
 // The same for a state of one workgroup's size, in one launch.
@@ -616,12 +656,13 @@ inline uint32_t grid_for(uint64_t items) {
 }  // namespace
 
 namespace {
+template <typename T>
 uint32_t reduce_blocks(uint64_t len) {
   // Four tiles a workgroup before the next one: fewer rows for the second
   // launch to add (19 qubits: a measurement's two kernels
   // 17.7 -> 14.5 us, with the rows added by a wavefront per column).
   const uint64_t tiles = (uint64_t)kUnroll * kThreads * 4;
-  return (uint32_t)std::min<uint64_t>((len + tiles - 1) / tiles, kReduceGrid);
+  return (uint32_t)std::min<uint64_t>((len + tiles - 1) / tiles, sizeof(T) == 8 ? kReduceGrid : 2 * kReduceGrid);
 }
 }  // namespace
 
@@ -635,17 +676,17 @@ void launch_reduce_branch(hipStream_t st, const void* state, uint32_t n, int32_t
                           double* out) {
   const uint64_t len = 1ull << n;
   const uint64_t qmask = qubit >= 0 ? (1ull << qubit) : 0ull;
-  hipLaunchKernelGGL((k_reduce_branch<T, 0>), dim3(reduce_blocks(len)), dim3(kThreads), 0, st, (const C2<T>*)state,
+  hipLaunchKernelGGL((k_reduce_branch<T, 0>), dim3(reduce_blocks<T>(len)), dim3(kThreads), 0, st, (const C2<T>*)state,
                      len, qmask, partials);
-  launch_reduce_rows(st, partials, reduce_blocks(len), out);
+  launch_reduce_rows(st, partials, reduce_blocks<T>(len), out);
 }
 
 template <typename T>
 void launch_sum_p2(hipStream_t st, const void* state, uint32_t n, double* partials, double* out) {
   const uint64_t len = 1ull << n;
-  hipLaunchKernelGGL((k_reduce_branch<T, 1>), dim3(reduce_blocks(len)), dim3(kThreads), 0, st, (const C2<T>*)state,
+  hipLaunchKernelGGL((k_reduce_branch<T, 1>), dim3(reduce_blocks<T>(len)), dim3(kThreads), 0, st, (const C2<T>*)state,
                      len, 0ull, partials);
-  launch_reduce_rows(st, partials, reduce_blocks(len), out);
+  launch_reduce_rows(st, partials, reduce_blocks<T>(len), out);
 }
 
 template <typename T>
@@ -671,6 +712,8 @@ void launch_expect_group(hipStream_t st, const void* state, uint32_t n, uint64_t
 
 // One workgroup up to 11 qubits (8 amplitudes a thread).
 constexpr uint32_t kMeasureSmallQubits = 11;
+// From here the collapse's own traffic outweighs a third launch.
+constexpr uint32_t kMeasureLargeQubits = 25;
 
 template <typename T>
 void launch_measure(hipStream_t st, void* state, uint32_t n, uint32_t qubit, double u, double tol, double* partials,
@@ -679,11 +722,19 @@ void launch_measure(hipStream_t st, void* state, uint32_t n, uint32_t qubit, dou
   if (n <= kMeasureSmallQubits) {
     hipLaunchKernelGGL(k_measure_small<T>, dim3(1), dim3(kThreads), 0, st, (C2<T>*)state, len, qubit, u, tol, host);
   } else {
-    const uint32_t rows = reduce_blocks(len);
+    const uint32_t rows = reduce_blocks<T>(len);
     hipLaunchKernelGGL((k_reduce_branch<T, 0>), dim3(rows), dim3(kThreads), 0, st, (const C2<T>*)state, len,
                        1ull << qubit, partials);
-    hipLaunchKernelGGL(k_measure<T>, dim3(std::min<uint32_t>(grid_for(len / 2), 2 * kReduceGrid)), dim3(kThreads), 0,
-                       st, (C2<T>*)state, len / 2, qubit, (const double*)partials, rows, u, tol, host);
+    if (n >= kMeasureLargeQubits) {
+      MeasureDecision* d = reinterpret_cast<MeasureDecision*>(partials + 3 * (size_t)kReduceBlocks);
+      hipLaunchKernelGGL(k_measure_decide, dim3(1), dim3(kThreads), 0, st, (const double*)partials, rows, u, tol, d,
+                         host);
+      hipLaunchKernelGGL(k_collapse<T>, dim3(grid_for(len)), dim3(kThreads), 0, st, (C2<T>*)state, len, 1ull << qubit,
+                         (const MeasureDecision*)d);
+    } else {
+      hipLaunchKernelGGL(k_measure<T>, dim3(std::min<uint32_t>(grid_for(len / 2), 2 * kReduceGrid)), dim3(kThreads), 0,
+                         st, (C2<T>*)state, len / 2, qubit, (const double*)partials, rows, u, tol, host);
+    }
   }
   ALEPH_HIP_CHECK(hipGetLastError());
 }

@@ -157,6 +157,32 @@ def test_measure_collapses_like_numpy(hip, n, qubit, precision):
     assert np.array_equal(st.amplitudes()[:-1], psi[:-1])
 
 
+# The first size whose collapse is a launch of its own.
+@pytest.mark.parametrize("precision", [64, 32])
+def test_measure_collapses_a_large_state(hip, precision):
+    n = 25
+    v = np.random.default_rng(3).standard_normal(1 << n)
+    st = hip.allocate(n, precision)
+    st.load(v / np.linalg.norm(v))
+    psi = st.amplitudes()
+    tol = 4e-16 if precision == 64 else 1.2e-7
+    for qubit, bit in ((0, True), (9, False), (n - 1, True)):
+        half = np.abs(psi.reshape(-1, 2, 1 << qubit)) ** 2
+        p1 = float(np.sum(half[:, 1]))
+        st.load(psi)
+        assert hip.measure_with_uniform(st, qubit, 0.5 * p1 if bit else 0.5 * (1 + p1)) == (bit, True)
+        got = st.amplitudes().reshape(-1, 2, 1 << qubit)
+        want = psi.reshape(-1, 2, 1 << qubit)[:, int(bit)] / np.sqrt(p1 if bit else 1.0 - p1)
+        assert not np.any(got[:, 1 - int(bit)])
+        # As above: two roundings of the product, and the sum behind p1.
+        assert np.max(np.abs(got[:, int(bit)] - want)) <= (tol + 1e-14) * np.max(np.abs(want))
+    psi[-1] = np.inf
+    st.load(psi)
+    with pytest.raises(InvalidState):
+        hip.measure_with_uniform(st, 3, 0.5)
+    assert np.array_equal(st.amplitudes()[:-1], psi[:-1])
+
+
 def test_unused_and_refused_draws_stay_in_the_generator(hip):
     a, b = HipSvBackend(seed=31), HipSvBackend(seed=31)
     sa, sb = a.allocate(5), b.allocate(5)
