@@ -52,27 +52,16 @@ __device__ __forceinline__ uint64_t roff(const uint64_t (&rg)[G], int r) {
   return o;
 }
 
-template <int G>
-__device__ __forceinline__ uint32_t loff(const uint32_t (&rl)[G], int r) {
-  uint32_t o = 0;
-#pragma unroll
-  for (int g = 0; g < G; g++)
-    if (r & (1 << g)) o |= rl[g];
-  return o;
-}
+// CTL: whether the op has controls (fixed by the plan).
+constexpr int kCtlNone = 0, kCtlSome = 1;
 
-// CTL: kCtlNone / kCtlSome when the plan fixes whether the op has controls
-// (kernels generated per pass), kCtlAny to decide from op->cmask.
-constexpr int kCtlNone = 0, kCtlSome = 1, kCtlAny = 2;
-
-template <typename T, int G, int B, int CTL = kCtlAny>
+template <typename T, int G, int B, int CTL>
 __device__ __forceinline__ void op_1q(C2<T> (&a)[1 << G], const DevOp* __restrict__ op, uint64_t tgo,
                                       const uint64_t (&rg)[G]) {
   const T* mm = reinterpret_cast<const T*>(op->m);  // matrix stored in the plan's precision
   const T m00r = mm[0], m00i = mm[1], m01r = mm[2], m01i = mm[3];
   const T m10r = mm[4], m10i = mm[5], m11r = mm[6], m11i = mm[7];
-  const uint64_t cm = op->cmask;
-  if (CTL == kCtlNone || (CTL == kCtlAny && cm == 0)) {
+  if constexpr (CTL == kCtlNone) {
 #pragma unroll
     for (int r = 0; r < (1 << G); r++) {
       if (r & (1 << B)) continue;
@@ -82,7 +71,7 @@ __device__ __forceinline__ void op_1q(C2<T> (&a)[1 << G], const DevOp* __restric
       a[s] = cmac2(m10r, m10i, x, m11r, m11i, y);
     }
   } else {
-    const uint64_t tc = tgo & cm;
+    const uint64_t cm = op->cmask, tc = tgo & cm;
 #pragma unroll
     for (int r = 0; r < (1 << G); r++) {
       if (r & (1 << B)) continue;
@@ -151,19 +140,18 @@ __device__ __forceinline__ void quartets_2q(C2<T> (&a)[1 << G], const DevOp* __r
   }
 }
 
-template <typename T, int G, int A, int B, int CTL = kCtlAny>  // A = matrix MSB register bit, B = LSB, A > B
+template <typename T, int G, int A, int B, int CTL>  // A = matrix MSB register bit, B = LSB, A > B
 __device__ __forceinline__ void op_2q(C2<T> (&a)[1 << G], const DevOp* __restrict__ op, uint64_t tgo,
                                       const uint64_t (&rg)[G]) {
-  const uint64_t cm = op->cmask;
   bool on[1 << (G - 2)];
-  if (CTL == kCtlNone || (CTL == kCtlAny && cm == 0)) {
+  if constexpr (CTL == kCtlNone) {
     quartets_2q<T, G, A, B, 0, false>(a, op, on);
-    return;
-  }
-  const uint64_t tc = tgo & cm;
+  } else {
+    const uint64_t cm = op->cmask, tc = tgo & cm;
 #pragma unroll
-  for (int q = 0; q < (1 << (G - 2)); q++) on[q] = (tc | (roff<G>(rg, ins0(ins0(q, B), A)) & cm)) == cm;
-  quartets_2q<T, G, A, B, 0, true>(a, op, on);
+    for (int q = 0; q < (1 << (G - 2)); q++) on[q] = (tc | (roff<G>(rg, ins0(ins0(q, B), A)) & cm)) == cm;
+    quartets_2q<T, G, A, B, 0, true>(a, op, on);
+  }
 }
 
 // FP32 4x4 op on the matrix cores: v_mfma_f32_4x4x1f32 (16 blocks of
@@ -253,21 +241,18 @@ __device__ __forceinline__ void op_diag(C2<T> (&a)[1 << G], const DevOp* __restr
   }
 }
 
-// RM >= 0: the register part of the mask fixed at compile time (generated
-// pass kernels), so only the matching slots are touched; RM < 0: op->a.
-template <typename T, int G, int RM = -1>
+// RM: the register part of the mask, so only the matching slots are touched.
+template <typename T, int G, int RM>
 __device__ __forceinline__ void op_sign(C2<T> (&a)[1 << G], const DevOp* __restrict__ op, uint64_t tgo) {
-  // Sign-bit XOR with (thread condition as a bit mask) & (uniform slot
-  // condition): no divergent branch, one bitop per word.
+  // Sign-bit XOR under the thread condition as a bit mask: no divergent
+  // branch, one bitop per word.
   const uint64_t mo = op->cmask;
-  const uint32_t rm = RM >= 0 ? (uint32_t)RM : op->a;
   const uint32_t tm = ((tgo & mo) == mo) ? ~0u : 0u;
 #pragma unroll
   for (int r = 0; r < (1 << G); r++) {
-    if (RM >= 0 && ((uint32_t)r & (uint32_t)RM) != (uint32_t)RM) continue;
-    const uint32_t sr = (((uint32_t)r & rm) == rm) ? 0x80000000u : 0u;   // uniform
-    a[r].x = flip_sign(a[r].x, sr, tm);
-    a[r].y = flip_sign(a[r].y, sr, tm);
+    if (((uint32_t)r & (uint32_t)RM) != (uint32_t)RM) continue;
+    a[r].x = flip_sign(a[r].x, 0x80000000u, tm);
+    a[r].y = flip_sign(a[r].y, 0x80000000u, tm);
   }
 }
 
