@@ -3,8 +3,9 @@
 // Staged programs keep the state in registers (k_staged, up to 14 qubits);
 // for the others states of up to 13 qubits live in LDS (one read of the
 // program from L2, no HBM traffic per gate) and wider ones in the
-// workgroup's own slice of a device buffer (k_trajectories).  The RNG is counter-based, so every thread of the
-// workgroup computes the same draw without communication.
+// workgroup's own slice of a device buffer (k_trajectories).  The RNG is
+// counter-based, so every thread of the workgroup computes the same draw
+// without communication.
 #include "common.hpp"
 #include "noise.hpp"
 
@@ -325,8 +326,12 @@ __global__ void __launch_bounds__(kLds ? kNoiseThreadsLds : kNoiseThreadsWide) k
 
 // ---- register-resident trajectories (TStage, noise.hpp) ----
 //
-// Measured on MI355X, the 12-qubit depth-10 noisy brickwall, 20 000 shots:
-// extern __shared__ double2 lds_state[];MEASUREDextern __shared__ double2 lds_state[];
+// Measured on MI355X against k_trajectories (state in LDS, one op at a time with
+// barriers, a norm reduction per Kraus channel): the 12-qubit depth-10 noisy
+// brickwall, 20 000 shots, 46.9 -> 9.3 ms a call (5.8 ms of it this kernel, the
+// rest on the host); 14 qubits, 2 048 shots, 63.3 -> 7.6 ms.  Bound by issue: four
+// waves per SIMD, vector instructions for the amplitudes and scalar ones for the
+// records (profiles/kernel_stats_measured_cases.md).
 
 // Register-slot patterns of register bit g: bit r of kSlots[g] is bit g of r.
 __device__ __constant__ constexpr uint32_t kSlots[4] = {0xAAAAu, 0xCCCCu, 0xF0F0u, 0xFF00u};

@@ -358,7 +358,9 @@ def outcomes(circuit: Circuit, model: NoiseModel, shots: int, seed: int, backend
 def _plan(n: int, shots: int, options: NoiseOptions, sparse: bool) -> int:
     """Buffer bytes of one call, checked against the budget before anything
     is allocated (plan_noisy, execution.rs:62-190): the outcomes, the
-    dense or sparse result and the device slices of wide states."""
+    dense or sparse result and the device slices of wide states (at 14 qubits
+    most programs run in registers and leave theirs unused; which do is known
+    to the library only)."""
     if options.memory_budget_bytes <= 0 or (options.max_workers is not None and options.max_workers <= 0):
         raise Configuration("budget and max_workers must be positive")
     result = min(shots, 1 << n) * 16 if sparse else (1 << n) * 8
