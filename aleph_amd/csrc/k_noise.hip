@@ -7,6 +7,7 @@
 // counter-based, so every thread of the workgroup computes the same draw
 // without communication.
 #include "common.hpp"
+#include "inplace.hpp"
 #include "noise.hpp"
 
 namespace aleph {
@@ -331,7 +332,7 @@ __global__ void __launch_bounds__(kLds ? kNoiseThreadsLds : kNoiseThreadsWide) k
 // brickwall, 20 000 shots, 46.9 -> 9.3 ms a call (5.8 ms of it this kernel, the
 // rest on the host); 14 qubits, 2 048 shots, 63.3 -> 7.6 ms.  Bound by issue: four
 // waves per SIMD, vector instructions for the amplitudes and scalar ones for the
-// records (profiles/kernel_stats_measured_cases.md).
+// records.
 
 // Register-slot patterns of register bit g: bit r of kSlots[g] is bit g of r.
 __device__ __constant__ constexpr uint32_t kSlots[4] = {0xAAAAu, 0xCCCCu, 0xF0F0u, 0xFF00u};
@@ -339,6 +340,11 @@ __device__ __constant__ constexpr uint32_t kSlots[4] = {0xAAAAu, 0xCCCCu, 0xF0F0
 __device__ __forceinline__ double flip_hi(double x, uint32_t s) {
   return __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, x) ^ ((uint64_t)s << 32));
 }
+
+// Conditions of the record loop go through opaque() so that exclusive ifs are
+// not rebuilt into a switch.
+using fused::opaque;
+using fused::pair_update;
 
 // Plain components: arrays of the HIP vector type stay in scratch memory.
 using Amp = C2<double>;
@@ -395,39 +401,6 @@ __device__ __forceinline__ Record record(const TOp* ops, uint32_t o) {
 }
 constexpr uint32_t kLook = 0x80000000u;   // the Kraus channel has to look at the state
 
-// (x, y) <- M (x, y), updated in place.  Written as one block because the
-// amplitudes are live across the record loop's branches: with the 2x2 in C++
-// the compiler put every result into a new register and copied all 2^G
-// amplitudes back where the branches join (250 moves a record beside 128
-// FMAs).  s_nop: the matrix may come from v_readfirstlane, which needs two
-// wait states before a vector read.
-__device__ __forceinline__ void pair_update(Amp& x, Amp& y, const Mat2& m) {
-  double t0, t1, t2, t3;
-  asm volatile(
-      "s_nop 1\n"
-      "v_mul_f64 %[t0], %[a], %[xr]\n"
-      "v_mul_f64 %[t1], %[a], %[xi]\n"
-      "v_mul_f64 %[t2], %[e], %[xr]\n"
-      "v_mul_f64 %[t3], %[e], %[xi]\n"
-      "v_fma_f64 %[t0], -%[b], %[xi], %[t0]\n"
-      "v_fma_f64 %[t1], %[b], %[xr], %[t1]\n"
-      "v_fma_f64 %[t2], -%[f], %[xi], %[t2]\n"
-      "v_fma_f64 %[t3], %[f], %[xr], %[t3]\n"
-      "v_fma_f64 %[t0], %[c], %[yr], %[t0]\n"
-      "v_fma_f64 %[t1], %[c], %[yi], %[t1]\n"
-      "v_fma_f64 %[t2], %[g], %[yr], %[t2]\n"
-      "v_fma_f64 %[t3], %[g], %[yi], %[t3]\n"
-      "v_fma_f64 %[xr], -%[d], %[yi], %[t0]\n"
-      "v_fma_f64 %[xi], %[d], %[yr], %[t1]\n"
-      "v_fma_f64 %[t3], %[h], %[yr], %[t3]\n"
-      "v_fma_f64 %[yr], -%[h], %[yi], %[t2]\n"
-      "v_mov_b64 %[yi], %[t3]\n"
-      : [xr] "+v"(x.x), [xi] "+v"(x.y), [yr] "+v"(y.x), [yi] "+v"(y.y), [t0] "=&v"(t0), [t1] "=&v"(t1),
-        [t2] "=&v"(t2), [t3] "=&v"(t3)
-      : [a] "s"(m.v[0]), [b] "s"(m.v[1]), [c] "s"(m.v[2]), [d] "s"(m.v[3]), [e] "s"(m.v[4]), [f] "s"(m.v[5]),
-        [g] "s"(m.v[6]), [h] "s"(m.v[7]));
-}
-
 template <int G, int B, bool kCtl>
 __device__ __forceinline__ void one_qubit(Amp (&a)[1 << G], const Mat2& m, uint32_t tctl, const uint32_t (&rl)[G],
                                           uint32_t fx, uint32_t cm) {
@@ -442,7 +415,7 @@ __device__ __forceinline__ void one_qubit(Amp (&a)[1 << G], const Mat2& m, uint3
         if (r & (1 << g)) ro |= rl[g];
       on = (((tctl | ro) ^ fx) & cm) == cm;
     }
-    if (on) pair_update(a[r], a[r | (1 << B)], m);
+    if (on) pair_update(a[r], a[r | (1 << B)], m.v);
   }
 }
 
@@ -525,10 +498,6 @@ __device__ __forceinline__ void dispatch_two(Amp (&a)[1 << G], uint32_t sel, Pro
     }
   }
 }
-
-// A uniform value the compiler knows nothing about: conditions of the record
-// loop go through it so that exclusive ifs are not rebuilt into a switch.
-__device__ __forceinline__ uint32_t opaque(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // Negate the slots whose bit is set in sgn.
 template <int G>
