@@ -266,10 +266,15 @@ void Batch::plan() {
   // run their chunks one after the other in a few workgroups.  A round launch
   // wants four items per resident workgroup; the persistent executor pays
   // 0.17 us an item (the L2 write-back of its device-wide release) and wants
-  // one per CU.  24 FP64 instances of 10..16 qubits, p = 3: 1.25 ms with 16
-  // chunks an item, 0.20 ms with 1 (rounds 1.20 / 0.14); 160 FP32 instances of
-  // 12..20 qubits, p = 4: persistent 10.3 ms with 1, 3.8 with 4, 3.1 with 16,
-  // rounds 2.5 / 2.1 / 2.6 with 1 / 4 / 16.
+  // one per CU.  Milliseconds with 1 / 4 / 16 chunks an item and by default:
+  //                               persistent                rounds
+  //   24 FP64, 10..16 qubits   0.19 0.33 1.07 -> 0.19   0.12 0.28 1.01 -> 0.12
+  //   40 FP64, 12..18          0.57 0.41 0.91 -> 0.42   0.24 0.31 0.87 -> 0.24
+  //   16 FP64, 16..20          0.59 0.42 0.95 -> 0.43   0.23 0.32 0.91 -> 0.23
+  //   32 FP32, 14..20          1.39 0.71 1.18 -> 0.77   0.33 0.41 1.05 -> 0.33
+  //   160 FP32, 12..20         10.4 3.75 2.55 -> 2.55   1.87 1.72 2.06 -> 1.68
+  //   256 FP32, 10..16         0.59 0.36 0.66 -> 0.37   0.16 0.21 0.60 -> 0.16
+  //   1024 FP32, 12..16        2.87 1.08 1.06 -> 1.04   0.51 0.52 0.77 -> 0.51
   uint64_t first_round = 0;
   for (uint32_t i = 0; i < N; i++)
     if (nq[i] < solo_q && inst_passes[i]) first_round += 1ull << (nq[i] - passes[pass_list[i][0]].m);

@@ -103,3 +103,21 @@ def test_equal_weight_phases_need_threads_for_their_table(n, cut):
         c.cx(u, v).rz(0.3, v).cx(u, v)
     phases = [o for o in HostPlan(c).ops if o.type == 5]
     assert phases and all(bool(o.cut) == cut for o in phases)
+
+
+@pytest.mark.parametrize("mode,want", [(0, 256), (1, 4096)])
+@pytest.mark.parametrize("count,n_min,n_max", [(1, 8, 8), (24, 10, 16), (160, 12, 20), (40, 16, 20)])
+def test_default_items_spread_the_first_round(count, n_min, n_max, mode, want):
+    # As many chunks an item as leave the first round enough items, 16 at most (one workgroup per CU for the
+    # persistent executor, four items per resident workgroup for a launch per round).
+    graphs, ga, be = W.qaoa_batch(count, seed=5, n_min=n_min, n_max=n_max, p=2)
+    hb = HostBatch(graphs, ga, be, mode=mode)
+    first = hb.items[:hb.round_begin[1]]
+    chunks = sum(i.chunk_count for i in first)
+    per_item = max(i.chunk_count for i in hb.items)
+    split = 16
+    while split > 1 and chunks // split < want:
+        split //= 2
+    assert per_item == min(split, max(1 << (n - hb.passes[i.pass_].m) for i in hb.items for n in [hb.num_qubits[i.inst]]))
+    explicit = HostBatch(graphs, ga, be, mode=mode, chunks_per_item=3)
+    assert max(i.chunk_count for i in explicit.items) <= 3
