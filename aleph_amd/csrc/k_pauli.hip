@@ -255,13 +255,16 @@ PauliPlan plan_pauli_sum(const std::vector<PauliTerm>& terms, uint32_t n) {
   const uint32_t m = std::min(n, kChunkBits), L = std::min(kRunBits, m);
   const uint64_t low = (1ull << L) - 1ull;
   plan.sweeps.push_back(PauliSweep{low, {}});
+  size_t k = 0;
+  uint64_t last = 0;
   for (uint32_t t : order) {
     const uint64_t x = terms[t].x;
     if ((uint32_t)__builtin_popcountll(low | x) > m) {
       plan.rest.push_back(t);
       continue;
     }
-    size_t k = 0;
+    if (x != last) k = 0;      // strings with one X mask follow each other and share a sweep
+    last = x;
     while (k < plan.sweeps.size() && (uint32_t)__builtin_popcountll(plan.sweeps[k].qubits | x) > m) k++;
     if (k == kMaxSweeps) {
       plan.rest.push_back(t);
