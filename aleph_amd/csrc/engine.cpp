@@ -634,7 +634,7 @@ void add_standalone(Plan& p, const LGate& g) {
 constexpr size_t kCutMinTerms = 8;
 
 uint32_t add_cut_phase(Plan& p, const std::vector<PhaseTerm>& reg, const std::vector<PhaseTerm>& gen,
-                       const PlannerCtx& pc, uint32_t m, const uint64_t* rg) {
+                       const PlannerCtx& pc, const uint64_t* rg) {
   if (!gen.empty() || reg.size() < kCutMinTerms || pc.G != 4 || pc.n > kCutQubits) return 0;
   struct Item {
     uint64_t mask;
@@ -715,11 +715,8 @@ uint32_t add_cut_phase(Plan& p, const std::vector<PhaseTerm>& reg, const std::ve
     c.below[q] = (uint32_t)(adj[q] & ((1ull << q) - 1ull) & ~regs);
   }
   // The bounds of K are loose (every qubit set, every pair counted): an op
-  // whose table would be too large keeps its terms, and so does one whose
-  // workgroup is too small to form it: eight entries a thread at most (a
-  // 4-qubit circuit, one thread: 30 entries took 1.4 times as long as the
-  // terms, 16 threads at 8 qubits 0.8 times).
-  if (hi - lo + 1 > (int64_t)std::min(kCutTable, 8u << (m - 4))) return 0;
+  // whose table would be too large keeps its terms.
+  if (hi - lo + 1 > (int64_t)kCutTable) return 0;
   c.k_min = (int32_t)lo;
   c.size = (uint32_t)(hi - lo + 1);
   for (uint32_t g = 0; g < 4; g++) {
@@ -906,7 +903,7 @@ void emit_fused_pass(Plan& p, const PlannerCtx& pc, uint64_t S, const std::vecto
         if (bounds[k] < bounds[k + 1]) ph.a |= 1u << k;
       p.terms.insert(p.terms.end(), pend_reg.begin(), pend_reg.end());
       p.terms.insert(p.terms.end(), pend_gen.begin(), pend_gen.end());
-      if (!p.opts.jit) ph.cut = add_cut_phase(p, pend_reg, pend_gen, pc, m, sd.rg);
+      if (!p.opts.jit) ph.cut = add_cut_phase(p, pend_reg, pend_gen, pc, sd.rg);
       p.ops.push_back(ph);
       pend_reg.clear();
       pend_gen.clear();

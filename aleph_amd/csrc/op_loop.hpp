@@ -259,8 +259,9 @@ __device__ __forceinline__ void loop_diag(C2<T> (&a)[1 << G], Prog<DevOp>* op, u
 // Process chunk `chunk` of pass `pd` on `state`.  With GUARD, threads with
 // tid >= 2^(m - G) hold no amplitudes but take part in every barrier, so a
 // workgroup sized for the largest chunk can run smaller passes; without it
-// the workgroup has exactly 2^(m - G) threads.  `lds` holds 2^m scalars of 8
-// bytes: the real, then the imaginary parts of FP64 amplitudes, whole FP32 ones.
+// the workgroup has exactly 2^(m - G) threads, or is one wavefront whose spare
+// lanes repeat the others' work.  `lds` holds 2^m scalars of 8 bytes: the
+// real, then the imaginary parts of FP64 amplitudes, whole FP32 ones.
 template <typename T, int G, int FEAT, bool NT, bool GUARD>
 __device__ __forceinline__ void fused_chunk(C2<T>* __restrict__ state, const PassDev* __restrict__ pass,
                                             const StageDev* __restrict__ stage_list, const DevOp* __restrict__ op_list,

@@ -9,8 +9,7 @@ import numpy as np
 import pytest
 
 from aleph_amd import workloads as W
-from aleph_amd.circuit import Circuit
-from aleph_amd.plan_tools import HostBatch, HostPlan
+from aleph_amd.plan_tools import HostBatch
 from tests.helpers import max_abs
 from tests.plan_emulator import emulate
 
@@ -94,15 +93,6 @@ def test_equal_weight_phases_stay_small_on_the_host():
     phases = [o for o in hb.ops if o.type == 5]
     assert phases and all(o.cut for o in phases)
     assert len(hb.terms) == sum(o.n_terms + 6 for o in phases)
-
-
-@pytest.mark.parametrize("n,cut", [(4, False), (6, False), (8, True), (12, True)])
-def test_equal_weight_phases_need_threads_for_their_table(n, cut):
-    c = Circuit(n)
-    for u, v in W.random_3_regular(n, 3):
-        c.cx(u, v).rz(0.3, v).cx(u, v)
-    phases = [o for o in HostPlan(c).ops if o.type == 5]
-    assert phases and all(bool(o.cut) == cut for o in phases)
 
 
 @pytest.mark.parametrize("mode,want", [(0, 256), (1, 4096)])
