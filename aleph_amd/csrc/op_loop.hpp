@@ -93,6 +93,7 @@ __device__ __forceinline__ void loop_2q(C2<T> (&a)[1 << G], const T* upper, Prog
                                         const uint64_t (&rg)[G], uint64_t cm) {
   C2<T> p[1 << (G - 1)];
   upper_rows<T, G, A, B>(a, p, upper);
+  asm volatile("" : "+s"(mm));      // the second half takes the scalar registers of the first
   T lower[16];
 #pragma unroll
   for (int e = 0; e < 16; e++) lower[e] = mm[16 + e];
