@@ -227,20 +227,17 @@ void Batch::plan() {
     }
     const Plan& p = *plans[i];
     const uint32_t sb = (uint32_t)stages.size(), ob = (uint32_t)ops.size(), tb = (uint32_t)terms.size();
-    for (const StageDev& sd : p.stages) {
-      StageDev c = sd;
-      c.op_begin += ob;
-      c.op_end += ob;
-      stages.push_back(c);
+    stages.insert(stages.end(), p.stages.begin(), p.stages.end());
+    for (uint32_t k = sb; k < stages.size(); k++) {
+      stages[k].op_begin += ob;
+      stages[k].op_end += ob;
     }
-    for (const DevOp& op : p.ops) {
-      DevOp c = op;
-      if (c.type == OP_PHASE) {
-        c.term_off += tb;
-        if (c.cut) c.cut += tb;
+    ops.insert(ops.end(), p.ops.begin(), p.ops.end());
+    for (uint32_t k = ob; k < ops.size(); k++)
+      if (ops[k].type == OP_PHASE) {
+        ops[k].term_off += tb;
+        if (ops[k].cut) ops[k].cut += tb;
       }
-      ops.push_back(c);
-    }
     terms.insert(terms.end(), p.terms.begin(), p.terms.end());
     for (const Step& s : p.steps) {
       PassDev pd = p.passes[s.pass];

@@ -867,6 +867,24 @@ void emit_fused_pass(Plan& p, const PlannerCtx& pc, uint64_t S, const std::vecto
       return rm;
     };
     std::vector<PhaseTerm> pend_reg, pend_gen;
+    // The unit factors of the last few angles: a layer of equal weights has
+    // two or three.
+    struct {
+      double angle = 0.0, c = 1.0, s = 0.0;
+    } units[4];
+    uint32_t next_unit = 0;
+    auto unit_factor = [&](PhaseTerm& t) {
+      for (const auto& u : units)
+        if (std::memcmp(&u.angle, &t.angle, sizeof(double)) == 0) {
+          t.c = u.c;
+          t.s = u.s;
+          return;
+        }
+      t.c = std::cos(t.angle);
+      t.s = std::sin(t.angle);
+      units[next_unit] = {t.angle, t.c, t.s};
+      next_unit = (next_unit + 1) % 4;
+    };
     // A term whose mask has no chunk bit outside the register bits depends
     // only on the chunk number: the same for every thread of a workgroup.
     auto thread_dep = [&](const PhaseTerm& t) { return (t.mask_out & S) != 0; };
@@ -956,8 +974,7 @@ void emit_fused_pass(Plan& p, const PlannerCtx& pc, uint64_t S, const std::vecto
             t.mask_out = mask & ~rphys;
             t.rmask = reg_mask(mask);
             t.angle = angle;
-            t.c = std::cos(angle);
-            t.s = std::sin(angle);
+            unit_factor(t);
             bool general = false;
             t.cls = phase_class(t.rmask, pc.G, &general);
             (general ? pend_gen : pend_reg).push_back(t);
