@@ -7,9 +7,9 @@
 // re-distributed through LDS between stages and written back once.
 //
 // Bound by vector issue and by how much latency its waves hide, so it is
-// written for few registers (92 to 128 in FP64 with one kind of dense or phase
-// op, 145 with both; 60 to 115 in FP32; none spilled), and a workgroup with
-// its SIMDs to itself by the scalar loads of the ops:
+// written for few vector registers (92 to 128 in FP64 with 4x4 or phase ops,
+// 144 with both; 60 to 117 in FP32; none spilled), and a workgroup with its
+// SIMDs to itself by the scalar loads of the ops:
 //  - the loop body is a row of plain ifs on selector words the compiler knows
 //    nothing about, behind one if per kind of op, and the operators change the
 //    amplitudes in place (one asm block per pair or quartet): with a chain of
